@@ -70,6 +70,7 @@ struct VarlenParams {
   int32_t kparts;
   int64_t rows;  // rows of qkv and out (the partial buffers' row count)
   float* part;
+  float split;   // != 0: out holds the split terms (split2) of its values times split
 };
 
 // ---- the model path's kernel ------------------------------------------------
@@ -305,8 +306,13 @@ __global__ __launch_bounds__(DL_NT) void attention_varlen_kernel(VarlenParams p)
     const float inv = 1.f / __shfl(l_tot, 4 * g + r, 64);
     if (qr < L) {
       float* orow = p.out + (int64_t)(start + qr) * OW + (int64_t)h * HD + dofs;
+      if (p.split != 0.f) {
 #pragma unroll
-      for (int db = 0; db < HALF / 16; db++) orow[db * 16 + lq] = oacc[db][r] * inv;
+        for (int db = 0; db < HALF / 16; db++) store_split1(orow, db * 16 + lq, oacc[db][r] * inv * p.split, true);
+      } else {
+#pragma unroll
+        for (int db = 0; db < HALF / 16; db++) orow[db * 16 + lq] = oacc[db][r] * inv;
+      }
     }
   }
 }
@@ -317,7 +323,7 @@ __global__ __launch_bounds__(DL_NT) void attention_varlen_kernel(VarlenParams p)
 template <int HD>
 __global__ __launch_bounds__(256) void attention_combine_kernel(const float* __restrict__ part, int kparts,
                                                                 int64_t rows, int64_t row_off, int64_t n, int H,
-                                                                float* __restrict__ out) {
+                                                                float* __restrict__ out, float split) {
   // rows: the partial buffers' row count; this launch sums rows row_off ..
   // row_off + n - 1 of them into out's rows 0 .. n - 1
   const int64_t lid = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);  // local row * H + head
@@ -367,7 +373,8 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const float* __r
     f32x4 o;
 #pragma unroll
     for (int e = 0; e < 4; e++) o[e] = acc[c][e] * inv;
-    *reinterpret_cast<f32x4*>(dst + c * 256) = o;
+    if (split != 0.f) store_split4_lanes(out + lrow * OW, h * HD + lane * 4 + c * 256, o * split);
+    else *reinterpret_cast<f32x4*>(dst + c * 256) = o;
   }
 }
 
@@ -453,6 +460,7 @@ struct TilesParams {
   const float* gq;
   const float *cs, *sn;
   float eps;
+  float split;  // != 0: out holds the split terms (split2) of its values times split
 };
 
 __device__ __forceinline__ void split_pack8(const f32x4& x0, const f32x4& x1, bf16x8& t0, bf16x8& t1, bf16x8& t2) {
@@ -995,9 +1003,14 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
     return;
   }
   const float inv = 1.f / l_tot;
-  float* orow = p.out + (start + tok) * OW + (int64_t)head * HD + 16 * NDB * hf + 4 * g;
+  float* orow = p.out + (start + tok) * OW + (int64_t)head * HD + 16 * NDB * hf;
+  if (p.split != 0.f) {
 #pragma unroll
-  for (int db = 0; db < NDB; db++) *reinterpret_cast<f32x4*>(orow + 16 * db) = oacc[db] * inv;
+    for (int db = 0; db < NDB; db++) store_split4(orow, 16 * db + 4 * g, oacc[db] * inv * p.split);
+  } else {
+#pragma unroll
+    for (int db = 0; db < NDB; db++) *reinterpret_cast<f32x4*>(orow + 16 * db + 4 * g) = oacc[db] * inv;
+  }
 }
 
 // ---- dense attention on the MFMA (the tensor.AttentionScaled drop-in) ----------
@@ -1264,6 +1277,7 @@ int launch_attention_varlen_items(fa_ctx* ctx, const AttnVarlenArgs& a, const in
   p.qkv = a.qkv; p.out = a.out; p.items = d_items; p.ext = a.item_ext; p.row0 = a.row0;
   p.H = a.H; p.Hkv = a.Hkv; p.window = a.window; p.scale = a.scale;
   p.kparts = a.kparts; p.rows = a.rows; p.part = a.part;
+  p.split = a.split;
   const dim3 grid((unsigned)((int64_t)n_items * a.kparts));
   if (a.D == 256)
     hipLaunchKernelGGL(attention_varlen_kernel<256>, grid, dim3(DL_NT), 0, s, p);
@@ -1277,10 +1291,10 @@ int launch_attention_varlen_items(fa_ctx* ctx, const AttnVarlenArgs& a, const in
     const dim3 g2((unsigned)((a.rows * a.H + per - 1) / per)), b2(64 * per);
     if (a.D == 256)
       hipLaunchKernelGGL(attention_combine_kernel<256>, g2, b2, 0, s, a.part, a.kparts, a.rows, (int64_t)0, a.rows,
-                         a.H, a.out);
+                         a.H, a.out, a.split);
     else
       hipLaunchKernelGGL(attention_combine_kernel<512>, g2, b2, 0, s, a.part, a.kparts, a.rows, (int64_t)0, a.rows,
-                         a.H, a.out);
+                         a.H, a.out, a.split);
   }
   FA_CHECK_LAUNCH(ctx);
   return FA_OK;
@@ -1310,7 +1324,7 @@ int launch_attention_tiles(fa_ctx* ctx, const AttnTilesArgs& a, const int32_t* d
   p.qkv = a.qkv; p.img = a.img; p.out = a.out; p.items = d_items; p.ext = a.item_ext;
   p.H = a.H; p.Hkv = a.Hkv; p.window = a.window; p.scale = a.scale; p.row0 = a.row0;
   p.kparts = a.kparts; p.rows = a.rows; p.part = a.part;
-  p.gq = a.gq; p.cs = a.cos_t; p.sn = a.sin_t; p.eps = a.eps;
+  p.gq = a.gq; p.cs = a.cos_t; p.sn = a.sin_t; p.eps = a.eps; p.split = a.split;
   const dim3 grid((unsigned)((int64_t)n_items * a.kparts));
   if (a.waves == 4 && tiles_pairs())
     hipLaunchKernelGGL((attention_tiles_kernel<8, 2>), grid, dim3(64 * 8), 0, s, p);
@@ -1320,7 +1334,7 @@ int launch_attention_tiles(fa_ctx* ctx, const AttnTilesArgs& a, const int32_t* d
     hipLaunchKernelGGL((attention_tiles_kernel<8, 1>), grid, dim3(64 * 8), 0, s, p);
   if (a.kparts > 1)
     hipLaunchKernelGGL(attention_combine_kernel<256>, dim3((unsigned)((a.nrows * a.H + 3) / 4)), dim3(256), 0, s,
-                       a.part, a.kparts, a.rows, a.row0, a.nrows, a.H, a.out);
+                       a.part, a.kparts, a.rows, a.row0, a.nrows, a.H, a.out, a.split);
   FA_CHECK_LAUNCH(ctx);
   return FA_OK;
 }

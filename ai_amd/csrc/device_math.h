@@ -130,7 +130,86 @@ __device__ __forceinline__ Split3 split3(float a) {
 // Two bf16 high halves packed as one dword, element `lo` first in memory.
 __device__ __forceinline__ uint32_t pack_hi16(uint32_t lo, uint32_t hi) { return (lo >> 16) | (hi & 0xFFFF0000u); }
 
+// Two-term fp16 split of an fp32 value a (|a| < 65520): hi = fp16(a), lo =
+// fp16((a - hi) * 2^11), packed as hi | lo << 16. a - hi is exact in fp32
+// (and so is the fma below: a * 2^11 is exact); lo keeps 11 of its at most
+// 12 significant bits, so hi + lo * 2^-11 is within 2^-23 of |a|, and three
+// values in four are exact. Below 2^-14 the terms are fp16 subnormals and
+// the error is at most 2^-36.
+__device__ __forceinline__ uint32_t split2(float a) {
+  const _Float16 hi = (_Float16)a;
+  const _Float16 lo = (_Float16)fmaf((float)hi, -0x1p11f, a * 0x1p11f);
+  return (uint32_t)__builtin_bit_cast(uint16_t, hi) | ((uint32_t)__builtin_bit_cast(uint16_t, lo) << 16);
+}
+
+// tanh-GELU as x * sigmoid(2 u), u = sqrt(2/pi) (x + 0.044715 x^3): with
+// s = 2^(-2 u log2 e) on the hardware exp2, x / (1 + s) by the hardware
+// reciprocal and one Newton step: half the VALU work of the rational tanh
+// (about 16 instead of 33 issue slots with the two quarter-rate functions),
+// which is what a GeGLU product's epilogue waits for. The exponent is capped
+// where 1 + s would leave float32's range (the result is then below 1e-36
+// |x|). Within 1.5e-7 of |x| of the exact function for every x, and nearer to
+// it than 1 + tanh for negative ones, where that sum cancels.
+__device__ __forceinline__ float gelu_sigmoid(float x) {
+  const float t = x * fmaf(x * x, -0.10294324f, -2.3022082f);  // -2 u log2 e
+  const float d = 1.f + __builtin_amdgcn_exp2f(fminf(t, 125.f));
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.f), r, r);
+  return x * r;
+}
+
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// A row of split values (split2): each 8 values as 16 bytes of hi terms,
+// then 16 bytes of lo terms, in the place of their 32 bytes of floats.
+// Byte offset of value col's hi term in its row (its lo term 16 bytes on).
+__device__ __forceinline__ int64_t split_off(int64_t col) { return (col >> 3) * 32 + (col & 7) * 2; }
+
+// Value col of a row, the lane to the left or right in its pair (col ^ 1)
+// storing its neighbour: the two swap halves so that the even column's lane
+// stores both hi terms and the odd one's both lo terms, four bytes each.
+__device__ __forceinline__ uint32_t split1_pair(float v) {
+  const uint32_t own = split2(v);
+  const uint32_t nb = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)own, 0xB1, 0xF, 0xF, false);  // quad_perm 1,0,3,2
+  // even lane: own.hi, nb.hi; odd lane: nb.lo, own.lo
+  return __builtin_amdgcn_perm(own, nb, (threadIdx.x & 1) ? 0x07060302u : 0x01000504u);
+}
+// Byte offset of the pair's dword that the lane of column col stores
+// (col's parity is the lane's).
+__device__ __forceinline__ int64_t split1_off(int64_t col) {
+  return split_off(col & ~(int64_t)1) + ((col & 1) ? 16 : 0);
+}
+__device__ __forceinline__ void store_split1(float* row, int64_t col, float v, bool ok) {
+  const uint32_t w = split1_pair(v);
+  if (ok) *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(row) + split1_off(col)) = w;
+}
+
+// Four values col .. col + 3 (col % 4 == 0) as two dwords of hi, two of lo.
+struct Split4 {
+  uint2 hi, lo;
+};
+__device__ __forceinline__ Split4 split2x4(const f32x4& v) {
+  const uint32_t a = split2(v.x), b = split2(v.y), c = split2(v.z), d = split2(v.w);
+  return {make_uint2((a & 0xFFFFu) | (b << 16), (c & 0xFFFFu) | (d << 16)),
+          make_uint2((a >> 16) | (b & 0xFFFF0000u), (c >> 16) | (d & 0xFFFF0000u))};
+}
+__device__ __forceinline__ void store_split4(float* row, int64_t col, const f32x4& v) {
+  const Split4 t = split2x4(v);
+  char* at = reinterpret_cast<char*>(row) + split_off(col);
+  *reinterpret_cast<uint2*>(at) = t.hi;
+  *reinterpret_cast<uint2*>(at + 16) = t.lo;
+}
+// The same where lane l of the wave holds columns base + 4 l .. + 3 (base a
+// multiple of 8): the even lane stores the pair's eight hi terms, the odd
+// one its eight lo terms, so the wave writes 1 KB in lane order.
+__device__ __forceinline__ void store_split4_lanes(float* row, int64_t col, const f32x4& v) {
+  const Split4 t = split2x4(v);
+  const bool odd = threadIdx.x & 1;
+  const uint32_t sx = odd ? t.hi.x : t.lo.x, sy = odd ? t.hi.y : t.lo.y;
+  const uint32_t rx = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sx, 0xB1, 0xF, 0xF, false);
+  const uint32_t ry = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sy, 0xB1, 0xF, 0xF, false);
+  *reinterpret_cast<uint4*>(row + col) = odd ? make_uint4(rx, ry, t.lo.x, t.lo.y) : make_uint4(t.hi.x, t.hi.y, rx, ry);
+}
 
 // Sum over the wave of the squares of a lane's NC float4 (a row of NC * 256
 // values spread 4 per lane per 256), fixed order per lane then wave_sum.
@@ -151,13 +230,16 @@ __device__ __forceinline__ float sumsq(const f32x4 (&v)[NC]) {
 // 256 c + 4 lane .. +3): x = (x + RMSNorm(o [+ parts]; g_post)) * scale,
 // then xn = RMSNorm(x; g_next) when g_next != null (models/gemma/embed.go:
 // 217-237). With o2 != null, a K-split product's other n2 partials sit at
-// o2 + j * pstride (j < n2) and are added to o in part order.
+// o2 + j * pstride (j < n2) and are added to o in part order. With split !=
+// 0, xn (or, without a next norm, x itself) goes to xn as split terms of
+// its values times split, the operand of the fp16 products; xn may be null
+// without a next norm.
 template <int NC>
 __device__ __forceinline__ void residual_norm_row(const float* __restrict__ o, const float* __restrict__ o2,
                                                   int n2, int64_t pstride,
                                                   float* __restrict__ x, float* __restrict__ xn, int64_t row,
                                                   const float* __restrict__ g_post, const float* __restrict__ g_next,
-                                                  float eps, float scale, int lane) {
+                                                  float eps, float scale, float split, int lane) {
   constexpr int d = NC * 256;
   f32x4 ov[NC], xv[NC], gp[NC], gn[NC];
 #pragma unroll
@@ -217,7 +299,13 @@ __device__ __forceinline__ void residual_norm_row(const float* __restrict__ o, c
     }
     *reinterpret_cast<f32x4*>(x + row * d + col) = xv[c];
   }
-  if (g_next == nullptr) return;
+  if (g_next == nullptr) {
+    if (split != 0.f && xn) {
+#pragma unroll
+      for (int c = 0; c < NC; c++) store_split4_lanes(xn + row * d, c * 256 + lane * 4, xv[c] * split);
+    }
+    return;
+  }
   const float inv2 = rms_inv(sumsq<NC>(xv), d, eps);
 #pragma unroll
   for (int c = 0; c < NC; c++) {
@@ -225,7 +313,8 @@ __device__ __forceinline__ void residual_norm_row(const float* __restrict__ o, c
     const f32x4 gg = gn[c];
     f32x4 r;
     r.x = xv[c].x * inv2 * gg.x; r.y = xv[c].y * inv2 * gg.y; r.z = xv[c].z * inv2 * gg.z; r.w = xv[c].w * inv2 * gg.w;
-    *reinterpret_cast<f32x4*>(xn + row * d + col) = r;
+    if (split != 0.f) store_split4_lanes(xn + row * d, col, r * split);
+    else *reinterpret_cast<f32x4*>(xn + row * d + col) = r;
   }
 }
 

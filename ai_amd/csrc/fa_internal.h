@@ -171,6 +171,43 @@ int launch_split_b(fa_ctx* ctx, const void* b, int b_dtype, int64_t ldb, int lay
 // [m x F] = gelu(gate) * up.
 int launch_gemm(fa_ctx* ctx, const GemmArgs& g, hipStream_t stream);
 
+// The encoder's products on split activations (gemm_h2.hip): A [m x k] as two
+// fp16 terms per value (split2, each 8 values 16 bytes of hi then 16 of lo,
+// rows of lda values), B fp16 [n x k], k % 32 == 0. C = epi(A . B^T * c_scale):
+// GeGLU as GemmArgs, Generic only act (none or GELU) and mul. out_scale != 0
+// (not with epi None): C receives the split terms of its values times
+// out_scale. ksplit as GemmArgs (epi None).
+struct GemmH2Args {
+  int64_t m = 0, n = 0, k = 0;
+  const float* a = nullptr;
+  int64_t lda = 0;
+  const uint16_t* b = nullptr;
+  int64_t ldb = 0;
+  float* c = nullptr;
+  int64_t ldc = 0;
+  float c_scale = 1.f, out_scale = 0.f;
+  Epi epi = Epi::None;
+  int act = FA_ACT_NONE;
+  const float* mul = nullptr;
+  int64_t ldm = 0;
+  int ksplit = 1;
+  int64_t c_split = 0;
+  bool shared = false;
+};
+int launch_gemm_h2(fa_ctx* ctx, const GemmH2Args& g, hipStream_t stream);
+// FA_GEMM_H2=0, FA_GEMM_MFMA=f32 or FA_GEMM_XTILE (comparisons) keep the
+// encoder on the products of launch_gemm.
+bool gemm_h2_enabled();
+
+// Preparation of bf16 weights for launch_gemm_h2: *max_bits (zeroed by the
+// caller) becomes the largest |w| as bf16 bits; norms[r] the 2-norm of row r;
+// dst = fp16(w * scale), *bad (zeroed by the caller) nonzero when one of them
+// is not exact.
+int launch_h2_absmax(fa_ctx* ctx, const uint16_t* w, int64_t n, uint32_t* max_bits, hipStream_t s);
+int launch_h2_row_norms(fa_ctx* ctx, const uint16_t* w, int64_t rows, int64_t cols, float* norms, hipStream_t s);
+int launch_h2_convert(fa_ctx* ctx, const uint16_t* w, int64_t n, float scale, uint16_t* dst, uint32_t* bad,
+                      hipStream_t s);
+
 // FA_GEMM_MFMA=f32 (comparisons): every product on the fp32-MFMA kernel, bf16
 // weights widened and float32 weights taken as they are (no three-plane
 // rewrite).
@@ -234,9 +271,11 @@ int launch_row_plan(fa_ctx* ctx, const int32_t* cu_seqlens, int32_t nseq, int32_
 // xn[r] = x[r] * rms_inv(x[r]) * g (the first layer's input norm).
 // E: bf16 [vocab x d], or with plane > 0 three planes hi, mid, lo plane
 // elements apart (a float32 table that is not bf16-exact), summed exactly.
+// split != 0: xn receives the split terms of its values times split; xs (may
+// be null) those of x times xs_scale.
 int launch_embed_gather(fa_ctx* ctx, const int32_t* d_ids, const int32_t* d_row_src, const uint16_t* E, int64_t plane,
                         int64_t vocab, int64_t rows, int32_t d, float scale, const float* g_next, float eps, float* x,
-                        float* xn, hipStream_t s);
+                        float* xn, hipStream_t s, float split = 0.f, float* xs = nullptr, float xs_scale = 0.f);
 
 // q/k RMSNorm with (1+g) and RoPE on the packed qkv buffer [rows x (H+2*Hkv)*D],
 // in place; positions from d_pos (null: row i is position i, the rows being one sequence).
@@ -254,10 +293,12 @@ int launch_ple_norm(fa_ctx* ctx, float* pl, int64_t rows, int32_t nl, int32_t P,
 // x = (x + RMSNorm(o; g_post)) * scale; then xn = RMSNorm(x; g_next)
 // (g_next may be null: then xn is not written).
 // o2 (optional): the other n2 (1..3) partial products of a K-split GEMM,
-// planes pstride floats apart, added to o in part order.
+// planes pstride floats apart, added to o in part order. split != 0: xn
+// receives the split terms of its values times split; without g_next, of x's.
 int launch_residual_norm(fa_ctx* ctx, const float* o, float* x, float* xn, int64_t rows, int32_t d,
                          const float* g_post, const float* g_next, float eps, hipStream_t s,
-                         const float* o2 = nullptr, float scale = 1.f, int n2 = 1, int64_t pstride = 0);
+                         const float* o2 = nullptr, float scale = 1.f, int n2 = 1, int64_t pstride = 0,
+                         float split = 0.f);
 
 // Fused varlen attention over packed tokens. qkv [rows x (H+2Hkv)*D]; out
 // [rows x H*D]; window: keys with |i-j| >= window are masked (window <= 0:
@@ -280,6 +321,9 @@ struct AttnVarlenArgs {
   int32_t kparts = 1;
   int64_t rows = 0;
   float* part = nullptr;
+  // != 0: out holds the split terms (split2, device_math.h) of its values
+  // times split, the operand of launch_gemm_h2
+  float split = 0.f;
 };
 constexpr int kMaxKeyParts = 8;
 inline int64_t attention_part_floats(int kparts, int64_t rows, int H, int D) {
@@ -327,6 +371,7 @@ struct AttnTilesArgs {
   // 16-row blocks per work item, 4 or 8 (64 or 128 rows; 64-row items run
   // on eight waves in head-dimension pairs unless FA_ATTN_PAIRS=0)
   int32_t waves = 8;
+  float split = 0.f;  // as AttnVarlenArgs::split
 };
 // d_items holds n_items triples (sequence, first row, kv head): one item per
 // attention_tiles_rows(a.waves) rows (token, query head of the kv head's

@@ -50,6 +50,7 @@
 
 #include "fa_internal.h"
 #include "device_math.h"
+#include "gemm_common.h"
 
 namespace fa {
 namespace {
@@ -107,18 +108,6 @@ struct GemmParams {
 };
 
 __device__ __forceinline__ float bf16_to_f32(uint32_t h) { return __uint_as_float(h << 16); }
-
-// Tile index of this workgroup. Workgroup ids are dealt to the 8 XCDs
-// round-robin; each XCD gets a contiguous run of tiles (row-major over n) so
-// the tiles sharing A rows and B columns share that XCD's L2.
-__device__ __forceinline__ int xcd_tile(const GemmParams& p) {
-  constexpr int kXcd = 8;
-  const int total = p.tiles_m * p.tiles_n;
-  int tile = blockIdx.x;
-  const int per = total / kXcd;
-  if (per > 0 && tile < per * kXcd) tile = (tile % kXcd) * per + tile / kXcd;
-  return tile;
-}
 
 // The Generic epilogue of one element (the reference's order,
 // internal/blas/gemm.go:276-347); None returns v.
@@ -395,7 +384,7 @@ __global__ __launch_bounds__(TL::NT) void gemm_kernel(GemmParams p) {
     }
   };
 
-  const int tile = xcd_tile(p);
+  const int tile = xcd_tile(p.tiles_m, p.tiles_n);
   m0 = (int64_t)(tile / p.tiles_n) * BM;
   n0 = (int64_t)(tile % p.tiles_n) * BN;
   mainloop(0, p.nk);
@@ -503,7 +492,7 @@ __global__ __launch_bounds__(TL::NT, TL::MINW) void gemm_x3_kernel(GemmParams p)
   const float* __restrict__ A = p.a;
   const uint16_t* __restrict__ B = static_cast<const uint16_t*>(p.b);
 
-  const int tile = xcd_tile(p);
+  const int tile = xcd_tile(p.tiles_m, p.tiles_n);
   const int64_t m0 = (int64_t)(tile / p.tiles_n) * BM;
   const int64_t n0 = (int64_t)(tile % p.tiles_n) * BN;
   const int nk = p.nk / p.ksplit;                      // slabs of this K range

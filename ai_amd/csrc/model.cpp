@@ -59,6 +59,10 @@ struct Mat {
   int64_t rows = 0, cols = 0;
   int terms = 1;
   int64_t plane() const { return rows * cols; }
+  // the values times h_scale in fp16 (prepare_h2), for the products on split
+  // activations
+  uint16_t* h = nullptr;
+  float h_scale = 1.f;
 };
 
 struct Layer {
@@ -76,6 +80,11 @@ struct Layer {
   Mat wple_proj;  // [d, P]
   float* g_ple_post = nullptr;
   float scalar = 1.f;
+  // prepare_h2: the powers of two by which the split operands of this
+  // layer's products are scaled (normed inputs of q|k|v and gate|up,
+  // attention output, GeGLU output; variant 2: the residual stream before
+  // the per-layer-input block and the block's gated input)
+  float s_in = 0, s_att = 0, s_ffn = 0, s_gu = 0, s_x = 0, s_ple = 0;
 };
 
 struct KernelStat {
@@ -111,6 +120,10 @@ struct fa_model {
   int d_local = 0, d_global = 0;  // head dims of the sliding and the full layers
   std::set<std::string> seen;
   bool finalized = false;
+  // the layers' products run on split activations (prepare_h2): every layer
+  // matrix is exact in fp16 and every operand's range is known
+  bool h2 = false;
+  float s_x0 = 0;  // variant 2: scale of the scaled embeddings
   // workspace
   fa::DevBuf ws, plan_dev;
   int64_t ws_rows = 0, ws_seqs = 0;
@@ -163,6 +176,155 @@ void set_b(GemmArgs& g, const Mat& w, int64_t row0 = 0) {
   g.ldb = w.cols;
   g.b_terms = w.terms;
   g.b_plane = w.plane();
+}
+
+// Decides whether the layers' products can run on split activations
+// (gemm_h2.hip) and prepares them: m->h2. It needs
+//  - every layer matrix bf16-exact (terms == 1) and exact in fp16 after one
+//    power of two for the matrix (its largest value just below 2^15: values
+//    down to 2^-32 of that keep all their bits);
+//  - a bound for every activation operand, from which its power of two is
+//    taken (the bound just below 2^15): a normed row has 2-norm at most
+//    sqrt(d) max|gain|, so |x_j| is at most that and |w . x| at most |w|
+//    times it; attention outputs are convex combinations of values; |gelu(g)
+//    u| <= |g| |u|; the residual stream is a sum of normed rows. The split
+//    then keeps 23 bits down to 2^-29 of the bound (device_math.h). Gains
+//    whose largest value is more than 64 times their root mean square would
+//    put typical values too far below the bounds: those models keep the
+//    three-term products, as do non-finite weights.
+int prepare_h2(fa_model* m) {
+  m->h2 = false;
+  if (!gemm_h2_enabled()) return FA_OK;
+  fa_ctx* ctx = m->ctx;
+  const fa_gemma_config& c = m->cfg;
+  const bool v2 = m->variant == 2;
+  const int d = c.hidden_size, H = c.num_attention_heads, F = c.intermediate_size, P = m->P;
+  std::vector<Mat*> mats;
+  for (auto& L : m->layers) {
+    mats.insert(mats.end(), {&L.wqkv, &L.wo, &L.wgu, &L.wdown});
+    if (v2) mats.insert(mats.end(), {&L.wple_gate, &L.wple_proj});
+  }
+  if (v2) mats.push_back(&m->wple_model);
+  int64_t norm_rows = 0;
+  for (Mat* w : mats) {
+    if (w->terms != 1 || w->cols % 32 != 0) return FA_OK;
+    norm_rows += w->rows;
+  }
+  // largest |w| of each matrix (and of the embedding table), row norms
+  const size_t nm = mats.size();
+  DevBuf tmp;
+  const size_t head = (2 * (nm + 1) + 63) / 64 * 64;
+  int rc = tmp.ensure(ctx, (head + (size_t)norm_rows) * 4);
+  std::vector<uint32_t> host;
+  hipStream_t s = ctx->stream;
+  uint32_t* bits = tmp.as<uint32_t>();
+  float* norms = tmp.as<float>() + head;
+  auto run = [&]() -> int {
+    int r;
+    if ((r = launch_zero(ctx, bits, head * 4, s))) return r;
+    int64_t at = 0;
+    for (size_t i = 0; i < nm; i++) {
+      if ((r = launch_h2_absmax(ctx, mats[i]->p, mats[i]->plane(), bits + i, s))) return r;
+      if ((r = launch_h2_row_norms(ctx, mats[i]->p, mats[i]->rows, mats[i]->cols, norms + at, s))) return r;
+      at += mats[i]->rows;
+    }
+    if ((r = launch_h2_absmax(ctx, m->embed.p, m->embed.plane(), bits + nm, s))) return r;
+    host.resize(head + norm_rows);
+    FA_HIP_CHECK(ctx, hipMemcpyAsync(host.data(), tmp.ptr, host.size() * 4, hipMemcpyDeviceToHost, s));
+    FA_HIP_CHECK(ctx, hipStreamSynchronize(s));
+    return FA_OK;
+  };
+  if (!rc) rc = run();
+  auto value = [&](size_t i) {
+    const uint32_t u = host[i] << 16;
+    float f;
+    std::memcpy(&f, &u, 4);
+    return f;
+  };
+  // the power of two that takes bound b just below 2^15; 0 if there is none
+  auto pow2_for = [](double b) -> float {
+    if (!(b > 0) || !std::isfinite(b)) return 0.f;
+    const int e = 14 - std::ilogb(b * 1.0001);
+    return e < -100 || e > 100 ? 0.f : std::ldexp(1.f, e);
+  };
+  bool ok = !rc;
+  for (size_t i = 0; i < nm && ok; i++) {
+    const float mx = value(i);
+    mats[i]->h_scale = mx == 0.f ? 1.f : pow2_for(mx);
+    ok = mats[i]->h_scale != 0.f;
+    if (ok && !mats[i]->h) {
+      void* np = nullptr;
+      if ((rc = alloc_dev(m, (size_t)mats[i]->plane() * 2, &np))) break;
+      mats[i]->h = (uint16_t*)np;
+    }
+    if (ok) rc = launch_h2_convert(ctx, mats[i]->p, mats[i]->plane(), mats[i]->h_scale, mats[i]->h, bits + nm + 1 + i, s);
+    if (rc) ok = false;
+  }
+  if (ok) {
+    std::vector<uint32_t> bad(nm);
+    if (hipMemcpyAsync(bad.data(), bits + nm + 1, nm * 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
+      rc = set_error(ctx, FA_ERR_HIP, "gemma: reading the weights' range failed");
+    for (uint32_t b : bad) ok = ok && b == 0;
+  }
+  // operand bounds
+  const double rd = std::sqrt((double)d);
+  auto gain = [&](const float* dev, int n) -> double {  // max |gain|; not finite: unusable
+    std::vector<float> v(n);
+    if (hipMemcpy(v.data(), dev, (size_t)n * 4, hipMemcpyDeviceToHost) != hipSuccess) return INFINITY;
+    double mx = 0, ss = 0;
+    for (float x : v) {
+      if (!std::isfinite(x)) return INFINITY;
+      mx = std::max(mx, std::fabs((double)x));
+      ss += (double)x * x;
+    }
+    return mx > 64 * std::sqrt(ss / n) ? INFINITY : mx;
+  };
+  if (ok && !rc) {
+    int64_t at = 0;
+    auto row_max = [&](int64_t r0, int64_t r1, int64_t group, int64_t which) {  // largest norm of the rows
+      double mx = 0;
+      for (int64_t r = r0; r < r1; r++)
+        if (group == 0 || (r / group) % 2 == which) {
+          float f;
+          std::memcpy(&f, &host[head + at + r], 4);
+          mx = std::max(mx, (double)f);
+        }
+      return mx;
+    };
+    double xb = value(nm) * 1.01 * rd;  // the residual stream's largest value (variant 2's products read it)
+    m->s_x0 = pow2_for(xb);
+    const double gple = v2 ? gain(m->g_ple_norm, P) * std::sqrt((double)P) : 0;
+    for (auto& L : m->layers) {
+      const double nin = rd * gain(L.g_in, d), nffn = rd * gain(L.g_pre_ffn, d);
+      L.s_in = pow2_for(nin);
+      L.s_att = pow2_for(v2 ? std::sqrt((double)L.D) : nin * row_max((int64_t)(H + L.Hkv) * L.D, L.width, 0, 0));
+      at += L.wqkv.rows + L.wo.rows;
+      L.s_ffn = pow2_for(nffn);
+      L.s_gu = pow2_for(nffn * row_max(0, 2LL * F, 32, 0) * nffn * row_max(0, 2LL * F, 32, 1));
+      at += L.wgu.rows + L.wdown.rows;
+      ok = ok && L.s_in != 0 && L.s_att != 0 && L.s_ffn != 0 && L.s_gu != 0;
+      if (v2) {
+        xb += rd * (gain(L.g_post_attn, d) + gain(L.g_post_ffn, d));
+        L.s_x = pow2_for(xb);
+        L.s_ple = pow2_for(row_max(0, P, 0, 0) * xb * rd * gple);
+        at += L.wple_gate.rows + L.wple_proj.rows;
+        xb = (xb + rd * gain(L.g_ple_post, d)) * std::fabs((double)L.scalar);
+        ok = ok && L.s_x != 0 && L.s_ple != 0;
+      }
+    }
+    if (v2) ok = ok && m->s_x0 != 0;
+    m->h2 = ok;
+  }
+  tmp.release();
+  return rc;
+}
+
+// Fills the operands of a product on split activations: A scaled by a_scale.
+void set_h2(GemmH2Args& g, const Mat& w, float a_scale) {
+  g.b = w.h;
+  g.ldb = w.cols;
+  g.c_scale = 1.f / (a_scale * w.h_scale);
 }
 
 hipEvent_t take_event(fa_model* m) {
@@ -277,18 +439,19 @@ int microbatch_count_forced() {
   return v;
 }
 
-// Group count by the batch, from sweeps of 2, 3 and 4 groups on MI355X:
-// long sequences (the mean key count per token, sum L^2 / sum L, at least
-// 1 024) make the forward attention-bound and gain from a fourth stream
-// (C4, 8 x 1 024..2 048: 11.80 ms against 11.84 with two and 11.97 with
-// three); from 24 576 tokens the products are large enough on their own and
-// two groups keep their tiles full (C3, 64 x 512: 27.45 ms against 28.0 with
-// three); else three (C2: 5.30 ms against 5.41 with two and 5.53 with four;
-// C5, 17 923 tokens: 13.74 against 13.91 and 14.26).
+// Group count by the batch, from sweeps of 2, 3 and 4 groups on MI355X (ms
+// per forward of the 24-layer model): three for most batches (32 x 64..256
+// tokens: 4.45 with two or three, 4.59 with four; 256 x 16..128: 11.83, 11.61
+// and 11.68), two where the mean key count per token (sum L^2 / sum L) is at
+// least 1 024 (8 x 1 024..2 048: 10.36, 10.41 and 10.35) and from 24 576
+// tokens (64 x 512: 24.48, 24.73 and 24.56), where each group's launches
+// fill the chip. Not four: a process has four hardware queues, so with
+// another stream in use (a framework's own) the fourth group waits behind
+// one of the others (two layers of 8 x 1 024..2 048: 1.49 ms with four
+// groups, 1.18 with two).
 int microbatch_count(int64_t tokens, double sum_l2) {
   if (const int f = microbatch_count_forced()) return f;
-  if (sum_l2 >= 1024.0 * (double)tokens) return 4;
-  return tokens >= 24576 ? 2 : 3;
+  return tokens >= 24576 || sum_l2 >= 1024.0 * (double)tokens ? 2 : 3;
 }
 
 // HBM bytes of one residual_norm launch: the product's K parts and x
@@ -793,6 +956,10 @@ int fa_gemma_finalize(fa_model* m) {
     FA_HIP_CHECK(ctx, hipMemcpy(m->cos_global, cs.data(), cs.size() * 4, hipMemcpyHostToDevice));
     FA_HIP_CHECK(ctx, hipMemcpy(m->sin_global, sn.data(), sn.size() * 4, hipMemcpyHostToDevice));
   }
+  {
+    const int rc_ = fa::prepare_h2(m);
+    if (rc_) return rc_;
+  }
   m->finalized = true;
   return FA_OK;
 }
@@ -971,6 +1138,29 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
   float* attn_part = reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(hbuf1 + (size_t)B * maxw) + 255) &
                                               ~(uintptr_t)255);
   hipStream_t s = ctx->stream;
+  // products on split activations: xn, att and gu hold split terms (the last
+  // layer's xn, the final hidden states, stays in floats)
+  const bool h2 = m->h2;
+  // One product: g as launch_gemm takes it, or on A's split terms (at a, its
+  // values times a_scale; out_scale != 0: the result split too)
+  auto product = [&](const fa::GemmArgs& g, const float* a, const fa::Mat& w, float a_scale, float out_scale, int kind,
+                     double flops, hipStream_t st) -> int {
+    fa::Probe pr(m, kind, flops, 0);
+    int r;
+    if (h2) {
+      fa::GemmH2Args q;
+      q.m = g.m; q.n = g.n; q.k = g.k; q.a = a; q.lda = g.lda; q.c = g.c; q.ldc = g.ldc;
+      fa::set_h2(q, w, a_scale);
+      q.out_scale = out_scale; q.epi = g.epi; q.act = g.act; q.mul = g.mul; q.ldm = g.ldm;
+      q.ksplit = g.ksplit; q.c_split = g.c_split; q.shared = g.shared;
+      r = fa::launch_gemm_h2(ctx, q, st);
+    } else {
+      r = fa::launch_gemm(ctx, g, st);
+    }
+    if (r) return r;
+    pr.done();
+    return FA_OK;
+  };
   // ---- row plan on device ----
   if ((rc = fa::launch_row_plan(ctx, cu_d, B, T, M, row_src_d, pos_d, s))) return rc;
   const float eps = c.rms_norm_eps;
@@ -982,7 +1172,8 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
   {
     fa::Probe pr(m, FA_K_GATHER, 0, (double)M * (2.0 * d + 8.0 * d + 4));
     if ((rc = fa::launch_embed_gather(ctx, d_ids, row_src_d, m->embed.p, m->embed.terms == 3 ? m->embed.plane() : 0,
-                                      c.vocab_size, M, d, emb_scale, m->layers[0].g_in, eps, x, xn, s)))
+                                      c.vocab_size, M, d, emb_scale, m->layers[0].g_in, eps, x, xn, s,
+                                      h2 && n_run > 0 ? m->layers[0].s_in : 0.f, h2 && v2 ? qkv : nullptr, m->s_x0)))
       return rc;
     pr.done();
   }
@@ -992,9 +1183,8 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
       fa::GemmArgs g;
       g.m = M; g.n = (int64_t)NL * P; g.k = d; g.a = x; g.lda = d; fa::set_b(g, m->wple_model); g.c = ple;
       g.ldc = (int64_t)NL * P;
-      fa::Probe pr(m, FA_K_GEMM_PLE, 2.0 * M * NL * P * d, 0);
-      if ((rc = fa::launch_gemm(ctx, g, s))) return rc;
-      pr.done();
+      // (split: the scaled embeddings' terms, in q|k|v's buffer until the layers run)
+      if ((rc = product(g, qkv, m->wple_model, m->s_x0, 0.f, FA_K_GEMM_PLE, 2.0 * M * NL * P * d, s))) return rc;
     }
     fa::Probe pr(m, FA_K_PLE_NORM, 0, (double)M * NL * P * 8.0);
     if ((rc = fa::launch_ple_norm(ctx, ple, M, NL, P, (float)(1 / std::sqrt((double)d)), m->g_ple_norm, eps, s)))
@@ -1055,9 +1245,7 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
         g.ksplit = 2;
         g.c_split = o - qkvr;
       }
-      fa::Probe pr(m, FA_K_GEMM_QKV, 2.0 * rows * L.width * d, 0);
-      if ((rc = fa::launch_gemm(ctx, g, st))) return rc;
-      pr.done();
+      if ((rc = product(g, g.a, L.wqkv, L.s_in, 0.f, FA_K_GEMM_QKV, 2.0 * rows * L.width * d, st))) return rc;
     }
     if (tiles) {
       // read k and v (4 bytes per element); write their images (6 bytes per
@@ -1087,6 +1275,7 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
       a.item_ext = ext_d + 4 * ((items_v - items_d) / 3);
       a.H = H; a.Hkv = Hkv; a.D = D; a.scale = att_scale;
       a.window = (sliding && c.sliding_window > 0) ? wbound : 0;
+      a.split = h2 ? L.s_att : 0.f;
       if (kparts_v > 1) {
         a.kparts = kparts_v; a.rows = rows; a.part = attn_part;
       }
@@ -1109,6 +1298,7 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
         at.item_ext = ext_d + 4 * ((items_t - items_d) / 3);
         at.H = H; at.Hkv = Hkv; at.window = a.window; at.scale = a.scale;
         at.gq = L.g_q; at.eps = eps; at.cos_t = L.cos_t; at.sin_t = L.sin_t; at.waves = waves_t;
+        at.split = a.split;
         if (kparts_t > 1) {
           at.kparts = kparts_t; at.rows = M; at.nrows = rows; at.part = attn_part;
         }
@@ -1123,14 +1313,12 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
       g.shared = groups > 1;
       g.m = rows; g.n = d; g.k = H * D; g.a = attr; g.lda = H * D; fa::set_b(g, L.wo); g.c = or_;
       g.ldc = d; g.ksplit = ks_o; g.c_split = M * d;
-      fa::Probe pr(m, FA_K_GEMM_O, 2.0 * rows * d * H * D, 0);
-      if ((rc = fa::launch_gemm(ctx, g, st))) return rc;
-      pr.done();
+      if ((rc = product(g, g.a, L.wo, L.s_att, 0.f, FA_K_GEMM_O, 2.0 * rows * d * H * D, st))) return rc;
     }
     {
       fa::Probe pr(m, FA_K_RESIDUAL_NORM, 0, fa::resnorm_bytes(rows, d, ks_o, L.g_pre_ffn));
       if ((rc = fa::launch_residual_norm(ctx, or_, xr, xnr, rows, d, L.g_post_attn, L.g_pre_ffn, eps, st, o2_o, 1.f,
-                                         ks_o - 1, M * d)))
+                                         ks_o - 1, M * d, h2 ? L.s_ffn : 0.f)))
         return rc;
       pr.done();
     }
@@ -1139,26 +1327,23 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
       g.shared = groups > 1;
       g.m = rows; g.n = 2 * F; g.k = d; g.a = xnr; g.lda = d; fa::set_b(g, L.wgu); g.c = gur; g.ldc = F;
       g.epi = fa::Epi::GeGLU;
-      fa::Probe pr(m, FA_K_GEMM_GATEUP, 2.0 * rows * 2 * F * d, 0);
-      if ((rc = fa::launch_gemm(ctx, g, st))) return rc;
-      pr.done();
+      if ((rc = product(g, g.a, L.wgu, L.s_ffn, L.s_gu, FA_K_GEMM_GATEUP, 2.0 * rows * 2 * F * d, st))) return rc;
     }
     {
       fa::GemmArgs g;
       g.shared = groups > 1;
       g.m = rows; g.n = d; g.k = F; g.a = gur; g.lda = F; fa::set_b(g, L.wdown); g.c = or_; g.ldc = d;
       g.ksplit = ks_down; g.c_split = M * d;
-      fa::Probe pr(m, FA_K_GEMM_DOWN, 2.0 * rows * d * F, 0);
-      if ((rc = fa::launch_gemm(ctx, g, st))) return rc;
-      pr.done();
+      if ((rc = product(g, g.a, L.wdown, L.s_gu, 0.f, FA_K_GEMM_DOWN, 2.0 * rows * d * F, st))) return rc;
     }
     // the last layer's "next norm" is the final RMSNorm (embed.go:237): xn = h
     const float* g_next = (l + 1 < NL) ? m->layers[l + 1].g_in : m->g_final;
+    const float s_next = h2 && l + 1 < NL ? m->layers[l + 1].s_in : 0.f;
     {
       // variant 2: the per-layer-input block reads x itself, so no norm here
       fa::Probe pr(m, FA_K_RESIDUAL_NORM, 0, fa::resnorm_bytes(rows, d, ks_down, v2 ? nullptr : g_next));
       if ((rc = fa::launch_residual_norm(ctx, or_, xr, xnr, rows, d, L.g_post_ffn, v2 ? nullptr : g_next, eps, st,
-                                         o2_dn, 1.f, ks_down - 1, M * d)))
+                                         o2_dn, 1.f, ks_down - 1, M * d, v2 ? (h2 ? L.s_x : 0.f) : s_next)))
         return rc;
       pr.done();
     }
@@ -1170,22 +1355,19 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
         g.m = rows; g.n = P; g.k = d; g.a = xr; g.lda = d; fa::set_b(g, L.wple_gate); g.c = gur; g.ldc = P;
         g.epi = fa::Epi::Generic; g.act = FA_ACT_GELU; g.mul = ple + r0 * NL * P + (int64_t)l * P;
         g.ldm = (int64_t)NL * P;
-        fa::Probe pr(m, FA_K_GEMM_PLE, 2.0 * rows * P * d, 0);
-        if ((rc = fa::launch_gemm(ctx, g, st))) return rc;
-        pr.done();
+        // (split: x's terms, which the residual step above left in xn)
+        if ((rc = product(g, xnr, L.wple_gate, L.s_x, L.s_ple, FA_K_GEMM_PLE, 2.0 * rows * P * d, st))) return rc;
       }
       {
         fa::GemmArgs g;
         g.shared = groups > 1;
         g.m = rows; g.n = d; g.k = P; g.a = gur; g.lda = P; fa::set_b(g, L.wple_proj); g.c = or_; g.ldc = d;
         g.ksplit = ks_ple; g.c_split = M * d;
-        fa::Probe pr(m, FA_K_GEMM_PLE, 2.0 * rows * d * P, 0);
-        if ((rc = fa::launch_gemm(ctx, g, st))) return rc;
-        pr.done();
+        if ((rc = product(g, g.a, L.wple_proj, L.s_ple, 0.f, FA_K_GEMM_PLE, 2.0 * rows * d * P, st))) return rc;
       }
       fa::Probe pr(m, FA_K_RESIDUAL_NORM, 0, fa::resnorm_bytes(rows, d, ks_ple, g_next));
       if ((rc = fa::launch_residual_norm(ctx, or_, xr, xnr, rows, d, L.g_ple_post, g_next, eps, st, o2_pl, L.scalar,
-                                         ks_ple - 1, M * d)))
+                                         ks_ple - 1, M * d, s_next)))
         return rc;
       pr.done();
     }

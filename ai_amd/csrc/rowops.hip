@@ -90,14 +90,17 @@ __global__ __launch_bounds__(256) void rope_kernel(const float* __restrict__ x, 
 // NC = hidden/256 float4 chunks per lane.
 
 
-// x[r] = E[ids[src[r]]] * scale; xn[r] = x[r] * rms_inv(x[r]) * g.
+// x[r] = E[ids[src[r]]] * scale; xn[r] = x[r] * rms_inv(x[r]) * g. With split
+// != 0, xn holds the split terms of its values times split; xs (may be null)
+// gets those of x times xs_scale.
 template <int NC>
 __global__ __launch_bounds__(256) void embed_gather_kernel(const int32_t* __restrict__ ids,
                                                            const int32_t* __restrict__ row_src,
                                                            const uint16_t* __restrict__ E, int64_t plane,
                                                            int64_t vocab, int64_t rows, float scale,
                                                            const float* __restrict__ g, float eps,
-                                                           float* __restrict__ x, float* __restrict__ xn) {
+                                                           float* __restrict__ x, float* __restrict__ xn,
+                                                           float split, float* __restrict__ xs, float xs_scale) {
   constexpr int d = NC * 256;
   int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   int lane = threadIdx.x & 63;
@@ -137,7 +140,9 @@ __global__ __launch_bounds__(256) void embed_gather_kernel(const int32_t* __rest
     f32x4 gg = *reinterpret_cast<const f32x4*>(g + col);
     f32x4 o;
     o.x = v[c].x * inv * gg.x; o.y = v[c].y * inv * gg.y; o.z = v[c].z * inv * gg.z; o.w = v[c].w * inv * gg.w;
-    *reinterpret_cast<f32x4*>(xn + row * d + col) = o;
+    if (split != 0.f) store_split4_lanes(xn + row * d, col, o * split);
+    else *reinterpret_cast<f32x4*>(xn + row * d + col) = o;
+    if (xs) store_split4_lanes(xs + row * d, col, v[c] * xs_scale);
   }
 }
 
@@ -152,10 +157,10 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(const float* __restr
                                                             float* __restrict__ x, float* __restrict__ xn,
                                                             int64_t rows, const float* __restrict__ g_post,
                                                             const float* __restrict__ g_next, float eps,
-                                                            float scale) {
+                                                            float scale, float split) {
   int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);  // one wave per row
   if (row >= rows) return;
-  residual_norm_row<NC>(o, o2, n2, pstride, x, xn, row, g_post, g_next, eps, scale, threadIdx.x & 63);
+  residual_norm_row<NC>(o, o2, n2, pstride, x, xn, row, g_post, g_next, eps, scale, split, threadIdx.x & 63);
 }
 
 // Per (token, head): RMSNorm over D (256 or 512) with the head's gain vector
@@ -650,14 +655,14 @@ int launch_rope(fa_ctx* ctx, const float* x, const float* cos_t, const float* si
 
 int launch_embed_gather(fa_ctx* ctx, const int32_t* d_ids, const int32_t* d_row_src, const uint16_t* E, int64_t plane,
                         int64_t vocab, int64_t rows, int32_t d, float scale, const float* g_next, float eps, float* x,
-                        float* xn, hipStream_t s) {
+                        float* xn, hipStream_t s, float split, float* xs, float xs_scale) {
   if (rows == 0) return FA_OK;
   dim3 grid(blocks_for(rows, 4)), block(256);
   switch (d) {
-    case 256: hipLaunchKernelGGL(embed_gather_kernel<1>, grid, block, 0, s, d_ids, d_row_src, E, plane, vocab, rows, scale, g_next, eps, x, xn); break;
-    case 512: hipLaunchKernelGGL(embed_gather_kernel<2>, grid, block, 0, s, d_ids, d_row_src, E, plane, vocab, rows, scale, g_next, eps, x, xn); break;
-    case 768: hipLaunchKernelGGL(embed_gather_kernel<3>, grid, block, 0, s, d_ids, d_row_src, E, plane, vocab, rows, scale, g_next, eps, x, xn); break;
-    case 1024: hipLaunchKernelGGL(embed_gather_kernel<4>, grid, block, 0, s, d_ids, d_row_src, E, plane, vocab, rows, scale, g_next, eps, x, xn); break;
+    case 256: hipLaunchKernelGGL(embed_gather_kernel<1>, grid, block, 0, s, d_ids, d_row_src, E, plane, vocab, rows, scale, g_next, eps, x, xn, split, xs, xs_scale); break;
+    case 512: hipLaunchKernelGGL(embed_gather_kernel<2>, grid, block, 0, s, d_ids, d_row_src, E, plane, vocab, rows, scale, g_next, eps, x, xn, split, xs, xs_scale); break;
+    case 768: hipLaunchKernelGGL(embed_gather_kernel<3>, grid, block, 0, s, d_ids, d_row_src, E, plane, vocab, rows, scale, g_next, eps, x, xn, split, xs, xs_scale); break;
+    case 1024: hipLaunchKernelGGL(embed_gather_kernel<4>, grid, block, 0, s, d_ids, d_row_src, E, plane, vocab, rows, scale, g_next, eps, x, xn, split, xs, xs_scale); break;
     default: return set_error(ctx, FA_ERR_UNSUPPORTED, "gemma: hidden size %d not in {256,512,768,1024}", d);
   }
   FA_CHECK_LAUNCH(ctx);
@@ -666,7 +671,7 @@ int launch_embed_gather(fa_ctx* ctx, const int32_t* d_ids, const int32_t* d_row_
 
 int launch_residual_norm(fa_ctx* ctx, const float* o, float* x, float* xn, int64_t rows, int32_t d,
                          const float* g_post, const float* g_next, float eps, hipStream_t s, const float* o2,
-                         float scale, int n2, int64_t pstride) {
+                         float scale, int n2, int64_t pstride, float split) {
   if (rows == 0) return FA_OK;
   if (o2 && (n2 < 1 || n2 > 3)) return set_error(ctx, FA_ERR_ARG, "residual norm: %d extra K parts (1..3)", n2);
   // a short batch (C1: 128 rows) takes one row per workgroup, spread over
@@ -677,10 +682,10 @@ int launch_residual_norm(fa_ctx* ctx, const float* o, float* x, float* xn, int64
   const int per = rows <= 4LL * cus ? 1 : 4;
   dim3 grid(blocks_for(rows, per)), block(64 * per);
   switch (d) {
-    case 256: hipLaunchKernelGGL(residual_norm_kernel<1>, grid, block, 0, s, o, o2, n2, pstride, x, xn, rows, g_post, g_next, eps, scale); break;
-    case 512: hipLaunchKernelGGL(residual_norm_kernel<2>, grid, block, 0, s, o, o2, n2, pstride, x, xn, rows, g_post, g_next, eps, scale); break;
-    case 768: hipLaunchKernelGGL(residual_norm_kernel<3>, grid, block, 0, s, o, o2, n2, pstride, x, xn, rows, g_post, g_next, eps, scale); break;
-    case 1024: hipLaunchKernelGGL(residual_norm_kernel<4>, grid, block, 0, s, o, o2, n2, pstride, x, xn, rows, g_post, g_next, eps, scale); break;
+    case 256: hipLaunchKernelGGL(residual_norm_kernel<1>, grid, block, 0, s, o, o2, n2, pstride, x, xn, rows, g_post, g_next, eps, scale, split); break;
+    case 512: hipLaunchKernelGGL(residual_norm_kernel<2>, grid, block, 0, s, o, o2, n2, pstride, x, xn, rows, g_post, g_next, eps, scale, split); break;
+    case 768: hipLaunchKernelGGL(residual_norm_kernel<3>, grid, block, 0, s, o, o2, n2, pstride, x, xn, rows, g_post, g_next, eps, scale, split); break;
+    case 1024: hipLaunchKernelGGL(residual_norm_kernel<4>, grid, block, 0, s, o, o2, n2, pstride, x, xn, rows, g_post, g_next, eps, scale, split); break;
     default: return set_error(ctx, FA_ERR_UNSUPPORTED, "gemma: hidden size %d not in {256,512,768,1024}", d);
   }
   FA_CHECK_LAUNCH(ctx);

@@ -37,6 +37,9 @@
  *                               kernel (bf16 weights widened, float32 weights without the
  *                               three-plane rewrite)
  *   FA_ATTN_DENSE=0             fa_attention on the per-row kernel for every head dim
+ *   FA_GEMM_H2=0                the encoder's products on the three-term bf16 kernels (also
+ *                               implied by FA_GEMM_MFMA=f32 and FA_GEMM_XTILE)
+ *   FA_GEMM_HTILE=128x128|64x128|128x256|small   force a split-fp16 product tile
  *   FA_GEMM_KSPLIT=1            no K-split products in the encoder (also implied by
  *                               FA_GEMM_MFMA=f32)
  *   FA_MICROBATCH=0|<rows>      micro-batches off / from this many tokens (2048)
@@ -379,8 +382,8 @@ int fa_gemma_embed_ids(fa_model* m, const int32_t* ids, const int32_t* lengths, 
 /* Same computation on device-resident data: d_ids [B x T] on the device,
  * lengths on the HOST (they set the launch shapes), d_out [B x dim] on the
  * device. Enqueues on fa_stream(ctx) and returns without waiting. From
- * 2 048 tokens on, the layers of two to four token-balanced groups of
- * sequences (four for long sequences, two from 16 384 tokens, else three)
+ * 2 048 tokens on, the layers of two or three token-balanced groups of
+ * sequences (two for long sequences and from 24 576 tokens, else three)
  * run on the model's own extra streams, forked from and joined back into
  * fa_stream(ctx), so the call stays ordered on that stream. */
 int fa_gemma_embed_ids_dev(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B, int32_t T,
