@@ -323,7 +323,7 @@ __global__ __launch_bounds__(DL_NT) void attention_varlen_kernel(VarlenParams p)
 template <int HD>
 __global__ __launch_bounds__(256) void attention_combine_kernel(const float* __restrict__ part, int kparts,
                                                                 int64_t rows, int64_t row_off, int64_t n, int H,
-                                                                float* __restrict__ out, float split) {
+                                                                float* __restrict__ out, float scale, int split) {
   // rows: the partial buffers' row count; this launch sums rows row_off ..
   // row_off + n - 1 of them into out's rows 0 .. n - 1
   const int64_t lid = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);  // local row * H + head
@@ -366,22 +366,23 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const float* __r
         for (int e = 0; e < 4; e++) acc[c][e] += w * ov[q][c][e];
     }
   }
-  const float inv = 1.f / Lsum;
+  const float inv = scale / Lsum;
   float* dst = out + lrow * OW + h * HD + lane * 4;
 #pragma unroll
   for (int c = 0; c < HD / 256; c++) {
     f32x4 o;
 #pragma unroll
     for (int e = 0; e < 4; e++) o[e] = acc[c][e] * inv;
-    if (split != 0.f) store_split4_lanes(out + lrow * OW, h * HD + lane * 4 + c * 256, o * split);
+    if (split) store_split4_lanes(out + lrow * OW, h * HD + lane * 4 + c * 256, o);
     else *reinterpret_cast<f32x4*>(dst + c * 256) = o;
   }
 }
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return *reinterpret_cast<const bf16x8*>(&v); }
+__device__ __forceinline__ f16x8 as_f16x8(u32x4 v) { return __builtin_bit_cast(f16x8, v); }
 
 // ---- split-bf16 model-path kernel over key/value tile images (head_dim 256) -----
 // attention_tiles_kernel computes attention_varlen_kernel<256>'s result on
@@ -436,8 +437,12 @@ __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return *reinterpret_cast<
 // load is conditional), then P.V of tile tt-1 with tile tt's softmax spread
 // among its blocks.
 constexpr int TL_KEYS = 32;              // keys per tile
-constexpr int TL_IMG = 3 * 32 * 256;     // bf16 per key or value image
-constexpr float TL_TAU = 8.f;            // lazy-maximum slack
+constexpr int TL_IMG = 2 * 32 * 256;     // fp16 per key or value image
+constexpr float TL_TAU = 4.f;            // lazy-maximum slack
+// Weights are held times 2^10: at most e^4 2^10 < 2^16, and the fp16 terms
+// of one are exact to 2^-35 of the row's sum (O and the sum carry the factor,
+// which the final division takes out).
+constexpr float TL_WEXP = 10.f;
 
 struct TilesParams {
   const float* qkv;
@@ -460,21 +465,34 @@ struct TilesParams {
   const float* gq;
   const float *cs, *sn;
   float eps;
-  float split;  // != 0: out holds the split terms (split2) of its values times split
+  float q_scale;  // q's power of two (scale is the score scale without it and the keys')
+  // out = O * out_scale (O carries the values' power of two), as floats or as
+  // split terms (split2)
+  float out_scale;
+  int split;
 };
 
-__device__ __forceinline__ void split_pack8(const f32x4& x0, const f32x4& x1, bf16x8& t0, bf16x8& t1, bf16x8& t2) {
-  uint32_t h[8], m[8], l[8];
+// Eight values as two fp16 terms, hi + lo (lo = fp16(x - hi), unscaled).
+__device__ __forceinline__ void split_pack8(const f32x4& x0, const f32x4& x1, f16x8& hi, f16x8& lo) {
 #pragma unroll
   for (int e = 0; e < 8; e++) {
-    const Split3 sp = split3(e < 4 ? x0[e] : x1[e - 4]);
-    h[e] = sp.h;
-    m[e] = sp.m;
-    l[e] = sp.l;
+    const float x = e < 4 ? x0[e] : x1[e - 4];
+    hi[e] = (_Float16)x;
+    lo[e] = (_Float16)(x - (float)hi[e]);
   }
-  t0 = as_bf16x8(u32x4{pack_hi16(h[0], h[1]), pack_hi16(h[2], h[3]), pack_hi16(h[4], h[5]), pack_hi16(h[6], h[7])});
-  t1 = as_bf16x8(u32x4{pack_hi16(m[0], m[1]), pack_hi16(m[2], m[3]), pack_hi16(m[4], m[5]), pack_hi16(m[6], m[7])});
-  t2 = as_bf16x8(u32x4{pack_hi16(l[0], l[1]), pack_hi16(l[2], l[3]), pack_hi16(l[4], l[5]), pack_hi16(l[6], l[7])});
+}
+
+// Two probabilities' terms, packed: hi pair and lo pair.
+__device__ __forceinline__ void split_pair(float w0, float w1, uint32_t& hi, uint32_t& lo) {
+  const f16x2 h = {(_Float16)w0, (_Float16)w1};
+  const f16x2 l = {(_Float16)(w0 - (float)h[0]), (_Float16)(w1 - (float)h[1])};
+  hi = __builtin_bit_cast(uint32_t, h);
+  lo = __builtin_bit_cast(uint32_t, l);
+}
+
+// A probability times 2^TL_WEXP; inputs below -87 give exactly 0 (exp_flush).
+__device__ __forceinline__ float weight(float x) {
+  return x < -87.f ? 0.f : __builtin_amdgcn_exp2f(fmaf(x, 1.4426950408889634f, TL_WEXP));
 }
 
 // TL_W waves of 16 rows: 8 (128-row items, two waves per SIMD) or 4
@@ -501,8 +519,9 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
   // operand reads one step ahead of the MFMAs that use them (12 more
   // VGPRs): the wave pairs' kernel has the registers to spare
   constexpr bool TL_PF = DS == 2;
-  constexpr int TERM = TL_IMG / 3;  // bf16 per term of an image
-  __shared__ __attribute__((aligned(16))) uint16_t Ks[TL_IMG];
+  constexpr int TERM = TL_IMG / 2;  // fp16 per term of an image
+  __shared__ __attribute__((aligned(16))) uint16_t Ks0[TL_IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t Ks1[TL_IMG];
   __shared__ __attribute__((aligned(16))) uint16_t Vs0[TL_IMG];
   __shared__ __attribute__((aligned(16))) uint16_t Vs1[TL_IMG];
   // partial scores of each wave (two 16-key blocks x 64 lanes), DS = 2
@@ -546,10 +565,10 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
 
   const uint16_t* img0 = p.img + ((int64_t)seq_tile * p.Hkv + hk) * (2 * TL_IMG);
   const int64_t tstride = (int64_t)p.Hkv * 2 * TL_IMG;
-  // 48 loads of 1 KB per image, six per wave
+  // 32 loads of 1 KB per image
   auto issue = [&](const uint16_t* src, uint16_t* dst) {
 #pragma unroll
-    for (int j = 0; j < 48 / TL_W; j++) {
+    for (int j = 0; j < 32 / TL_W; j++) {
       const int c = wave + TL_W * j;
       __builtin_amdgcn_global_load_lds(src + c * 512 + lane * 8, (__attribute__((address_space(3))) void*)&dst[c * 512],
                                        16, 0, 0);
@@ -567,9 +586,9 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
   if (k_first) {
     const uint16_t* src = img0 + min(tb, te - 1) * tstride;
 #pragma unroll
-    for (int j = 0; j < 96 / TL_W; j++) {
+    for (int j = 0; j < 64 / TL_W; j++) {
       const int c = (wave - TL_W / 2) + (TL_W / 2) * j;
-      __builtin_amdgcn_global_load_lds(src + c * 512 + lane * 8, (__attribute__((address_space(3))) void*)&Ks[c * 512],
+      __builtin_amdgcn_global_load_lds(src + c * 512 + lane * 8, (__attribute__((address_space(3))) void*)&Ks0[c * 512],
                                        16, 0, 0);
     }
   }
@@ -582,18 +601,19 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
     if constexpr (DS == 2) dl_barrier<0xC07F>();  // the pairs' q row exchange below
     if (tb < te) {
       for (int tt = tb; tt < te; tt++) {
-        dl_barrier<0x0F70>();
-        issue(img0 + tt * tstride + TL_IMG, ((tt - tb) & 1) ? Vs1 : Vs0);
-        dl_barrier<0xC07F>();
-        issue(img0 + min(tt + 1, te - 1) * tstride, Ks);
+        const bool odd = (tt - tb) & 1;
+        dl_barrier<0x0070>();
+        issue(img0 + tt * tstride + TL_IMG, odd ? Vs1 : Vs0);
+        issue(img0 + min(tt + 1, te - 1) * tstride, odd ? Ks0 : Ks1);
+        if constexpr (DS == 2) dl_barrier<0xC07F>();
       }
-      dl_barrier<0x0F70>();
+      dl_barrier<0x0070>();
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): a first image issued above
     return;
   }
 
-  bf16x8 qt[3][NC];
+  f16x8 qt[2][NC];
   if constexpr (DS == 2) {
     // Wave pairs: each wave norms (RMSNorm, gain) and rotates (RoPE at the
     // token's position) 8 of the pair's 16 rows, all 256 dims: lane l takes
@@ -641,8 +661,8 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
     ss = ss + dpp_f32<0xB1>(ss);   // quad_perm [1, 0, 3, 2]
     ss = ss + dpp_f32<0x4E>(ss);   // quad_perm [2, 3, 0, 1]
     ss = ss + dpp_f32<0x141>(ss);  // row_half_mirror
-    const float inv = rms_inv(ss, HD, p.eps);
-    f32x4* qs = reinterpret_cast<f32x4*>((rbw < 3 ? Vs0 : Vs1) + (rbw % 3) * 8192);  // the pair's 16 rows
+    const float inv = rms_inv(ss, HD, p.eps) * p.q_scale;
+    f32x4* qs = reinterpret_cast<f32x4*>((rbw < 2 ? Vs0 : Vs1) + (rbw & 1) * 8192);  // the pair's 16 rows
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       f32x4 yl, yh;
@@ -663,7 +683,7 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
       const int k = 8 * (NC * hf + c) + 2 * g;
       f32x4 x0 = qs[lq * 64 + (k ^ lq)], x1 = qs[lq * 64 + ((k + 1) ^ lq)];
       if (!qvalid) x0 = x1 = f32x4{0.f, 0.f, 0.f, 0.f};
-      split_pack8(x0, x1, qt[0][c], qt[1][c], qt[2][c]);
+      split_pack8(x0, x1, qt[0][c], qt[1][c]);
     }
   } else {
     // q normed (RMSNorm, gain) and rotated (RoPE at the token's position)
@@ -683,7 +703,7 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
 #pragma unroll
       for (int e = 0; e < 8; e++) ss = fmaf(x[c][e >> 2][e & 3], x[c][e >> 2][e & 3], ss);
     ss = rows4_sum(ss);
-    const float inv = rms_inv(ss, HD, p.eps);
+    const float inv = rms_inv(ss, HD, p.eps) * p.q_scale;
     const float* gr = p.gq + 8 * g;
     const float* cr = p.cs + (int64_t)tok * (HD / 2) + 8 * g;
     const float* sr = p.sn + (int64_t)tok * (HD / 2) + 8 * g;
@@ -709,7 +729,7 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
     for (int c = 0; c < NC; c++) {
       f32x4 x0 = x[c][0], x1 = x[c][1];
       if (!qvalid) x0 = x1 = f32x4{0.f, 0.f, 0.f, 0.f};
-      split_pack8(x0, x1, qt[0][c], qt[1][c], qt[2][c]);
+      split_pack8(x0, x1, qt[0][c], qt[1][c]);
     }
   }
 
@@ -726,32 +746,28 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
     khi = min(L, tok + p.window);
   }
 
-  // The six term products of one 16-key block and one 32-dim chunk, in a
-  // fixed order (smallest terms first), accumulated into s.
-  auto qk_chunk = [&](f32x4& s, const bf16x8& k0, const bf16x8& k1, const bf16x8& k2, int c) {
-    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, qt[0][c], s, 0, 0, 0);
-    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qt[2][c], s, 0, 0, 0);
-    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qt[1][c], s, 0, 0, 0);
-    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qt[0][c], s, 0, 0, 0);
-    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qt[1][c], s, 0, 0, 0);
-    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qt[0][c], s, 0, 0, 0);
+  // The three term products of one 16-key block and one 32-dim chunk (lo . lo,
+  // below 2^-24 of the product, is dropped), smallest first, into s.
+  auto qk_chunk = [&](f32x4& s, const f16x8& k0, const f16x8& k1, int c) {
+    s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, qt[0][c], s, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qt[1][c], s, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qt[0][c], s, 0, 0, 0);
   };
   auto qk = [&](const uint16_t* Kc, f32x4 (&sacc)[2]) {
+    sacc[0] = f32x4{0.f, 0.f, 0.f, 0.f};
+    sacc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
     if constexpr (TL_PF) {
       // The two key blocks' chains interleaved (each MFMA's accumulator was
       // written two MFMAs earlier, not one), and the key terms of chunk c + 1
-      // read while chunk c's products run. Each block's products keep the
-      // order above, so the scores are the same bits.
-      sacc[0] = f32x4{0.f, 0.f, 0.f, 0.f};
-      sacc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-      bf16x8 kt[2][2][3];  // [chunk parity][key block][term]
-      auto rd = [&](int c, bf16x8 (&dst)[2][3]) {
+      // read while chunk c's products run.
+      f16x8 kt[2][2][2];  // [chunk parity][key block][term]
+      auto rd = [&](int c, f16x8 (&dst)[2][2]) {
 #pragma unroll
         for (int kb = 0; kb < 2; kb++) {
           const int key = 16 * kb + lq;
           const uint16_t* kr = Kc + key * HD + ((4 * (NC * hf + c) + g) ^ key) * 8;
 #pragma unroll
-          for (int t = 0; t < 3; t++) dst[kb][t] = *reinterpret_cast<const bf16x8*>(kr + t * TERM);
+          for (int t = 0; t < 2; t++) dst[kb][t] = *reinterpret_cast<const f16x8*>(kr + t * TERM);
         }
       };
       rd(0, kt[0]);
@@ -760,45 +776,42 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
         if (c + 1 < NC) rd(c + 1, kt[(c + 1) & 1]);
         __builtin_amdgcn_sched_barrier(0);  // the next chunk's reads issue before this chunk's products
         const int b = c & 1;
-        sacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][0][2], qt[0][c], sacc[0], 0, 0, 0);
-        sacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][1][2], qt[0][c], sacc[1], 0, 0, 0);
-        sacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][0][0], qt[2][c], sacc[0], 0, 0, 0);
-        sacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][1][0], qt[2][c], sacc[1], 0, 0, 0);
-        sacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][0][1], qt[1][c], sacc[0], 0, 0, 0);
-        sacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][1][1], qt[1][c], sacc[1], 0, 0, 0);
-        sacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][0][1], qt[0][c], sacc[0], 0, 0, 0);
-        sacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][1][1], qt[0][c], sacc[1], 0, 0, 0);
-        sacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][0][0], qt[1][c], sacc[0], 0, 0, 0);
-        sacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][1][0], qt[1][c], sacc[1], 0, 0, 0);
-        sacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][0][0], qt[0][c], sacc[0], 0, 0, 0);
-        sacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[b][1][0], qt[0][c], sacc[1], 0, 0, 0);
+        sacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt[b][0][1], qt[0][c], sacc[0], 0, 0, 0);
+        sacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt[b][1][1], qt[0][c], sacc[1], 0, 0, 0);
+        sacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt[b][0][0], qt[1][c], sacc[0], 0, 0, 0);
+        sacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt[b][1][0], qt[1][c], sacc[1], 0, 0, 0);
+        sacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt[b][0][0], qt[0][c], sacc[0], 0, 0, 0);
+        sacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt[b][1][0], qt[0][c], sacc[1], 0, 0, 0);
       }
     } else {
 #pragma unroll
       for (int kb = 0; kb < 2; kb++) {
-        sacc[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
         const int key = 16 * kb + lq;
         const uint16_t* kr = Kc + key * HD;
 #pragma unroll
         for (int c = 0; c < NC; c++) {
           const int pos = ((4 * (NC * hf + c) + g) ^ key) * 8;
-          const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(kr + pos);
-          const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(kr + TERM + pos);
-          const bf16x8 k2 = *reinterpret_cast<const bf16x8*>(kr + 2 * TERM + pos);
-          qk_chunk(sacc[kb], k0, k1, k2, c);
+          const f16x8 k0 = *reinterpret_cast<const f16x8*>(kr + pos);
+          const f16x8 k1 = *reinterpret_cast<const f16x8*>(kr + TERM + pos);
+          qk_chunk(sacc[kb], k0, k1, c);
         }
       }
     }
   };
-  // O^T += V^T . P^T for one tile (terms b0, b1, b2 of the probabilities)
   // the value terms of block db (with TL_PF read one block ahead)
-  auto vread = [&](const uint16_t* Vc, int db, bf16x8 (&dst)[3]) {
+  auto vread = [&](const uint16_t* Vc, int db, f16x8 (&dst)[2]) {
     const uint16_t* vr = Vc + (16 * (NDB * hf + db) + lq) * 32 + (g ^ vsw) * 8;
 #pragma unroll
-    for (int t = 0; t < 3; t++) dst[t] = *reinterpret_cast<const bf16x8*>(vr + t * TERM);
+    for (int t = 0; t < 2; t++) dst[t] = *reinterpret_cast<const f16x8*>(vr + t * TERM);
   };
-  auto pv = [&](const uint16_t* Vc, const bf16x8& b0, const bf16x8& b1, const bf16x8& b2) {
-    bf16x8 vt[2][3];
+  auto pv_block = [&](int db, const f16x8 (&v)[2], const f16x8& b0, const f16x8& b1) {
+    oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v[1], b0, oacc[db], 0, 0, 0);
+    oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v[0], b1, oacc[db], 0, 0, 0);
+    oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v[0], b0, oacc[db], 0, 0, 0);
+  };
+  // O^T += V^T . P^T for one tile (terms b0, b1 of the probabilities)
+  auto pv = [&](const uint16_t* Vc, const f16x8& b0, const f16x8& b1) {
+    f16x8 vt[2][2];
     if constexpr (TL_PF) vread(Vc, 0, vt[0]);
 #pragma unroll
     for (int db = 0; db < NDB; db++) {
@@ -808,27 +821,24 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
       } else {
         vread(Vc, db, vt[db & 1]);
       }
-      const bf16x8 v0 = vt[db & 1][0], v1 = vt[db & 1][1], v2 = vt[db & 1][2];
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v2, b0, oacc[db], 0, 0, 0);
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, b2, oacc[db], 0, 0, 0);
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, b1, oacc[db], 0, 0, 0);
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, b0, oacc[db], 0, 0, 0);
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, b1, oacc[db], 0, 0, 0);
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, b0, oacc[db], 0, 0, 0);
+      pv_block(db, vt[db & 1], b0, b1);
     }
+  };
+  // the scaled, masked score e of tile tt
+  auto score = [&](int tt, const f32x4 (&sacc)[2], int e) -> float {
+    const int j = tt * TL_KEYS + 16 * (e >> 2) + 4 * g + (e & 3);
+    const bool ok = (unsigned)(j - klo) < (unsigned)(khi - klo);
+    return ok ? sacc[e >> 2][e & 3] * p.scale : -INFINITY;
   };
   // softmax of tile tt's scores against the lazy offset: the new offset and
   // the scale alpha for what O and the sum held, this tile's probability
   // terms and their sum
-  auto softmax = [&](int tt, const f32x4 (&sacc)[2], float& alpha, bool& moved, bf16x8& b0, bf16x8& b1,
-                     bf16x8& b2) {
+  auto softmax = [&](int tt, const f32x4 (&sacc)[2], float& alpha, bool& moved, f16x8& b0, f16x8& b1) {
     float t[8];
     float tmax = -INFINITY;
 #pragma unroll
     for (int e = 0; e < 8; e++) {
-      const int j = tt * TL_KEYS + 16 * (e >> 2) + 4 * g + (e & 3);
-      const bool ok = (unsigned)(j - klo) < (unsigned)(khi - klo);
-      t[e] = ok ? sacc[e >> 2][e & 3] * p.scale : -INFINITY;
+      t[e] = score(tt, sacc, e);
       tmax = fmaxf(tmax, t[e]);
     }
     tmax = rows4_max(tmax);
@@ -837,65 +847,52 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
     const float mn = need ? tmax : m_run;
     alpha = exp_flush(m_run - mn);  // 1 where the offset stays, 0 for the first valid tile
     m_run = mn;
-    uint32_t ph[8], pm[8], pl[8];
+    uint32_t ph[4], pl[4];
     float psum = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const float pv_ = exp_flush(t[e] - mn);  // masked keys: -inf, flushed to 0
-      psum += pv_;
-      const Split3 sp = split3(pv_);
-      ph[e] = sp.h;
-      pm[e] = sp.m;
-      pl[e] = sp.l;
+    for (int e = 0; e < 8; e += 2) {
+      const float w0 = weight(t[e] - mn), w1 = weight(t[e + 1] - mn);  // masked keys: -inf, flushed to 0
+      psum += w0;
+      psum += w1;
+      split_pair(w0, w1, ph[e / 2], pl[e / 2]);
     }
     l_part = l_part * alpha + psum;
-    b0 = as_bf16x8(u32x4{pack_hi16(ph[0], ph[1]), pack_hi16(ph[2], ph[3]), pack_hi16(ph[4], ph[5]),
-                         pack_hi16(ph[6], ph[7])});
-    b1 = as_bf16x8(u32x4{pack_hi16(pm[0], pm[1]), pack_hi16(pm[2], pm[3]), pack_hi16(pm[4], pm[5]),
-                         pack_hi16(pm[6], pm[7])});
-    b2 = as_bf16x8(u32x4{pack_hi16(pl[0], pl[1]), pack_hi16(pl[2], pl[3]), pack_hi16(pl[4], pl[5]),
-                         pack_hi16(pl[6], pl[7])});
+    b0 = as_f16x8(u32x4{ph[0], ph[1], ph[2], ph[3]});
+    b1 = as_f16x8(u32x4{pl[0], pl[1], pl[2], pl[3]});
   };
 
-  // Software pipeline, iteration tt: [barrier: K(tt), V(tt-1) landed; every
-  // wave done with iteration tt-1] load V(tt); S(tt) = K(tt).Q^T; [barrier:
-  // every wave done with the keys] load K(tt+1) (the last again past the
-  // end); P.V of tile tt-1 with the softmax of tile tt written between its
-  // blocks in four stages (each stage's results pinned where it is written,
-  // so the VALU work sits among the MFMAs instead of after them), then O's
-  // rescale, which must see tile tt-1's terms. Then P.V of the last tile. One key buffer and two
-  // value buffers (144 KB).
-  bf16x8 pb0, pb1, pb2;  // tile tt-1's probability terms
-  // Tile tb + i's values go to Vs0 for even i, Vs1 for odd i: every LDS
-  // access names its buffer statically (the compiler then keeps the other
-  // buffer's loads in flight across the reads).
-  // barrier, this tile's value loads into Vn, scores, barrier, the next
-  // tile's key loads
-  auto front = [&](int tt, uint16_t* Vn, f32x4 (&sacc)[2]) {
-    dl_barrier<0x0F70>();  // vmcnt(0): K(tt), V(tt-1) landed (own loads, then everyone's)
+  // Software pipeline, iteration tt (two key and two value buffers, 128 KB):
+  // [barrier: K(tt), V(tt-1) landed; every wave done with iteration tt-1]
+  // load V(tt) and K(tt+1) (the last again past the end); S(tt) = K(tt).Q^T;
+  // P.V of tile tt-1 with the softmax of tile tt written between its blocks
+  // in stages (each stage's results pinned where it is written, so the VALU
+  // work sits among the MFMAs instead of after them), then O's rescale,
+  // which must see tile tt-1's terms. Then P.V of the last tile. With a
+  // second key buffer the next keys load during the whole iteration and a
+  // tile has one barrier (the wave pairs' exchange keeps a second one).
+  f16x8 pb0, pb1;  // tile tt-1's probability terms
+  // Tile tb + i's keys and values sit in buffers 0 for even i, 1 for odd i:
+  // every LDS access names its buffer statically (the compiler then keeps
+  // the other buffers' loads in flight across the reads).
+  auto front = [&](int tt, const uint16_t* Kc, uint16_t* Kn, uint16_t* Vn, f32x4 (&sacc)[2]) {
+    dl_barrier<0x0070>();  // vmcnt(0) lgkmcnt(0): K(tt), V(tt-1) landed (own loads, then everyone's)
     issue(img0 + tt * tstride + TL_IMG, Vn);
-    qk(Ks, sacc);
+    issue(img0 + min(tt + 1, te - 1) * tstride, Kn);
+    qk(Kc, sacc);
     if constexpr (DS == 2) {
       Xs[(2 * wave) * 64 + lane] = sacc[0];
       Xs[(2 * wave + 1) * 64 + lane] = sacc[1];
-    }
-    dl_barrier<0xC07F>();  // every wave's key reads (and partial-score writes) done; no wait for the loads
-    issue(img0 + min(tt + 1, te - 1) * tstride, Ks);
-    if constexpr (DS == 2) {  // the partner's half (it writes again only after the next barrier)
-      const int pw = wave ^ RB;
+      dl_barrier<0xC07F>();  // the partial scores written; no wait for the loads
+      const int pw = wave ^ RB;  // the partner's half (it writes again only after the next barrier)
       sacc[0] = sacc[0] + Xs[(2 * pw) * 64 + lane];
       sacc[1] = sacc[1] + Xs[(2 * pw + 1) * 64 + lane];
     }
   };
-  // P.V of tile tt-1 (terms pb*) with the softmax of tile tt (scores sacc)
-  // written between its blocks of 16 dims, in four stages, so that the
-  // VALU work sits among the MFMAs; the new terms replace pb* at the end
   auto pv_softmax = [&](const uint16_t* Vp, int tt, const f32x4 (&sacc)[2], float& alpha, bool& moved) {
     float t[8];
     float tmax = -INFINITY, mn = 0.f, psum = 0.f;
-    uint32_t ph[8], pm[8], pl[8];
-    constexpr int WPS = DS == 2 ? 2 : 1;  // weights per block in the last stage
-    bf16x8 vt[2][3];
+    uint32_t ph[4], pl[4];
+    f16x8 vt[2][2];
     if constexpr (TL_PF) vread(Vp, 0, vt[0]);
 #pragma unroll
     for (int db = 0; db < NDB; db++) {
@@ -905,19 +902,11 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
       } else {
         vread(Vp, db, vt[db & 1]);
       }
-      const bf16x8 v0 = vt[db & 1][0], v1 = vt[db & 1][1], v2 = vt[db & 1][2];
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v2, pb0, oacc[db], 0, 0, 0);
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, pb2, oacc[db], 0, 0, 0);
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, pb1, oacc[db], 0, 0, 0);
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, pb0, oacc[db], 0, 0, 0);
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, pb1, oacc[db], 0, 0, 0);
-      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, pb0, oacc[db], 0, 0, 0);
+      pv_block(db, vt[db & 1], pb0, pb1);
       if (db < 2) {  // scaled, masked scores (four per block) and the lane's maximum
 #pragma unroll
         for (int e = 4 * db; e < 4 * db + 4; e++) {
-          const int j = tt * TL_KEYS + 16 * (e >> 2) + 4 * g + (e & 3);
-          const bool ok = (unsigned)(j - klo) < (unsigned)(khi - klo);
-          t[e] = ok ? sacc[e >> 2][e & 3] * p.scale : -INFINITY;
+          t[e] = score(tt, sacc, e);
           tmax = fmaxf(tmax, t[e]);
           asm volatile("" ::"v"(t[e]));  // computed here, not sunk to the use
         }
@@ -931,32 +920,23 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
         alpha = exp_flush(m_run - mn);  // 1 where the offset stays, 0 for the first valid tile
         m_run = mn;
         asm volatile("" ::"v"(alpha), "v"(mn));
-      } else if (db >= 4 && db < 4 + 8 / WPS) {  // WPS weights (masked keys: -inf, flushed to 0) and their exact bf16 terms
-#pragma unroll
-        for (int u = 0; u < WPS; u++) {
-          const int e = (db - 4) * WPS + u;
-          const float w = exp_flush(t[e] - mn);
-          psum += w;
-          const Split3 sp = split3(w);
-          ph[e] = sp.h;
-          pm[e] = sp.m;
-          pl[e] = sp.l;
-          asm volatile("" ::"v"(ph[e]), "v"(pm[e]), "v"(pl[e]), "v"(psum));
-        }
+      } else if (db < 8) {  // two weights (masked keys: -inf, flushed to 0) and their terms
+        const int e = 2 * (db - 4);
+        const float w0 = weight(t[e] - mn), w1 = weight(t[e + 1] - mn);
+        psum += w0;
+        psum += w1;
+        split_pair(w0, w1, ph[e / 2], pl[e / 2]);
+        asm volatile("" ::"v"(ph[e / 2]), "v"(pl[e / 2]), "v"(psum));
       }
       __builtin_amdgcn_sched_barrier(0);
     }
     l_part = l_part * alpha + psum;
-    pb0 = as_bf16x8(u32x4{pack_hi16(ph[0], ph[1]), pack_hi16(ph[2], ph[3]), pack_hi16(ph[4], ph[5]),
-                          pack_hi16(ph[6], ph[7])});
-    pb1 = as_bf16x8(u32x4{pack_hi16(pm[0], pm[1]), pack_hi16(pm[2], pm[3]), pack_hi16(pm[4], pm[5]),
-                          pack_hi16(pm[6], pm[7])});
-    pb2 = as_bf16x8(u32x4{pack_hi16(pl[0], pl[1]), pack_hi16(pl[2], pl[3]), pack_hi16(pl[4], pl[5]),
-                          pack_hi16(pl[6], pl[7])});
+    pb0 = as_f16x8(u32x4{ph[0], ph[1], ph[2], ph[3]});
+    pb1 = as_f16x8(u32x4{pl[0], pl[1], pl[2], pl[3]});
   };
-  auto iter = [&](int tt, uint16_t* Vn, const uint16_t* Vp) {
+  auto iter = [&](int tt, const uint16_t* Kc, uint16_t* Kn, uint16_t* Vn, const uint16_t* Vp) {
     f32x4 sacc[2];
-    front(tt, Vn, sacc);
+    front(tt, Kc, Kn, Vn, sacc);
     float alpha;
     bool moved;
     pv_softmax(Vp, tt, sacc, alpha, moved);
@@ -968,22 +948,22 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
   if (tb < te) {
     {
       f32x4 sacc[2];
-      front(tb, Vs0, sacc);
+      front(tb, Ks0, Ks1, Vs0, sacc);
       float alpha;
       bool moved;
-      softmax(tb, sacc, alpha, moved, pb0, pb1, pb2);  // O is still zero
+      softmax(tb, sacc, alpha, moved, pb0, pb1);  // O is still zero
     }
     int tt = tb + 1;
     for (; tt + 1 < te; tt += 2) {
-      iter(tt, Vs1, Vs0);
+      iter(tt, Ks1, Ks0, Vs1, Vs0);
       __builtin_amdgcn_sched_barrier(0);  // no code motion between the two halves (register pressure)
-      iter(tt + 1, Vs0, Vs1);
+      iter(tt + 1, Ks0, Ks1, Vs0, Vs1);
     }
-    if (tt < te) iter(tt, Vs1, Vs0);
-    dl_barrier<0x0F70>();  // V(te-1) landed everywhere
+    if (tt < te) iter(tt, Ks1, Ks0, Vs1, Vs0);
+    dl_barrier<0x0070>();  // V(te-1) landed everywhere
     // the last tile's values: one P.V for either parity (no loads follow,
     // so the buffer need not be named statically here)
-    pv(((te - 1 - tb) & 1) ? Vs1 : Vs0, pb0, pb1, pb2);
+    pv(((te - 1 - tb) & 1) ? Vs1 : Vs0, pb0, pb1);
   } else {
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the first image issued above
   }
@@ -1002,11 +982,11 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
     }
     return;
   }
-  const float inv = 1.f / l_tot;
+  const float inv = p.out_scale / l_tot;
   float* orow = p.out + (start + tok) * OW + (int64_t)head * HD + 16 * NDB * hf;
-  if (p.split != 0.f) {
+  if (p.split) {
 #pragma unroll
-    for (int db = 0; db < NDB; db++) store_split4(orow, 16 * db + 4 * g, oacc[db] * inv * p.split);
+    for (int db = 0; db < NDB; db++) store_split4(orow, 16 * db + 4 * g, oacc[db] * inv);
   } else {
 #pragma unroll
     for (int db = 0; db < NDB; db++) *reinterpret_cast<f32x4*>(orow + 16 * db + 4 * g) = oacc[db] * inv;
@@ -1291,10 +1271,10 @@ int launch_attention_varlen_items(fa_ctx* ctx, const AttnVarlenArgs& a, const in
     const dim3 g2((unsigned)((a.rows * a.H + per - 1) / per)), b2(64 * per);
     if (a.D == 256)
       hipLaunchKernelGGL(attention_combine_kernel<256>, g2, b2, 0, s, a.part, a.kparts, a.rows, (int64_t)0, a.rows,
-                         a.H, a.out, a.split);
+                         a.H, a.out, a.split != 0.f ? a.split : 1.f, a.split != 0.f ? 1 : 0);
     else
       hipLaunchKernelGGL(attention_combine_kernel<512>, g2, b2, 0, s, a.part, a.kparts, a.rows, (int64_t)0, a.rows,
-                         a.H, a.out, a.split);
+                         a.H, a.out, a.split != 0.f ? a.split : 1.f, a.split != 0.f ? 1 : 0);
   }
   FA_CHECK_LAUNCH(ctx);
   return FA_OK;
@@ -1324,7 +1304,11 @@ int launch_attention_tiles(fa_ctx* ctx, const AttnTilesArgs& a, const int32_t* d
   p.qkv = a.qkv; p.img = a.img; p.out = a.out; p.items = d_items; p.ext = a.item_ext;
   p.H = a.H; p.Hkv = a.Hkv; p.window = a.window; p.scale = a.scale; p.row0 = a.row0;
   p.kparts = a.kparts; p.rows = a.rows; p.part = a.part;
-  p.gq = a.gq; p.cs = a.cos_t; p.sn = a.sin_t; p.eps = a.eps; p.split = a.split;
+  p.gq = a.gq; p.cs = a.cos_t; p.sn = a.sin_t; p.eps = a.eps;
+  p.q_scale = a.q_scale;
+  p.scale = a.scale / (a.q_scale * a.k_scale);
+  p.out_scale = (a.split != 0.f ? a.split : 1.f) / a.v_scale;
+  p.split = a.split != 0.f ? 1 : 0;
   const dim3 grid((unsigned)((int64_t)n_items * a.kparts));
   if (a.waves == 4 && tiles_pairs())
     hipLaunchKernelGGL((attention_tiles_kernel<8, 2>), grid, dim3(64 * 8), 0, s, p);
@@ -1334,7 +1318,7 @@ int launch_attention_tiles(fa_ctx* ctx, const AttnTilesArgs& a, const int32_t* d
     hipLaunchKernelGGL((attention_tiles_kernel<8, 1>), grid, dim3(64 * 8), 0, s, p);
   if (a.kparts > 1)
     hipLaunchKernelGGL(attention_combine_kernel<256>, dim3((unsigned)((a.nrows * a.H + 3) / 4)), dim3(256), 0, s,
-                       a.part, a.kparts, a.rows, a.row0, a.nrows, a.H, a.out, a.split);
+                       a.part, a.kparts, a.rows, a.row0, a.nrows, a.H, a.out, p.out_scale, p.split);
   FA_CHECK_LAUNCH(ctx);
   return FA_OK;
 }

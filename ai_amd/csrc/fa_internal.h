@@ -336,17 +336,18 @@ int launch_attention_varlen_items(fa_ctx* ctx, const AttnVarlenArgs& a, const in
                                   hipStream_t s);
 // Queries per workgroup of the varlen kernel (the item granularity).
 int attention_varlen_qblock();
-// head_dim 256, split-bf16 attention over key/value tile images: writes,
+// head_dim 256, split-fp16 attention over key/value tile images: writes,
 // for tiles [t_lo, t_lo + tiles), the key image (keys normed, gained,
 // rotated) and value image of each (tile, kv head) into img
-// [tile][Hkv][2][3*32*256] bf16. Every sequence starts a tile; tile tt
+// [tile][Hkv][2][2*32*256] fp16 (two terms of keys times k_scale and values
+// times v_scale, powers of two that keep both inside fp16's range). Every sequence starts a tile; tile tt
 // holds up to 32 consecutive tokens of one sequence, described by
 // d_tile_ext[4 tt ..] (16-byte aligned): its first token's packed row, its
 // token count (1..32), its first token's position in the sequence (for
 // RoPE), 0. qkv starts at packed row row0.
 int launch_kv_tiles(fa_ctx* ctx, const float* qkv, int64_t row0, int32_t H, int32_t Hkv, const float* gk, float eps,
                     const float* cos_t, const float* sin_t, const int32_t* d_tile_ext, int32_t t_lo, int32_t tiles,
-                    uint16_t* img, hipStream_t s, bool norm_v = false);
+                    uint16_t* img, hipStream_t s, bool norm_v, float k_scale, float v_scale);
 
 struct AttnTilesArgs {
   const float* qkv;       // raw q read here (rows of the launch start at packed row row0)
@@ -372,6 +373,8 @@ struct AttnTilesArgs {
   // on eight waves in head-dimension pairs unless FA_ATTN_PAIRS=0)
   int32_t waves = 8;
   float split = 0.f;  // as AttnVarlenArgs::split
+  // powers of two of q, of the key images and of the value images
+  float q_scale = 1.f, k_scale = 1.f, v_scale = 1.f;
 };
 // d_items holds n_items triples (sequence, first row, kv head): one item per
 // attention_tiles_rows(a.waves) rows (token, query head of the kv head's

@@ -85,6 +85,8 @@ struct Layer {
   // attention output, GeGLU output; variant 2: the residual stream before
   // the per-layer-input block and the block's gated input)
   float s_in = 0, s_att = 0, s_ffn = 0, s_gu = 0, s_x = 0, s_ple = 0;
+  // and of the tile attention's q and key images (its value images: s_att)
+  float s_q = 0, s_k = 0;
 };
 
 struct KernelStat {
@@ -123,6 +125,9 @@ struct fa_model {
   // the layers' products run on split activations (prepare_h2): every layer
   // matrix is exact in fp16 and every operand's range is known
   bool h2 = false;
+  // the split-fp16 tile attention can run (prepare_h2: every head_dim-256
+  // layer's q, keys and values have a known range)
+  bool tiles = false;
   float s_x0 = 0;  // variant 2: scale of the scaled embeddings
   // workspace
   fa::DevBuf ws, plan_dev;
@@ -179,22 +184,24 @@ void set_b(GemmArgs& g, const Mat& w, int64_t row0 = 0) {
 }
 
 // Decides whether the layers' products can run on split activations
-// (gemm_h2.hip) and prepares them: m->h2. It needs
-//  - every layer matrix bf16-exact (terms == 1) and exact in fp16 after one
-//    power of two for the matrix (its largest value just below 2^15: values
-//    down to 2^-32 of that keep all their bits);
-//  - a bound for every activation operand, from which its power of two is
-//    taken (the bound just below 2^15): a normed row has 2-norm at most
-//    sqrt(d) max|gain|, so |x_j| is at most that and |w . x| at most |w|
-//    times it; attention outputs are convex combinations of values; |gelu(g)
-//    u| <= |g| |u|; the residual stream is a sum of normed rows. The split
-//    then keeps 23 bits down to 2^-29 of the bound (device_math.h). Gains
-//    whose largest value is more than 64 times their root mean square would
-//    put typical values too far below the bounds: those models keep the
-//    three-term products, as do non-finite weights.
+// (gemm_h2.hip) and the head_dim-256 layers on the tile attention, and
+// prepares both: m->h2, m->tiles. They need
+//  - a bound for every split operand, from which its power of two is taken
+//    (the bound just below 2^15): a normed row has 2-norm at most sqrt(d)
+//    max|gain|, so |x_j| is at most that and |w . x| at most |w| times it;
+//    attention outputs are convex combinations of values; |gelu(g) u| <= |g|
+//    |u|; the residual stream is a sum of normed rows. The activations'
+//    split then keeps 23 bits down to 2^-29 of the bound (split2,
+//    device_math.h), the attention's, whose lo terms have no scale of their
+//    own, down to 2^-18. Gains whose largest value is far above their root
+//    mean square would put typical values too far below the bounds (64 times
+//    for the products and values, 1 024 for q and k): those models keep the
+//    three-term products and the fp32 attention, as do non-finite weights;
+//  - for the products, every layer matrix bf16-exact (terms == 1) and exact
+//    in fp16 after one power of two for the matrix (its largest value just
+//    below 2^15: values down to 2^-32 of that keep all their bits).
 int prepare_h2(fa_model* m) {
-  m->h2 = false;
-  if (!gemm_h2_enabled()) return FA_OK;
+  m->h2 = m->tiles = false;
   fa_ctx* ctx = m->ctx;
   const fa_gemma_config& c = m->cfg;
   const bool v2 = m->variant == 2;
@@ -206,8 +213,9 @@ int prepare_h2(fa_model* m) {
   }
   if (v2) mats.push_back(&m->wple_model);
   int64_t norm_rows = 0;
+  bool ok = gemm_h2_enabled();
   for (Mat* w : mats) {
-    if (w->terms != 1 || w->cols % 32 != 0) return FA_OK;
+    ok = ok && w->terms == 1 && w->cols % 32 == 0;
     norm_rows += w->rows;
   }
   // largest |w| of each matrix (and of the embedding table), row norms
@@ -247,7 +255,7 @@ int prepare_h2(fa_model* m) {
     const int e = 14 - std::ilogb(b * 1.0001);
     return e < -100 || e > 100 ? 0.f : std::ldexp(1.f, e);
   };
-  bool ok = !rc;
+  ok = ok && !rc;
   for (size_t i = 0; i < nm && ok; i++) {
     const float mx = value(i);
     mats[i]->h_scale = mx == 0.f ? 1.f : pow2_for(mx);
@@ -267,9 +275,9 @@ int prepare_h2(fa_model* m) {
       rc = set_error(ctx, FA_ERR_HIP, "gemma: reading the weights' range failed");
     for (uint32_t b : bad) ok = ok && b == 0;
   }
-  // operand bounds
+  // operand bounds (three-plane matrices: of the hi plane, 1 % below theirs at most)
   const double rd = std::sqrt((double)d);
-  auto gain = [&](const float* dev, int n) -> double {  // max |gain|; not finite: unusable
+  auto gain = [&](const float* dev, int n, double most) -> double {  // max |gain|; infinite: unusable
     std::vector<float> v(n);
     if (hipMemcpy(v.data(), dev, (size_t)n * 4, hipMemcpyDeviceToHost) != hipSuccess) return INFINITY;
     double mx = 0, ss = 0;
@@ -278,9 +286,9 @@ int prepare_h2(fa_model* m) {
       mx = std::max(mx, std::fabs((double)x));
       ss += (double)x * x;
     }
-    return mx > 64 * std::sqrt(ss / n) ? INFINITY : mx;
+    return mx > most * std::sqrt(ss / n) ? INFINITY : mx;
   };
-  if (ok && !rc) {
+  if (!rc) {
     int64_t at = 0;
     auto row_max = [&](int64_t r0, int64_t r1, int64_t group, int64_t which) {  // largest norm of the rows
       double mx = 0;
@@ -288,33 +296,41 @@ int prepare_h2(fa_model* m) {
         if (group == 0 || (r / group) % 2 == which) {
           float f;
           std::memcpy(&f, &host[head + at + r], 4);
+          if (!std::isfinite(f)) return (double)INFINITY;
           mx = std::max(mx, (double)f);
         }
-      return mx;
+      return 1.01 * mx;
     };
     double xb = value(nm) * 1.01 * rd;  // the residual stream's largest value (variant 2's products read it)
     m->s_x0 = pow2_for(xb);
-    const double gple = v2 ? gain(m->g_ple_norm, P) * std::sqrt((double)P) : 0;
+    const double gple = v2 ? gain(m->g_ple_norm, P, 64) * std::sqrt((double)P) : 0;
+    bool tiles = true;
     for (auto& L : m->layers) {
-      const double nin = rd * gain(L.g_in, d), nffn = rd * gain(L.g_pre_ffn, d);
+      const double nin = rd * gain(L.g_in, d, 64), nffn = rd * gain(L.g_pre_ffn, d, 64);
       L.s_in = pow2_for(nin);
       L.s_att = pow2_for(v2 ? std::sqrt((double)L.D) : nin * row_max((int64_t)(H + L.Hkv) * L.D, L.width, 0, 0));
+      if (L.D == 256) {
+        L.s_q = pow2_for(16 * gain(L.g_q, 256, 1024));  // a rotated row keeps its norm
+        L.s_k = pow2_for(16 * gain(L.g_k, 256, 1024));
+        tiles = tiles && L.s_q != 0 && L.s_k != 0 && L.s_att != 0;
+      }
       at += L.wqkv.rows + L.wo.rows;
       L.s_ffn = pow2_for(nffn);
       L.s_gu = pow2_for(nffn * row_max(0, 2LL * F, 32, 0) * nffn * row_max(0, 2LL * F, 32, 1));
       at += L.wgu.rows + L.wdown.rows;
       ok = ok && L.s_in != 0 && L.s_att != 0 && L.s_ffn != 0 && L.s_gu != 0;
       if (v2) {
-        xb += rd * (gain(L.g_post_attn, d) + gain(L.g_post_ffn, d));
+        xb += rd * (gain(L.g_post_attn, d, 64) + gain(L.g_post_ffn, d, 64));
         L.s_x = pow2_for(xb);
         L.s_ple = pow2_for(row_max(0, P, 0, 0) * xb * rd * gple);
         at += L.wple_gate.rows + L.wple_proj.rows;
-        xb = (xb + rd * gain(L.g_ple_post, d)) * std::fabs((double)L.scalar);
+        xb = (xb + rd * gain(L.g_ple_post, d, 64)) * std::fabs((double)L.scalar);
         ok = ok && L.s_x != 0 && L.s_ple != 0;
       }
     }
     if (v2) ok = ok && m->s_x0 != 0;
     m->h2 = ok;
+    m->tiles = tiles;
   }
   tmp.release();
   return rc;
@@ -1039,6 +1055,7 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
   pin.forced_rows = fa::attention_rows_forced();
   pin.forced_xcd = fa::attention_xcd_forced();
   pin.tile_min_rows = fa::tile_min_rows();
+  pin.tiles_allowed = m->tiles;
   fa::AttnPlan ap;
   fa::plan_attention(pin, ap);
   const int64_t n_items_t = ap.n_items_t, n_items = ap.n_items_t + ap.n_items_v, n_tiles = ap.n_tiles;
@@ -1118,8 +1135,8 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
   for (int o : m->dense_out) maxw = std::max(maxw, o);
   const int kparts_max = std::max(kparts_t, kparts_v);
   const int64_t part_floats = kparts_max > 1 ? fa::attention_part_floats(kparts_max, M, H, m->max_hd / H) : 0;
-  // key/value tile images: [tile][Hkv][key | value][3 * 32 * 256] bf16
-  const size_t img_bytes = (size_t)n_tiles * hkv_t * 2 * (3 * 32 * 256) * 2;
+  // key/value tile images: [tile][Hkv][key | value][2 * 32 * 256] fp16
+  const size_t img_bytes = (size_t)n_tiles * hkv_t * 2 * (2 * 32 * 256) * 2;
   const size_t f32_bytes = ((size_t)M * ncols + (size_t)B * (d + 2 * (size_t)maxw) + (size_t)part_floats) * 4 + 256;
   const size_t img_off = (f32_bytes + 255) & ~(size_t)255;
   const size_t ws_bytes = img_off + img_bytes + 4096;
@@ -1248,16 +1265,16 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
       if ((rc = product(g, g.a, L.wqkv, L.s_in, 0.f, FA_K_GEMM_QKV, 2.0 * rows * L.width * d, st))) return rc;
     }
     if (tiles) {
-      // read k and v (4 bytes per element); write their images (6 bytes per
+      // read k and v (4 bytes per element); write their images (4 bytes per
       // element each, tiles padded to 32 tokens); q is normed and rotated
       // by the attention as it loads it
       const int64_t ntl = cut_h[b1] - cut_h[b0];
       // (variant 2 norms the values too: each value half-block also reads
       // the other half of its keys' values for the sum of squares)
       fa::Probe pr(m, FA_K_QKNORM_ROPE, 0,
-                   (double)rows * (v2 ? 3 : 2) * Hkv * 4.0 * D + (double)ntl * Hkv * 2 * 3 * 32 * 256 * 2);
+                   (double)rows * (v2 ? 3 : 2) * Hkv * 4.0 * D + (double)ntl * Hkv * 2 * 2 * 32 * 256 * 2);
       if ((rc = fa::launch_kv_tiles(ctx, qkvr, r0, H, Hkv, L.g_k, eps, L.cos_t, L.sin_t, text_d, cut_h[b0],
-                                    (int32_t)ntl, img, st, v2)))
+                                    (int32_t)ntl, img, st, v2, L.s_k, L.s_att)))
         return rc;
       pr.done();
     } else {
@@ -1299,6 +1316,7 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
         at.H = H; at.Hkv = Hkv; at.window = a.window; at.scale = a.scale;
         at.gq = L.g_q; at.eps = eps; at.cos_t = L.cos_t; at.sin_t = L.sin_t; at.waves = waves_t;
         at.split = a.split;
+        at.q_scale = L.s_q; at.k_scale = L.s_k; at.v_scale = L.s_att;
         if (kparts_t > 1) {
           at.kparts = kparts_t; at.rows = M; at.nrows = rows; at.part = attn_part;
         }

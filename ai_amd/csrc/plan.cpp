@@ -41,7 +41,7 @@ void plan_attention(const AttnPlanIn& in, AttnPlan& p) {
   // fp32 kernel.
   double pairs = 0;
   for (int b = 0; b < in.B; b++) pairs += (double)in.lengths[b] * in.lengths[b];
-  p.tiles_ok = (p.M > in.tile_min_rows || pairs >= (double)in.tile_min_pairs) && p.M >= 32LL * in.B;
+  p.tiles_ok = in.tiles_allowed && (p.M > in.tile_min_rows || pairs >= (double)in.tile_min_pairs) && p.M >= 32LL * in.B;
   for (int l = 0; l < in.n_layers; l++) {
     if (in.layer_D[l] != 256) continue;
     if (p.hkv_t && in.layer_Hkv[l] != p.hkv_t) p.mixed_hkv = true;

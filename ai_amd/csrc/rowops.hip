@@ -298,9 +298,9 @@ __global__ __launch_bounds__(1024) void pool_kernel(const float* __restrict__ h,
 // Key and value images of head_dim-256 layers for attention_tiles_kernel,
 // one block per (tile of 32 tokens of one sequence, kv head): tile tt of
 // sequence b (cut[b] <= tt < cut[b+1]) holds tokens 32 (tt - cut[b]) .. +31.
-// Image pair [tt][kv head][key image | value image], 3 * 32 * 256 bf16 each:
-//   key image [term][key][256]: the normed, gained and rotated key's exact
-//   split terms, the 16-byte chunk c (dims 8c .. 8c+7) of key k at
+// Image pair [tt][kv head][key image | value image], 2 * 32 * 256 fp16 each:
+//   key image [term][key][256]: the normed, gained and rotated key times
+//   k_scale as two fp16 terms (hi, and lo = fp16(x - hi)), the 16-byte chunk c (dims 8c .. 8c+7) of key k at
 //   position c ^ k (the 16 keys of one operand read hit distinct banks);
 //   value image [term][dim][32 slots]: slot 8g + 4h + r holds key 16h + 4g +
 //   r (the order in which the attention's probabilities meet the values),
@@ -319,9 +319,12 @@ struct KvTilesParams {
   int t_lo, tiles;
   uint16_t* img;
   int norm_v;  // values RMS-normed with unit gain first (EmbeddingGemma 2, gemma2.go)
+  float k_scale, v_scale;  // the keys' and values' powers of two
 };
 
-constexpr int kTileImg = 3 * 32 * 256;  // bf16 per key or value image
+constexpr int kTileImg = 2 * 32 * 256;  // fp16 per key or value image
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 // floats per LDS row of the value transpose (128 dims): the column reads of
 // one wave (16 consecutive dims x keys 4c + const, c = 0..3) land on banks
 // 16c + dim mod 64, all distinct, since 4 * 132 = 16 (mod 64)
@@ -363,7 +366,7 @@ __device__ __forceinline__ void key_tile(const KvTilesParams& a, int tile, int h
   for (int j = 0; j < KPW; j++) {
     const int k = kb + wave + 4 * j;
     f32x4 x[1] = {v[j]};
-    const float inv = rms_inv(sumsq<1>(x), D, a.eps);
+    const float inv = rms_inv(sumsq<1>(x), D, a.eps) * a.k_scale;
     x[0].x = x[0].x * inv * gg.x; x[0].y = x[0].y * inv * gg.y;
     x[0].z = x[0].z * inv * gg.z; x[0].w = x[0].w * inv * gg.w;
     f32x4 o;
@@ -378,19 +381,26 @@ __device__ __forceinline__ void key_tile(const KvTilesParams& a, int tile, int h
       r.z = o.z * sv[j].z + x[0].z * c[j].z; r.w = o.w * sv[j].w + x[0].w * c[j].w;
     }
     if (k >= n) r = f32x4{0.f, 0.f, 0.f, 0.f};
-    uint32_t th[4], tm[4], tl[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const Split3 sp = split3(r[e]);
-      th[e] = sp.h;
-      tm[e] = sp.m;
-      tl[e] = sp.l;
-    }
+    const f16x4 th = __builtin_convertvector(r, f16x4);
+    const f16x4 tl = __builtin_convertvector(r - __builtin_convertvector(th, f32x4), f16x4);
     uint16_t* o16 = kimg + k * D + (((lane >> 1) ^ k) * 8) + (lane & 1) * 4;
-    *reinterpret_cast<uint2*>(o16) = make_uint2(pack_hi16(th[0], th[1]), pack_hi16(th[2], th[3]));
-    *reinterpret_cast<uint2*>(o16 + 32 * D) = make_uint2(pack_hi16(tm[0], tm[1]), pack_hi16(tm[2], tm[3]));
-    *reinterpret_cast<uint2*>(o16 + 64 * D) = make_uint2(pack_hi16(tl[0], tl[1]), pack_hi16(tl[2], tl[3]));
+    *reinterpret_cast<f16x4*>(o16) = th;
+    *reinterpret_cast<f16x4*>(o16 + 32 * D) = tl;
   }
+}
+
+// One chunk of the value image: the eight slots of dim dl and chunk c, from
+// the LDS rows Vt, times v_scale, hi terms at o and lo terms one term on.
+__device__ __forceinline__ void value_chunk(const float (*Vt)[kVtStride], int dl, int c, float v_scale, uint16_t* o) {
+  f16x8 th, tl;
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const float x = Vt[(e >> 2) * 16 + 4 * c + (e & 3)][dl] * v_scale;
+    th[e] = (_Float16)x;
+    tl[e] = (_Float16)(x - (float)th[e]);
+  }
+  *reinterpret_cast<f16x8*>(o) = th;
+  *reinterpret_cast<f16x8*>(o + 32 * 256) = tl;
 }
 
 // Dims 128*half .. 128*half + 127 of the value image of (tile, hk): rows
@@ -441,21 +451,7 @@ __device__ __forceinline__ void value_tile(const KvTilesParams& a, int tile, int
     const int u = tid + 256 * i;
     const int dl = u >> 2, c = u & 3;  // local dim, chunk of 8 slots: keys 4c .. 4c+3, 16 + 4c .. 16 + 4c+3
     const int d = 128 * half_ + dl;
-    uint32_t th[8], tm[8], tl[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const Split3 sp = split3(Vt[(e >> 2) * 16 + 4 * c + (e & 3)][dl]);
-      th[e] = sp.h;
-      tm[e] = sp.m;
-      tl[e] = sp.l;
-    }
-    uint16_t* o = vimg + d * 32 + ((c ^ ((d >> 1) & 3)) * 8);
-    *reinterpret_cast<uint4*>(o) = make_uint4(pack_hi16(th[0], th[1]), pack_hi16(th[2], th[3]),
-                                              pack_hi16(th[4], th[5]), pack_hi16(th[6], th[7]));
-    *reinterpret_cast<uint4*>(o + 32 * D) = make_uint4(pack_hi16(tm[0], tm[1]), pack_hi16(tm[2], tm[3]),
-                                                       pack_hi16(tm[4], tm[5]), pack_hi16(tm[6], tm[7]));
-    *reinterpret_cast<uint4*>(o + 64 * D) = make_uint4(pack_hi16(tl[0], tl[1]), pack_hi16(tl[2], tl[3]),
-                                                       pack_hi16(tl[4], tl[5]), pack_hi16(tl[6], tl[7]));
+    value_chunk(Vt, dl, c, a.v_scale, vimg + d * 32 + ((c ^ ((d >> 1) & 3)) * 8));
   }
 }
 
@@ -487,21 +483,7 @@ __device__ __forceinline__ void value_quarter(const KvTilesParams& a, int tile, 
   const int u = wave * 64 + lane;
   const int dl = u >> 2, c = u & 3;  // local dim, chunk of 8 slots: keys 4c .. 4c+3, 16 + 4c .. 16 + 4c+3
   const int d = 64 * q + dl;
-  uint32_t th[8], tm[8], tl[8];
-#pragma unroll
-  for (int e = 0; e < 8; e++) {
-    const Split3 sp = split3(Vt[(e >> 2) * 16 + 4 * c + (e & 3)][dl]);
-    th[e] = sp.h;
-    tm[e] = sp.m;
-    tl[e] = sp.l;
-  }
-  uint16_t* o = vimg + d * 32 + ((c ^ ((d >> 1) & 3)) * 8);
-  *reinterpret_cast<uint4*>(o) = make_uint4(pack_hi16(th[0], th[1]), pack_hi16(th[2], th[3]),
-                                            pack_hi16(th[4], th[5]), pack_hi16(th[6], th[7]));
-  *reinterpret_cast<uint4*>(o + 32 * D) = make_uint4(pack_hi16(tm[0], tm[1]), pack_hi16(tm[2], tm[3]),
-                                                     pack_hi16(tm[4], tm[5]), pack_hi16(tm[6], tm[7]));
-  *reinterpret_cast<uint4*>(o + 64 * D) = make_uint4(pack_hi16(tl[0], tl[1]), pack_hi16(tl[2], tl[3]),
-                                                     pack_hi16(tl[4], tl[5]), pack_hi16(tl[6], tl[7]));
+  value_chunk(Vt, dl, c, a.v_scale, vimg + d * 32 + ((c ^ ((d >> 1) & 3)) * 8));
 }
 
 // QUARTERS (values not normed): blocks 8i + j of (tile t_lo + i / Hkv, kv
@@ -731,13 +713,14 @@ int launch_l2norm(fa_ctx* ctx, const float* y, int32_t nseq, int32_t width, int3
 
 int launch_kv_tiles(fa_ctx* ctx, const float* qkv, int64_t row0, int32_t H, int32_t Hkv, const float* gk, float eps,
                     const float* cos_t, const float* sin_t, const int32_t* d_tile_ext, int32_t t_lo, int32_t tiles,
-                    uint16_t* img, hipStream_t s, bool norm_v) {
+                    uint16_t* img, hipStream_t s, bool norm_v, float k_scale, float v_scale) {
   if (tiles == 0) return FA_OK;
   if (!d_tile_ext) return set_error(ctx, FA_ERR_ARG, "key/value tiles: no tile extents");
   KvTilesParams a;
   a.qkv = qkv; a.row0 = row0; a.H = H; a.Hkv = Hkv; a.gk = gk; a.eps = eps; a.cs = cos_t; a.sn = sin_t;
   a.tile_ext = d_tile_ext; a.t_lo = t_lo; a.tiles = tiles; a.img = img;
   a.norm_v = norm_v ? 1 : 0;
+  a.k_scale = k_scale; a.v_scale = v_scale;
   if (norm_v)
     hipLaunchKernelGGL(kv_tiles_kernel<false>, dim3((unsigned)(4 * (int64_t)tiles * Hkv)), dim3(256), 0, s, a);
   else
