@@ -257,6 +257,14 @@ bool score_fused_ok(const float* q, int64_t ldq, const float* docs, int64_t ldd,
 int launch_score_topk(fa_ctx* ctx, const float* q, int64_t nq, int64_t ldq, const float* docs, int64_t nd,
                       int64_t ldd, int d, int topk, int32_t* idx, float* val, void* scratch, int nwg,
                       hipStream_t s);
+// Few queries (up to kScoreFewMax): one streaming pass over the documents
+// on the fp32 MFMA with the selection fused (score_few.hip).
+// Scratch: score_few_scratch bytes.
+constexpr int64_t kScoreFewMax = 32;
+bool score_few_ok(const float* q, int64_t nq, const float* docs, int64_t nd, int d, int topk);
+size_t score_few_scratch(int64_t nq, int64_t nd, int topk);
+int launch_score_few(fa_ctx* ctx, const float* q, int64_t nq, const float* docs, int64_t nd, int d, int topk,
+                     int32_t* idx, float* val, void* scratch, hipStream_t s);
 int launch_topk(fa_ctx* ctx, const float* scores, int64_t nq, int64_t nd, int32_t topk, int32_t* idx, float* val,
                 void* scratch, hipStream_t s);
 

@@ -231,9 +231,10 @@ int fa_attention_dev(fa_ctx* ctx, const float* q, const float* k, const float* v
  * selects one); slots past a row's non-NaN scores get index -1 and value NaN.
  * From 128 queries with d % 32 == 0, topk <= 16 and 16-byte aligned rows the
  * scores are the exact dot products rounded to float32 and no score matrix is
- * formed (blocks of 256 queries); otherwise an fp32-MFMA product (fp32
- * accumulation, within a few units of the last place of the exact score) is
- * followed by a two-pass top-k. A query's scores, and its order among
+ * formed (blocks of 256 queries); otherwise the scores are fp32-MFMA sums
+ * (within a few units of the last place of the exact score), up to 32
+ * queries with d % 16 == 0 and 16-byte aligned rows in one pass over the docs
+ * that selects as it goes, else by a product and a two-pass top-k. A query's scores, and its order among
  * candidates whose scores agree to that precision, can therefore differ
  * between a call with fewer than 128 queries (or topk > 16) and one with
  * more; fa_similarities_topk_dev_noalloc takes the exact path for any nq. */

@@ -134,3 +134,38 @@ def test_fused_and_per_query_paths_agree(ctx):
         srt = -np.sort(-s64[i])[:11]
         if np.diff(-srt).min() > 2e-6:
             assert fi[i].tolist() == oi[0].tolist(), i
+
+
+@pytest.mark.parametrize("nq", [1, 16, 17, 32])
+@pytest.mark.parametrize("nd,d,k", [(1, 16, 1), (15, 48, 7), (33, 16, 32), (127, 64, 10), (129, 768, 10), (1025, 32, 32),
+                                    (17000, 16, 10), (140000, 16, 3)])
+def test_few_queries_streaming(nq, nd, d, k):
+    """The streaming kernel for up to 32 queries at the edges of its blocks (16
+    documents per wave, 16..128 per workgroup) against a stable sort. Entries
+    are small integers, so every score is exact and ties are frequent; one
+    document scores NaN."""
+    r = np.random.default_rng(nd * 33 + nq)
+    q = r.integers(-2, 3, (nq, d)).astype(np.float32)
+    docs = r.integers(-2, 3, (nd, d)).astype(np.float32)
+    if nd > 20:
+        docs[7] = np.nan
+    s = q.astype(np.float64) @ docs.astype(np.float64).T
+    order = np.argsort(np.where(np.isnan(s), np.inf, -s), axis=1, kind="stable")[:, :k]
+    want = np.take_along_axis(s, order, 1)
+    with N.Context(0) as ctx:
+        idx, val = np.empty((nq, k), np.int32), np.empty((nq, k), np.float32)
+        N.check(ctx.h, N.lib().fa_similarities_topk(ctx.h, N.ptr(q), nq, N.ptr(docs), nd, d, k, N.ptr(idx),
+                                                    N.ptr(val)))
+    gone = np.isnan(want)
+    assert np.array_equal(idx, np.where(gone, -1, order))
+    assert np.array_equal(val[~gone], want[~gone].astype(np.float32)) and np.isnan(val[gone]).all()
+
+
+@pytest.mark.parametrize("nd", [200, 20000])
+def test_few_queries_all_equal(nd):
+    """Every score equal: more candidates at the bound than the merge keeps."""
+    q, docs = np.ones((3, 32), np.float32), np.ones((nd, 32), np.float32)
+    idx, val = np.empty((3, 10), np.int32), np.empty((3, 10), np.float32)
+    with N.Context(0) as ctx:
+        N.check(ctx.h, N.lib().fa_similarities_topk(ctx.h, N.ptr(q), 3, N.ptr(docs), nd, 32, 10, N.ptr(idx), N.ptr(val)))
+    assert np.array_equal(idx, np.tile(np.arange(10), (3, 1))) and (val == 32).all()
