@@ -9,14 +9,14 @@
 // all of them are drawn up front) and reads the per-iteration change count
 // and centre sizes for the early stop and the empty-centre restarts.
 //   k-means++ (cluster.go:51-85): per new centre, kpp_weights_kernel scores
-//     every row against the newest centre, keeps the best similarity and
-//     writes the float64 weight (1 - best)^2; block_sums_kernel sums the
-//     weights in blocks of 256; kpp_pick_kernel (one workgroup) scans the
+//     every row against the newest centre, keeps the best similarity,
+//     writes the float64 weight (1 - best)^2 and sums the weights in blocks
+//     of 256; kpp_pick_kernel (one workgroup) scans the
 //     block sums, scales the uniform draw by the total, finds the block and
 //     then the row where the running subtraction crosses zero, and copies
 //     that row into the centre list.
-//   Lloyd rounds (cluster.go:86-129): sim product, argmax_rows_kernel
-//     (assignment, similarity), count_kernel (per-chunk centre counts and
+//   Lloyd rounds (cluster.go:86-129): nearest_kernel, or the sim product and
+//     argmax_rows_kernel (assignment, similarity), count_kernel (per-chunk centre counts and
 //     change counts), a stable counting sort of the row indices by centre
 //     (chunk_scan_kernel, offsets_kernel, scatter_kernel), then
 //     colsum_kernel adds each centre's rows in increasing row order, one
@@ -38,9 +38,8 @@ namespace {
 constexpr int kRowWG = 256;        // one wave per row, 4 rows per workgroup
 constexpr int kChunk = 256;        // rows per counting-sort chunk (one per thread of count_kernel)
 constexpr int kCntWindow = 8192;   // centres per LDS counter window
-constexpr int kPickThreads = 1024;
 constexpr int kSumBlock = 256;     // weights per partial sum of the k-means++ pick
-constexpr int kColTile = 32;       // rows loaded ahead by colsum_kernel
+constexpr int kColTile = 64;       // rows per load group of colsum_kernel (one per lane)
 
 inline unsigned row_blocks(int64_t n) { return (unsigned)((n + 3) / 4); }
 
@@ -51,14 +50,28 @@ __global__ __launch_bounds__(kRowWG) void normalize_rows_kernel(const float* x, 
   const int lane = threadIdx.x & 63;
   if (row >= n) return;
   const float* xr = x + row * d;
+  float* orow = out + row * d;
   float ss = 0.f;
+  constexpr int kHeld = 16;  // up to 1 024 columns: the row's loads all in flight (40 x 768: 8.0 -> 3.2 us)
+  if (d <= 64 * kHeld) {
+    float v[kHeld];
+#pragma unroll
+    for (int i = 0; i < kHeld; i++) v[i] = lane + 64 * i < d ? xr[lane + 64 * i] : 0.f;
+#pragma unroll
+    for (int i = 0; i < kHeld; i++) ss += v[i] * v[i];
+    float nrm = sqrtf(wave_sum(ss));
+    if (nrm == 0.f) nrm = 1.f;
+#pragma unroll
+    for (int i = 0; i < kHeld; i++)
+      if (lane + 64 * i < d) orow[lane + 64 * i] = v[i] / nrm;
+    return;
+  }
   for (int j = lane; j < d; j += 64) {
     const float v = xr[j];
     ss += v * v;
   }
   float nrm = sqrtf(wave_sum(ss));
   if (nrm == 0.f) nrm = 1.f;
-  float* orow = out + row * d;
   for (int j = lane; j < d; j += 64) orow[j] = xr[j] / nrm;
 }
 
@@ -96,6 +109,129 @@ __global__ __launch_bounds__(kRowWG) void argmax_rows_kernel(const float* __rest
   simil[row] = sr[bi];
 }
 
+// Product and first-max argmax in one pass for up to 64 centres (d % 8 == 0,
+// 16-byte aligned rows): bound by reading x once (154 MB at 50 000 x 768,
+// 31 us at a large copy's rate; the fp32 MFMAs take as long). A wave takes 32
+// rows, their values loaded from global memory straight into the operand
+// registers of v_mfma_f32_32x32x2_f32 (two groups of eight 16-byte loads in
+// flight per lane); the centres pass through LDS 128 columns at a time,
+// shared by the workgroup's four waves. Operands and order of the additions are
+// gemm_kernel's, so the similarities are the same bits as the product's (a
+// row between two centres falls to the same one). Lane l holds centre 32 b +
+// l%32 (block b) against rows 8 (r/4) + 4 (l/32) + r%4: a row's argmax is a
+// maximum over blocks and five exchanges, then the lowest index that has it.
+// 67 us at 50 000 x 768 and 40 centres against 61 + 12 for the product and the
+// argmax of its stored rows: the MFMA pipes set it (391 workgroups of four
+// waves leave some SIMDs two waves of 32 rows, 47 us of fp32 MFMAs).
+constexpr int kNearCols = 128, kNearSteps = 8, kNearMax = 64;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// max / min over lanes l ^ 1, 2, 4, 8, 16: the 32 lanes of a half wave
+template <class F>
+__device__ __forceinline__ uint32_t half_wave(uint32_t v, F f) {
+  auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = f((uint32_t)a[0], (uint32_t)a[1]);
+  v = f(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, false));
+  v = f(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xF, 0xF, false));
+  v = f(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xF, 0xF, false));
+  v = f(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xF, 0xF, false));
+  return v;
+}
+
+template <int CB>
+__global__ __launch_bounds__(256) void nearest_kernel(const float* __restrict__ x, int64_t n, int d,
+                                                      const float* __restrict__ centres, int k,
+                                                      int32_t* __restrict__ assign, float* __restrict__ simil) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  constexpr int LD = kNearCols + 4;  // rows four banks apart
+  __shared__ __attribute__((aligned(16))) float cs[32 * CB * LD];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lq = lane & 31, h = lane >> 5;
+  const int64_t row0 = ((int64_t)blockIdx.x * 4 + wave) * 32;
+  const float* xr = x + min(row0 + lq, n - 1) * d + 4 * h;
+  const int steps = d / 8;
+  f32x16 acc[CB];
+#pragma unroll
+  for (int b = 0; b < CB; b++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[b][r] = 0.f;
+  auto load = [&](f4 (&a)[kNearSteps], int s0) {
+#pragma unroll
+    for (int u = 0; u < kNearSteps; u++) a[u] = *reinterpret_cast<const f4*>(xr + 8 * min(s0 + u, steps - 1));
+  };
+  auto compute = [&](const f4 (&a)[kNearSteps], int s0, int c0) {
+#pragma unroll
+    for (int u = 0; u < kNearSteps; u++) {
+      if (s0 + u < steps) {
+        f4 c[CB];
+#pragma unroll
+        for (int b = 0; b < CB; b++)
+          c[b] = *reinterpret_cast<const f4*>(cs + (32 * b + lq) * LD + 8 * (s0 + u) - c0 + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+          for (int b = 0; b < CB; b++)
+            acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][e], c[b][e], acc[b], 0, 0, 0);
+      }
+    }
+  };
+  // the next columns of the centres load into registers while the current
+  // ones are used (centres past k repeat the last, columns past d its last)
+  constexpr int NC = 32 * CB * (kNearCols / 4) / 256;
+  f4 pre[NC];
+  auto fetch = [&](int c0) {
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+      const int at = threadIdx.x + 256 * i, r = at / (kNearCols / 4), c = at % (kNearCols / 4);
+      pre[i] = *reinterpret_cast<const f4*>(centres + (int64_t)min(r, k - 1) * d + min(c0 + 4 * c, d - 4));
+    }
+  };
+  f4 a0[kNearSteps], a1[kNearSteps];
+  fetch(0);
+  load(a0, 0);
+  for (int c0 = 0; c0 < d; c0 += kNearCols) {
+    __syncthreads();  // the previous columns were read
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+      const int at = threadIdx.x + 256 * i;
+      *reinterpret_cast<f4*>(cs + at / (kNearCols / 4) * LD + at % (kNearCols / 4) * 4) = pre[i];
+    }
+    __syncthreads();
+    const int s0 = c0 / 8;
+    fetch(c0 + kNearCols);
+    load(a1, s0 + kNearSteps);
+    compute(a0, s0, c0);
+    load(a0, s0 + 2 * kNearSteps);
+    if (s0 + kNearSteps < steps) compute(a1, s0 + kNearSteps, c0);
+  }
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    // floats as ordered integers; 0 for NaN and for centres past k
+    uint32_t key = 0, idx = 0xFFFFFFFFu;
+#pragma unroll
+    for (int b = 0; b < CB; b++) {
+      const float v = acc[b][r];
+      const uint32_t u = __float_as_uint(v + 0.f);
+      const uint32_t o = v != v || 32 * b + lq >= k ? 0u : (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+      if (o > key) {
+        key = o;
+        idx = 32 * b + lq;
+      }
+    }
+    const uint32_t top = half_wave(key, [](uint32_t p, uint32_t q) { return max(p, q); });
+    const uint32_t at = half_wave(key == top ? idx : 0xFFFFFFFFu, [](uint32_t p, uint32_t q) { return min(p, q); });
+    const float first = __shfl(acc[0][r], 32 * h, 64);  // centre 0
+    const int64_t row = row0 + (r >> 2) * 8 + 4 * h + (r & 3);
+    // no number above -inf, or NaN at index 0 where the sequential scan
+    // starts: index 0
+    const bool zero = at == 0xFFFFFFFFu || top == 0x007FFFFFu || isnan(first);
+    if (row < n && lq == (zero ? 0 : (int)(at & 31))) {
+      assign[row] = zero ? 0 : (int)at;
+      simil[row] = zero ? first : (CB == 2 && at >= 32 ? acc[CB - 1][r] : acc[0][r]);
+    }
+  }
+}
+
 // Per chunk of kChunk rows: rows per centre (chunk_cnt[c][ch], centre-major)
 // and rows whose centre differs from the previous round's
 // (chunk_changed[ch]); then the previous assignment is brought up to date.
@@ -125,42 +261,60 @@ __global__ __launch_bounds__(kChunk) void count_kernel(const int32_t* __restrict
 }
 
 // k-means++ step over all rows: s = x[i] . c, best[i] = max(best[i], s),
-// w[i] = float64(1 - best[i])^2 (cluster.go:62-72).
-__global__ __launch_bounds__(kRowWG) void kpp_weights_kernel(const float* __restrict__ x, int64_t n, int d,
-                                                             const float* __restrict__ c, float* best, double* w) {
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= n) return;
-  const float* xr = x + row * d;
-  float s = 0.f;
-  if ((d & 3) == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(c)) & 15) == 0) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    const f4* xv = reinterpret_cast<const f4*>(xr);
-    const f4* cv = reinterpret_cast<const f4*>(c);
-    for (int j = lane; j < d / 4; j += 64) {
-      const f4 a = xv[j], b = cv[j];
-      s += a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
-    }
-  } else {
-    for (int j = lane; j < d; j += 64) s += xr[j] * c[j];
-  }
-  s = wave_sum(s);
-  if (lane != 0) return;
-  float b = best[row];
-  if (s > b) b = s;
-  best[row] = b;
-  const double om = (double)(1.f - b);
-  w[row] = om * om;
-}
-
-// part[b] = sum of w[b*kSumBlock ...] in a fixed tree order.
-__global__ __launch_bounds__(kSumBlock) void block_sums_kernel(const double* __restrict__ w, int64_t n,
-                                                               double* __restrict__ part) {
+// w[i] = float64(1 - best[i])^2 (cluster.go:62-72), and part[b] = the sum of
+// w[b * kSumBlock ...] in a fixed tree order. One workgroup of 16 waves per
+// kSumBlock rows, each wave four rows at a time (bound by reading x: 25 us at
+// 50 000 x 768; the block sums were a launch of their own, 4.7 us and a gap
+// per centre).
+constexpr int kKppWaves = 16;
+__global__ __launch_bounds__(64 * kKppWaves) void kpp_weights_kernel(const float* __restrict__ x, int64_t n, int d,
+                                                                     const float* __restrict__ c, float* best,
+                                                                     double* w, double* __restrict__ part) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
   __shared__ double buf[kSumBlock];
-  const int t = threadIdx.x;
-  const int64_t i = (int64_t)blockIdx.x * kSumBlock + t;
-  buf[t] = i < n ? w[i] : 0.0;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t r0 = (int64_t)blockIdx.x * kSumBlock;
+  const bool vec = (d & 3) == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(c)) & 15) == 0;
+  constexpr int U = 4;
+  for (int i = wave * U; i < kSumBlock; i += kKppWaves * U) {
+    float s[U] = {0.f, 0.f, 0.f, 0.f};
+    const float* xr[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) xr[u] = x + min(r0 + i + u, n - 1) * d;
+    if (vec) {
+      for (int j = lane; j < d / 4; j += 64) {
+        const f4 b = reinterpret_cast<const f4*>(c)[j];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const f4 a = reinterpret_cast<const f4*>(xr[u])[j];
+          s[u] += a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
+        }
+      }
+    } else {
+      for (int j = lane; j < d; j += 64) {
+#pragma unroll
+        for (int u = 0; u < U; u++) s[u] += xr[u][j] * c[j];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) s[u] = wave_sum(s[u]);
+    if (lane < U) {
+      const int64_t row = r0 + i + lane;
+      const float v = lane == 0 ? s[0] : lane == 1 ? s[1] : lane == 2 ? s[2] : s[3];
+      double om = 0.0;
+      if (row < n) {
+        float b = best[row];
+        if (v > b) b = v;
+        best[row] = b;
+        om = (double)(1.f - b);
+        om = om * om;
+        w[row] = om;
+      }
+      buf[i + lane] = om;
+    }
+  }
   __syncthreads();
+  const int t = threadIdx.x;
   for (int o = kSumBlock / 2; o > 0; o >>= 1) {
     if (t < o) buf[t] += buf[t + o];
     __syncthreads();
@@ -173,6 +327,9 @@ __global__ __launch_bounds__(kSumBlock) void block_sums_kernel(const double* __r
 // it positive). The block partial sums' inclusive prefix locates the
 // crossing block, whose weights are then walked one by one. The row is
 // copied to centre_out.
+// kPickThreads: 256 for up to 65 536 rows (one tile of partial sums, four
+// waves at each barrier), else 1 024.
+template <int kPickThreads>
 __global__ __launch_bounds__(kPickThreads) void kpp_pick_kernel(const double* __restrict__ w, int64_t n,
                                                                 const double* __restrict__ part, int nparts, double u,
                                                                 const float* __restrict__ x, int d,
@@ -240,12 +397,21 @@ __global__ __launch_bounds__(kPickThreads) void kpp_pick_kernel(const double* __
     int64_t idx = n - 1;
     if (fb != INT32_MAX) {
       double p = pick - total_s;
-      int64_t i = b0;
-      for (; i < min(n, b0 + kSumBlock); i++) {
-        p -= wblk[i - b0];
-        if (p <= 0) break;
+      // 16 weights read ahead of their subtractions (past the rows: zeros,
+      // which leave p as it is)
+      int at = kSumBlock;
+      for (int j = 0; j < kSumBlock && at == kSumBlock; j += 16) {
+        double v[16];
+#pragma unroll
+        for (int e = 0; e < 16; e++) v[e] = wblk[j + e];
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+          p -= at == kSumBlock ? v[e] : 0.0;
+          if (p <= 0 && at == kSumBlock) at = j + e;
+        }
       }
-      if (i >= min(n, b0 + kSumBlock))  // rounding: keep walking
+      int64_t i = min(n, b0 + at);
+      if (at == kSumBlock)  // rounding: keep walking
         for (; i < n; i++) {
           p -= w[i];
           if (p <= 0) break;
@@ -287,10 +453,10 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(int32_t* chunk_cnt, int
   if (t == 0) sizes[blockIdx.x] = carry;
 }
 
-// offsets[c] = sizes[0] + ... + sizes[c-1]; *changed = sum of the chunks'
-// change counts. One workgroup.
+// offsets[c] = sizes[0] + ... + sizes[c-1]; summary = the sizes and the sum of
+// the chunks' change counts, what the host reads per round. One workgroup.
 __global__ __launch_bounds__(1024) void offsets_kernel(const int32_t* sizes, int k, int32_t* offsets,
-                                                       const int32_t* chunk_changed, int nchunks, int32_t* changed) {
+                                                       const int32_t* chunk_changed, int nchunks, int32_t* summary) {
   __shared__ int32_t buf[1024];
   __shared__ int32_t carry;
   const int t = threadIdx.x;
@@ -306,7 +472,10 @@ __global__ __launch_bounds__(1024) void offsets_kernel(const int32_t* sizes, int
       buf[t] += add;
       __syncthreads();
     }
-    if (base + t < k) offsets[base + t] = carry + buf[t] - v;
+    if (base + t < k) {
+      offsets[base + t] = carry + buf[t] - v;
+      summary[base + t] = v;
+    }
     __syncthreads();
     if (t == 0) carry += buf[1023];
     __syncthreads();
@@ -319,7 +488,7 @@ __global__ __launch_bounds__(1024) void offsets_kernel(const int32_t* sizes, int
     if (t < o) buf[t] += buf[t + o];
     __syncthreads();
   }
-  if (t == 0) *changed = buf[0];
+  if (t == 0) summary[k] = buf[0];
 }
 
 // Stable scatter of row indices by centre: list[offsets[a] + (rows of a in
@@ -342,14 +511,16 @@ __global__ __launch_bounds__(64) void scatter_kernel(const int32_t* __restrict__
       const int64_t row = r0 + sub + lane;
       int a = row < n ? assign[row] : -1;
       if (a < w0 || a >= w1) a = -1;
-      int rank = 0, later = 0;
-      for (int j = 0; j < 64; j++) {
-        const int aj = __shfl(a, j, 64);
-        if (aj == a) {
-          rank += j < lane;
-          later += j > lane;
-        }
+      // the lanes with the same centre, bit by bit (an absent row is a
+      // value of its own)
+      const uint32_t key = a < 0 ? (uint32_t)(w1 - w0) : (uint32_t)(a - w0);
+      uint64_t same = ~0ull;
+      for (int b = 0; (w1 - w0) >> b; b++) {
+        const uint64_t m = __ballot((key >> b) & 1);
+        same &= (key >> b) & 1 ? m : ~m;
       }
+      const uint64_t below = (1ull << lane) - 1;
+      const int rank = __popcll(same & below), later = __popcll(same & ~below) - 1;
       if (a >= 0) list[offsets[a] + chunk_pre[(int64_t)a * nchunks + ch] + cnt[a - w0] + rank] = (int32_t)row;
       __syncthreads();
       if (a >= 0 && later == 0) cnt[a - w0] += rank + 1;
@@ -360,27 +531,52 @@ __global__ __launch_bounds__(64) void scatter_kernel(const int32_t* __restrict__
 
 // sums[c][j] = sum over c's rows in increasing row order of x[row][j],
 // accumulated in float32 from 0 (cluster.go:100-112). One wave per (centre,
-// 64 columns); kColTile rows are loaded ahead of their additions.
+// 64 columns). Latency bound (a lane's additions are one chain, and k * d / 64
+// waves are about two per CU): groups of kColTile rows, the next group's
+// loads in flight while the current one is added, and a group's row indices one
+// per lane (69 -> 50 us at 50 000 x 768 and 40 centres against 32 rows loaded,
+// then added).
 __global__ __launch_bounds__(64) void colsum_kernel(const float* __restrict__ x, int d,
                                                     const int32_t* __restrict__ list,
                                                     const int32_t* __restrict__ offsets,
                                                     const int32_t* __restrict__ sizes, float* __restrict__ sums) {
   const int c = blockIdx.x;
   const int j = blockIdx.y * 64 + threadIdx.x;
-  if (j >= d) return;
   const int32_t* rows = list + offsets[c];
   const int m = sizes[c];
   float acc = 0.f;
-  int p = 0;
-  for (; p + kColTile <= m; p += kColTile) {
-    float v[kColTile];
+  if (m > 0) {
+    const float* xc = x + min(j, d - 1);
+    // lane u holds the group's u-th row (past the last: the last again; its
+    // value is not added)
+    auto index = [&](int p) { return rows[min(p + (int)threadIdx.x, m - 1)]; };
+    auto load = [&](float (&v)[kColTile], int32_t iv) {
 #pragma unroll
-    for (int u = 0; u < kColTile; u++) v[u] = x[(int64_t)rows[p + u] * d + j];
+      for (int u = 0; u < kColTile; u++) v[u] = xc[(int64_t)__builtin_amdgcn_readlane(iv, u) * d];
+    };
+    auto add = [&](const float (&v)[kColTile], int p) {
+      if (p + kColTile <= m) {
 #pragma unroll
-    for (int u = 0; u < kColTile; u++) acc += v[u];
+        for (int u = 0; u < kColTile; u++) acc += v[u];
+      } else {
+#pragma unroll
+        for (int u = 0; u < kColTile; u++)
+          if (p + u < m) acc += v[u];
+      }
+    };
+    float va[kColTile], vb[kColTile];
+    int32_t ia = index(0), ib = index(kColTile);
+    load(va, ia);
+    for (int p = 0; p < m; p += 2 * kColTile) {
+      ia = index(p + 2 * kColTile);
+      load(vb, ib);
+      add(va, p);
+      ib = index(p + 3 * kColTile);
+      load(va, ia);
+      if (p + kColTile < m) add(vb, p + kColTile);
+    }
   }
-  for (; p < m; p++) acc += x[(int64_t)rows[p] * d + j];
-  sums[(int64_t)c * d + j] = acc;
+  if (j < d) sums[(int64_t)c * d + j] = acc;
 }
 
 // Empty-centre restart (cluster.go:113-124): worst = the first index of the
@@ -501,6 +697,26 @@ int launch_sim(fa_ctx* ctx, const float* x, int64_t n, const float* c, int64_t k
   return launch_gemm(ctx, g, ctx->stream);
 }
 
+// assign, simil of every row: fused, or (more than 64 centres, other widths or
+// alignments) the product into sim [n x k] and the argmax of its rows.
+bool nearest_fused_ok(const float* x, const float* c, int64_t k, int d) {
+  return k <= kNearMax && d % 8 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(c)) & 15) == 0;
+}
+int launch_nearest(fa_ctx* ctx, const float* x, int64_t n, const float* c, int64_t k, int d, float* sim,
+                   int32_t* assign, float* simil) {
+  if (nearest_fused_ok(x, c, k, d)) {
+    const dim3 grid((unsigned)((n + 127) / 128)), block(256);
+    if (k <= 32) hipLaunchKernelGGL(nearest_kernel<1>, grid, block, 0, ctx->stream, x, n, d, c, (int)k, assign, simil);
+    else hipLaunchKernelGGL(nearest_kernel<2>, grid, block, 0, ctx->stream, x, n, d, c, (int)k, assign, simil);
+  } else {
+    if (const int rc = launch_sim(ctx, x, n, c, k, d, sim)) return rc;
+    hipLaunchKernelGGL(argmax_rows_kernel, dim3(row_blocks(n)), dim3(kRowWG), 0, ctx->stream, (const float*)sim, n,
+                       (int)k, assign, simil);
+  }
+  FA_CHECK_LAUNCH(ctx);
+  return FA_OK;
+}
+
 }  // namespace
 }  // namespace fa
 
@@ -556,13 +772,8 @@ int fa_cluster_nearest_dev(fa_ctx* ctx, const float* x, int64_t n, const float* 
   }
   FA_HIP_CHECK(ctx, hipSetDevice(ctx->device));
   fa::DevBuf& ws = ctx->slot(S_CL_WORK);
-  if ((rc = ws.ensure(ctx, (size_t)n * k * 4))) return rc;
-  float* sim = ws.as<float>();
-  if ((rc = fa::launch_sim(ctx, x, n, centres, k, d, sim))) return rc;
-  hipLaunchKernelGGL(fa::argmax_rows_kernel, dim3(fa::row_blocks(n)), dim3(fa::kRowWG), 0, ctx->stream, sim, n,
-                     (int)k, index, similarity);
-  FA_CHECK_LAUNCH(ctx);
-  return FA_OK;
+  if (!fa::nearest_fused_ok(x, centres, k, d) && (rc = ws.ensure(ctx, (size_t)n * k * 4))) return rc;
+  return fa::launch_nearest(ctx, x, n, centres, k, d, ws.as<float>(), index, similarity);
 }
 
 int fa_cluster_nearest(fa_ctx* ctx, const float* x, int64_t n, const float* centres, int64_t k, int32_t d,
@@ -622,9 +833,9 @@ int fa_cluster_kmeans_dev(fa_ctx* ctx, const float* x, int64_t n, int32_t d, int
     return o;
   };
   const size_t o_raw = take((size_t)k * d * 4), o_sums = take((size_t)k * d * 4), o_best = take((size_t)n * 4),
-               o_w = take((size_t)n * 8), o_part = take((size_t)nparts * 8), o_sim = take((size_t)n * k * 4),
+               o_w = take((size_t)n * 8), o_part = take((size_t)nparts * 8), o_sim = take(fa::nearest_fused_ok(x, centres, k, d) ? 0 : (size_t)n * k * 4),
                o_cnt = take((size_t)nchunks * k * 4), o_chg = take((size_t)nchunks * 4), o_offs = take((size_t)k * 4),
-               o_list = take((size_t)n * 4), o_prev = take((size_t)n * 4), o_changed = take(4),
+               o_list = take((size_t)n * 4), o_prev = take((size_t)n * 4), o_summary = take(((size_t)k + 1) * 4),
                o_chosen = take((size_t)k * 4);
   fa::DevBuf& ws = ctx->slot(S_CL_WORK);
   if ((rc = ws.ensure(ctx, off))) return rc;
@@ -640,7 +851,7 @@ int fa_cluster_kmeans_dev(fa_ctx* ctx, const float* x, int64_t n, int32_t d, int
   int32_t* offs = (int32_t*)(base + o_offs);
   int32_t* list = (int32_t*)(base + o_list);
   int32_t* prev = (int32_t*)(base + o_prev);
-  int32_t* changed = (int32_t*)(base + o_changed);
+  int32_t* summary = (int32_t*)(base + o_summary);
   int32_t* chosen = (int32_t*)(base + o_chosen);
 
   // k-means++ seeding (cluster.go:47-85); every draw up front
@@ -652,14 +863,15 @@ int fa_cluster_kmeans_dev(fa_ctx* ctx, const float* x, int64_t n, int32_t d, int
   hipLaunchKernelGGL(fa::fill_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, best, n, -1.f);
   FA_CHECK_LAUNCH(ctx);
   for (int r = 1; r < k; r++) {
-    hipLaunchKernelGGL(fa::kpp_weights_kernel, dim3(fa::row_blocks(n)), dim3(fa::kRowWG), 0, st, x, n, (int)d,
-                       (const float*)(raw + (size_t)(r - 1) * d), best, w);
+    hipLaunchKernelGGL(fa::kpp_weights_kernel, dim3((unsigned)nparts), dim3(64 * fa::kKppWaves), 0, st, x, n, (int)d,
+                       (const float*)(raw + (size_t)(r - 1) * d), best, w, part);
     FA_CHECK_LAUNCH(ctx);
-    hipLaunchKernelGGL(fa::block_sums_kernel, dim3((unsigned)nparts), dim3(fa::kSumBlock), 0, st, (const double*)w,
-                       n, part);
-    FA_CHECK_LAUNCH(ctx);
-    hipLaunchKernelGGL(fa::kpp_pick_kernel, dim3(1), dim3(fa::kPickThreads), 0, st, (const double*)w, n,
-                       (const double*)part, nparts, u[r], x, (int)d, raw + (size_t)r * d, chosen + r);
+    if (nparts <= 256)
+      hipLaunchKernelGGL(fa::kpp_pick_kernel<256>, dim3(1), dim3(256), 0, st, (const double*)w, n,
+                         (const double*)part, nparts, u[r], x, (int)d, raw + (size_t)r * d, chosen + r);
+    else
+      hipLaunchKernelGGL(fa::kpp_pick_kernel<1024>, dim3(1), dim3(1024), 0, st, (const double*)w, n,
+                         (const double*)part, nparts, u[r], x, (int)d, raw + (size_t)r * d, chosen + r);
     FA_CHECK_LAUNCH(ctx);
   }
   if ((rc = fa::launch_normalize(ctx, raw, k, d, centres))) return rc;
@@ -673,17 +885,14 @@ int fa_cluster_kmeans_dev(fa_ctx* ctx, const float* x, int64_t n, int32_t d, int
   int it_done = 0;
   for (int it = 1; it <= iters; it++) {
     it_done = it;
-    if ((rc = fa::launch_sim(ctx, x, n, centres, k, d, sim))) return rc;
-    hipLaunchKernelGGL(fa::argmax_rows_kernel, dim3(fa::row_blocks(n)), dim3(fa::kRowWG), 0, st,
-                       (const float*)sim, n, (int)k, assignment, similarity);
-    FA_CHECK_LAUNCH(ctx);
+    if ((rc = fa::launch_nearest(ctx, x, n, centres, k, d, sim, assignment, similarity))) return rc;
     hipLaunchKernelGGL(fa::count_kernel, dim3((unsigned)nchunks), dim3(fa::kChunk), 0, st,
                        (const int32_t*)assignment, prev, n, (int)k, nchunks, cnt, chg);
     FA_CHECK_LAUNCH(ctx);
     hipLaunchKernelGGL(fa::chunk_scan_kernel, dim3((unsigned)k), dim3(256), 0, st, cnt, nchunks, sizes);
     FA_CHECK_LAUNCH(ctx);
     hipLaunchKernelGGL(fa::offsets_kernel, dim3(1), dim3(1024), 0, st, (const int32_t*)sizes, (int)k, offs,
-                       (const int32_t*)chg, nchunks, changed);
+                       (const int32_t*)chg, nchunks, summary);
     FA_CHECK_LAUNCH(ctx);
     hipLaunchKernelGGL(fa::scatter_kernel, dim3((unsigned)nchunks), dim3(64), 0, st, (const int32_t*)assignment, n,
                        (int)k, nchunks, (const int32_t*)offs, (const int32_t*)cnt, list);
@@ -691,8 +900,7 @@ int fa_cluster_kmeans_dev(fa_ctx* ctx, const float* x, int64_t n, int32_t d, int
     hipLaunchKernelGGL(fa::colsum_kernel, dim3((unsigned)k, (unsigned)((d + 63) / 64)), dim3(64), 0, st, x, (int)d,
                        (const int32_t*)list, (const int32_t*)offs, (const int32_t*)sizes, sums);
     FA_CHECK_LAUNCH(ctx);
-    FA_HIP_CHECK(ctx, hipMemcpyAsync(host.data(), sizes, (size_t)k * 4, hipMemcpyDeviceToHost, st));
-    FA_HIP_CHECK(ctx, hipMemcpyAsync(host.data() + k, changed, 4, hipMemcpyDeviceToHost, st));
+    FA_HIP_CHECK(ctx, hipMemcpyAsync(host.data(), summary, ((size_t)k + 1) * 4, hipMemcpyDeviceToHost, st));
     FA_HIP_CHECK(ctx, hipStreamSynchronize(st));
     for (int c = 0; c < k; c++) {
       if (host[c] != 0) continue;

@@ -172,3 +172,36 @@ def test_nearest_and_kmeans_speed():
     t = time.perf_counter()
     r = CL.KMeans(x, 40, 20, 1)
     print(f"KMeans 50000x768 k=40 iters={r.Iterations}: {(time.perf_counter() - t) * 1e3:.1f} ms", flush=True)
+
+
+@pytest.mark.parametrize("n,k,d", [(1, 1, 16), (31, 2, 8), (127, 16, 120), (129, 32, 128), (300, 33, 136), (513, 49, 264),
+                                   (1000, 64, 768)])
+def test_nearest_fused_edges(n, k, d):
+    """The fused product and argmax at the edges of its 32-row and 32-centre
+    blocks and 128-column parts. Entries are small integers: every similarity
+    is exact and ties are frequent (the first index wins); a NaN row takes
+    centre 0, a NaN centre is never taken except as index 0 (the rule of
+    Argmax, tensor/reduce.go:269-297)."""
+    r = np.random.default_rng(n + d)
+    x, c = (r.integers(-2, 3, (m, d)).astype(np.float32) for m in (n, k))
+    if n > 4:
+        x[2] = np.nan
+    if k > 3:
+        c[3] = np.nan
+    s = x.astype(np.float64) @ c.astype(np.float64).T
+    want = np.argmax(np.where(np.isnan(s), -np.inf, s), axis=1)
+    want[np.isnan(s[:, 0])] = 0
+    idx, sim = CL.Nearest(x, c)
+    assert np.array_equal(idx, want)
+    np.testing.assert_array_equal(sim, s[np.arange(n), want].astype(np.float32))
+
+
+@pytest.mark.parametrize("n,k", [(65, 2), (256, 7), (257, 40), (70000, 3)])
+def test_kmeans_group_edges(n, k):
+    """Row counts around the 256-row weight blocks and the 64-row sum groups,
+    and more than 256 weight blocks."""
+    rng = np.random.default_rng(n)
+    x, _ = planted(rng, n, 32, k, 0.02)
+    got, want = CL.KMeans(x, k, 10, 5), O.cluster_kmeans(x, k, 10, 5)
+    assert np.array_equal(got.Assignment, want["assignment"]) and np.array_equal(got.Sizes, want["sizes"])
+    np.testing.assert_allclose(got.Centres, want["centres"], rtol=0, atol=1e-5)
