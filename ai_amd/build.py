@@ -36,7 +36,7 @@ HIP_FLAGS = [
     "-I", INCLUDE, "-I", CSRC,
 ]
 
-ROCM_SOURCES = ["context.cpp", "matmul.cpp", "model.cpp", "plan.cpp", "gemm.hip", "gemm_h2.hip", "rowops.hip", "attention.hip", "score.hip", "score_few.hip", "cluster.hip"]
+ROCM_SOURCES = ["context.cpp", "matmul.cpp", "model.cpp", "plan.cpp", "gemm.hip", "gemm_h2.hip", "rowops.hip", "attention.hip", "attention_split.hip", "score.hip", "score_few.hip", "cluster.hip"]
 
 
 def _run(cmd: list[str], verbose: bool) -> None:

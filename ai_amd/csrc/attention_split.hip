@@ -1,0 +1,520 @@
+// The tensor.AttentionScaled drop-in at head_dim 64, 128 and 256 on the 16-bit
+// MFMA with fp32 accuracy, for any operands: attention_dense_kernel
+// (attention.hip) runs the same products on the fp32 MFMA, a sixteenth of
+// that rate, and stays for small calls and head_dim 512. 8 x 8 heads x 512 x 512,
+// head_dim 64: 62 -> 40 us per call (8 of them the image pass); 32 x 3 x 256 x 256
+// on one kv head, head_dim 256, padded: 102 -> 65. What bounds it now: the
+// softmax's VALU work at head_dim 64, the operand reads from LDS (2.4 of 2.9 us
+// per 32 keys) and the prologue at 256.
+//
+// Scores: q and k as two fp16 terms each, hi = fp16(x s) and lo = fp16((x s -
+// hi) 2^11) with one power of two s per row (query or key) that brings the
+// row's largest value to [2^14, 2^15): 23 bits down to 2^-27 of the row's
+// largest value. Three MFMAs per pair, hi.hi, hi.lo and lo.hi (one factor of
+// each product with a lo carries 2^-11), and each score times its row's and
+// its key's power of two. Values and probabilities: three exact bf16 terms
+// each (split3), six MFMAs per pair. bf16 has float32's range, so a masked
+// key may hold any finite value without touching its neighbours.
+//
+// split_kv_kernel writes, per (batch, kv head, tile of 32 keys), a key image
+// [term][key][HD], a value image [term][dim][32 slots] and the keys' powers
+// of two, in the order in which the attention's direct global->LDS loads and
+// operand reads take them: 16-byte chunk c of key k at c ^ (k mod 16) (head_dim
+// 64: c ^ (k / 2 mod 8)), slot 8g + 4h + r of a dim holding key 16h + 4g + r,
+// chunk g of dim d at g ^ (d / 4 mod 4); 16 lanes then read 16 different bank
+// groups. Heads that share one key/value head share its images.
+//
+// attention_split_kernel: a workgroup of W waves takes 16 W queries of one
+// (batch, head), a wave 16 (v_mfma_f32_16x16x32): S^T = K . Q^T puts a query's
+// scores in the four lanes that share l % 16, and its probabilities are then
+// the B operand of O^T += V^T . P^T as they are. Per stage of SK keys (64 at
+// head_dim 64): [barrier: this stage's keys and the previous stage's values
+// landed] load this stage's values and the next keys (head_dim 256 has room for
+// one key buffer: they load after a second barrier); scores; P.V of the previous
+// stage; softmax. P.V one stage behind leaves the values a whole stage to land
+// (2 048 queries and keys, 3 heads
+// of 256: 211 -> 192 us per call). The row maximum is lazy: the
+// offset moves when a stage's maximum exceeds it by more than 8.
+#include <cstdlib>
+
+#include "fa_internal.h"
+#include "device_math.h"
+
+namespace fa {
+namespace {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr float kSplitTau = 8.f;
+
+template <int HD>
+__device__ __forceinline__ int key_chunk(int key, int c) {
+  return HD == 64 ? c ^ ((key >> 1) & 7) : c ^ (key & 15);
+}
+__device__ __forceinline__ int slot_chunk(int dim, int g) { return g ^ ((dim >> 2) & 3); }
+
+// The power of two that brings m (>= 0) to [2^14, 2^15), and its inverse; 1
+// for 0, infinities and NaN (whose terms are not finite either way).
+__device__ __forceinline__ void row_pow2(float m, float& s, float& inv) {
+  const int e = (int)((__float_as_uint(m) >> 23) & 0xFF) - 127;  // exponent; 128: not finite
+  const int sh = m == 0.f || e == 128 ? 0 : 14 - max(e, -100);
+  s = ldexpf(1.f, min(sh, 120));
+  inv = ldexpf(1.f, -min(sh, 120));
+}
+
+__device__ __forceinline__ void split_row8(const float (&x)[8], float s, f16x8& hi, f16x8& lo) {
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const uint32_t w = split2(x[e] * s);
+    hi[e] = __builtin_bit_cast(_Float16, (uint16_t)(w & 0xFFFFu));
+    lo[e] = __builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
+  }
+}
+
+struct SplitKvParams {
+  const float *k, *v;
+  int64_t k_sb, k_sh, v_sb, v_sh;
+  int Hk, S, tiles;  // kv heads with images of their own; tiles per (batch, kv head)
+  uint16_t *kimg, *vimg;
+  float* kinv;
+};
+
+template <int HD>
+__global__ __launch_bounds__(256) void split_kv_kernel(SplitKvParams p) {
+  constexpr int VST = HD + 4;
+  __shared__ __attribute__((aligned(16))) float Vt[32 * VST];
+  const int64_t at = blockIdx.x;  // (batch * Hk + kv head) * tiles + tile
+  const int64_t bh = at / p.tiles;
+  const int t0 = (int)(at - bh * p.tiles) * 32, n = p.S - t0;  // n <= 0: a padding tile
+  const int b = (int)(bh / p.Hk), h = (int)(bh - (int64_t)b * p.Hk);
+  const float* kb = p.k + b * p.k_sb + h * p.k_sh;
+  const float* vb = p.v + b * p.v_sb + h * p.v_sh;
+  uint16_t* ko = p.kimg + at * (2 * 32 * HD);
+  uint16_t* vo = p.vimg + at * (3 * 32 * HD);
+  constexpr int CH = HD / 8;          // chunks (threads) per key
+  constexpr int KPP = 256 / CH;       // keys per pass
+  const int c = threadIdx.x % CH;
+  float x[32 / KPP][8], y[32 / KPP][8];
+#pragma unroll
+  for (int i = 0; i < 32 / KPP; i++) {
+    const int key = threadIdx.x / CH + i * KPP;
+    const int64_t row = (int64_t)min(t0 + key, p.S - 1) * HD + 8 * c;
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(kb + row + e), w = *reinterpret_cast<const f32x4*>(vb + row + e);
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        x[i][e + q] = key < n ? a[q] : 0.f;
+        y[i][e + q] = key < n ? w[q] : 0.f;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 32 / KPP; i++) {
+    const int key = threadIdx.x / CH + i * KPP;
+    float m = 0.f;
+    bool fin = true;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      m = fmaxf(m, fabsf(x[i][e]));
+      fin = fin && x[i][e] == x[i][e];
+    }
+    if (!fin) m = INFINITY;
+#pragma unroll
+    for (int o = CH / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    float s, inv;
+    row_pow2(m, s, inv);
+    f16x8 hi, lo;
+    split_row8(x[i], s, hi, lo);
+    uint16_t* o16 = ko + key * HD + key_chunk<HD>(key, c) * 8;
+    *reinterpret_cast<f16x8*>(o16) = hi;
+    *reinterpret_cast<f16x8*>(o16 + 32 * HD) = lo;
+    if (c == 0) p.kinv[at * 32 + key] = inv;
+#pragma unroll
+    for (int e = 0; e < 8; e += 4)
+      *reinterpret_cast<f32x4*>(&Vt[key * VST + 8 * c + e]) = f32x4{y[i][e], y[i][e + 1], y[i][e + 2], y[i][e + 3]};
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < HD * 4 / 256; i++) {
+    const int u = threadIdx.x + 256 * i, d = u >> 2, g = u & 3;
+    uint32_t th[8], tm[8], tl[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const Split3 sp = split3(Vt[((e >> 2) * 16 + 4 * g + (e & 3)) * VST + d]);
+      th[e] = sp.h;
+      tm[e] = sp.m;
+      tl[e] = sp.l;
+    }
+    uint16_t* o = vo + d * 32 + slot_chunk(d, g) * 8;
+    *reinterpret_cast<uint4*>(o) =
+        make_uint4(pack_hi16(th[0], th[1]), pack_hi16(th[2], th[3]), pack_hi16(th[4], th[5]), pack_hi16(th[6], th[7]));
+    *reinterpret_cast<uint4*>(o + 32 * HD) =
+        make_uint4(pack_hi16(tm[0], tm[1]), pack_hi16(tm[2], tm[3]), pack_hi16(tm[4], tm[5]), pack_hi16(tm[6], tm[7]));
+    *reinterpret_cast<uint4*>(o + 64 * HD) =
+        make_uint4(pack_hi16(tl[0], tl[1]), pack_hi16(tl[2], tl[3]), pack_hi16(tl[4], tl[5]), pack_hi16(tl[6], tl[7]));
+  }
+}
+
+struct SplitParams {
+  const float *q, *mask;
+  const uint16_t *kimg, *vimg;
+  const float* kinv;
+  float* out;
+  int H, Hk, T, S, tiles, qblocks;
+  int64_t q_sb, q_sh, m_sb, m_sh, m_sr, m_sc;
+  float scale;
+};
+
+// Workgroup barriers after the wave's vector loads and LDS accesses, and after
+// its LDS accesses alone.
+__device__ __forceinline__ void split_barrier() {
+  __builtin_amdgcn_s_waitcnt(7 << 4);  // vmcnt(0) lgkmcnt(0)
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+__device__ __forceinline__ void split_lds_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+__device__ __forceinline__ float lanes4_max(float x) {  // lanes l, l ^ 16, l ^ 32, l ^ 48
+  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float lanes4_sum(float x) {
+  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+template <int HD, int W, bool MASK>
+__global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams p) {
+  constexpr int SK = HD == 64 ? 64 : 32;  // keys per stage
+  constexpr int NT = SK / 32;             // tiles per stage
+  constexpr int NC = HD / 32, NDB = HD / 16;
+  constexpr int KI = 2 * 32 * HD, VI = 3 * 32 * HD;  // 16-bit values of a tile's images
+  static_assert(NT * KI % (64 * W * 8) == 0 && NT * VI % (64 * W * 8) == 0, "whole loads");
+  constexpr bool KD = HD < 256;  // two key buffers
+  __shared__ __attribute__((aligned(16))) uint16_t K0[NT * KI], K1[KD ? NT * KI : 8], V0[NT * VI], V1[NT * VI];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lq = lane & 15, g = lane >> 4;
+  const int bh = blockIdx.x / p.qblocks, qblk = blockIdx.x % p.qblocks;
+  const int b = bh / p.H, h = bh % p.H;
+  const int64_t img = ((int64_t)b * p.Hk + (p.Hk == 1 ? 0 : h)) * p.tiles;
+  const uint16_t* kimg = p.kimg + img * KI;
+  const uint16_t* vimg = p.vimg + img * VI;
+  const float* kinv = p.kinv + img * 32;
+  const int stages = (p.S + SK - 1) / SK;
+
+  auto load_k = [&](uint16_t* dst, int st) {
+#pragma unroll
+    for (int i = 0; i < NT * KI / 8 / 64 / W; i++)
+      __builtin_amdgcn_global_load_lds(kimg + (int64_t)st * NT * KI + ((i * W + wave) * 64 + lane) * 8,
+                                       (__attribute__((address_space(3))) void*)(dst + (i * W + wave) * 512), 16, 0, 0);
+  };
+  auto load_v = [&](uint16_t* dst, int st) {
+#pragma unroll
+    for (int i = 0; i < NT * VI / 8 / 64 / W; i++)
+      __builtin_amdgcn_global_load_lds(vimg + (int64_t)st * NT * VI + ((i * W + wave) * 64 + lane) * 8,
+                                       (__attribute__((address_space(3))) void*)(dst + (i * W + wave) * 512), 16, 0, 0);
+  };
+  load_k(K0, 0);
+
+  // the wave's queries: their terms in registers (qh2 = qh 2^-11, the factor
+  // of the keys' lo terms)
+  const int qi = (qblk * W + wave) * 16 + lq;
+  const bool qvalid = qi < p.T;
+  const int qc = min(qi, p.T - 1);
+  f16x8 qh[NC], qh2[NC], ql[NC];
+  float qinv;
+  {
+    const float* qr = p.q + b * p.q_sb + h * p.q_sh + (int64_t)qc * HD + 8 * g;
+    float x[NC][8];
+    float m = 0.f;
+    bool fin = true;
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(qr + 32 * c + e);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          x[c][e + u] = a[u];
+          m = fmaxf(m, fabsf(a[u]));
+          fin = fin && a[u] == a[u];
+        }
+      }
+    if (!fin) m = INFINITY;
+    m = lanes4_max(m);
+    float s;
+    row_pow2(m, s, qinv);
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      split_row8(x[c], s, qh[c], ql[c]);
+      qh2[c] = qh[c] * (_Float16)0x1p-11f;
+    }
+  }
+  const float* mrow = MASK ? p.mask + b * p.m_sb + h * p.m_sh + (int64_t)qc * p.m_sr : nullptr;
+  const float qf = qinv * p.scale;
+
+  f32x4 oacc[NDB];  // O^T: dims 16 db + 4 g + r of query lq
+#pragma unroll
+  for (int db = 0; db < NDB; db++) oacc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -1e30f, l_part = 0.f;
+
+  bf16x8 pt[NT][3];   // the previous stage's probability terms
+  bool live = false;  // whether any of them is not 0
+  auto pv = [&](const uint16_t* Vc) {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int db = 0; db < NDB; db++) {
+        const int dim = 16 * db + lq;
+        const uint16_t* vr = Vc + t * VI + dim * 32 + slot_chunk(dim, g) * 8;
+        const bf16x8 v0 = *reinterpret_cast<const bf16x8*>(vr);
+        const bf16x8 v1 = *reinterpret_cast<const bf16x8*>(vr + 32 * HD);
+        const bf16x8 v2 = *reinterpret_cast<const bf16x8*>(vr + 64 * HD);
+        f32x4 o = oacc[db];
+        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v2, pt[t][0], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, pt[t][2], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, pt[t][1], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, pt[t][0], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, pt[t][1], o, 0, 0, 0);
+        oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, pt[t][0], o, 0, 0, 0);
+      }
+  };
+  // a stage's key factors and mask values: keys 4g .. + 3 of the tiles' halves
+  float kn[NT][8], mn_[NT][8];
+  auto fetch = [&](int st) {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        const int j0 = st * SK + 32 * t + 4 * e + 4 * g;
+        const f32x4 a = *reinterpret_cast<const f32x4*>(kinv + j0);
+#pragma unroll
+        for (int u = 0; u < 4; u++) kn[t][e + u] = a[u];
+        if constexpr (MASK) {
+#pragma unroll
+          for (int u = 0; u < 4; u++) mn_[t][e + u] = mrow[(int64_t)min(j0 + u, p.S - 1) * p.m_sc];
+        }
+      }
+  };
+  fetch(0);
+  auto stage = [&](int st, const uint16_t* Kc, uint16_t* Kn, uint16_t* Vn, const uint16_t* Vp) {
+    split_barrier();  // this stage's keys, the last one's values landed; every wave is done with the last stage
+    // the key factors and mask values loaded during the last stage: taken here,
+    // where the barrier has waited for them. A use after the loads below would
+    // wait for those too (the compiler does not count direct loads in order).
+    float kf[NT][8], mv[NT][8];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        asm volatile("" : "+v"(kn[t][e]));
+        kf[t][e] = kn[t][e];
+        if constexpr (MASK) {
+          asm volatile("" : "+v"(mn_[t][e]));
+          mv[t][e] = mn_[t][e];
+        }
+      }
+    fetch(min(st + 1, stages - 1));
+    load_v(Vn, st);
+    if constexpr (KD) load_k(Kn, min(st + 1, stages - 1));
+    f32x4 sacc[NT][2];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int kb = 0; kb < 2; kb++) {
+        f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int key = 16 * kb + lq;
+        const uint16_t* kr = Kc + t * KI + key * HD;
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          const int pos = key_chunk<HD>(key, 4 * c + g) * 8;
+          const f16x8 k0 = *reinterpret_cast<const f16x8*>(kr + pos);
+          const f16x8 k1 = *reinterpret_cast<const f16x8*>(kr + 32 * HD + pos);
+          s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, qh2[c], s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0 * (_Float16)0x1p-11f, ql[c], s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qh[c], s, 0, 0, 0);
+        }
+        sacc[t][kb] = s;
+      }
+    if constexpr (!KD) {
+      split_lds_barrier();  // every wave has read the keys
+      load_k(Kn, min(st + 1, stages - 1));
+    }
+    if (live) pv(Vp);
+    float w[NT][8];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        w[t][e] = sacc[t][e >> 2][e & 3] * (kf[t][e] * qf);
+        if constexpr (MASK) w[t][e] += mv[t][e];
+      }
+    if (st * SK + SK > p.S) {  // the last stage: no keys past S
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          if (st * SK + 32 * t + 16 * (e >> 2) + 4 * g + (e & 3) >= p.S) w[t][e] = -INFINITY;
+    }
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) tmax = fmaxf(tmax, w[t][e]);
+    tmax = lanes4_max(tmax);
+    const bool need = tmax > m_run + kSplitTau;
+    const float mn = need ? tmax : m_run;
+    if (__any(need)) {
+      const float alpha = exp_flush(m_run - mn);  // 0 for the first stage
+      l_part *= alpha;
+#pragma unroll
+      for (int db = 0; db < NDB; db++) oacc[db] *= alpha;
+    }
+    m_run = mn;
+    // a stage whose every weight flushes to 0 (padding, outside a window)
+    // adds nothing: no weights, no P.V, unless a score is NaN (which the
+    // maximum passes over)
+    live = __any(tmax - mn >= -87.f);
+    if (!live) {
+      bool nan = false;
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) nan = nan || w[t][e] != w[t][e];
+      live = __any(nan);
+    }
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      if (!live) break;
+      uint32_t ph[8], pm[8], pl[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const float x = exp_flush(w[t][e] - mn);
+        l_part += x;
+        const Split3 sp = split3(x);
+        ph[e] = sp.h;
+        pm[e] = sp.m;
+        pl[e] = sp.l;
+      }
+      pt[t][0] = __builtin_bit_cast(bf16x8, (u32x4){pack_hi16(ph[0], ph[1]), pack_hi16(ph[2], ph[3]),
+                                                    pack_hi16(ph[4], ph[5]), pack_hi16(ph[6], ph[7])});
+      pt[t][1] = __builtin_bit_cast(bf16x8, (u32x4){pack_hi16(pm[0], pm[1]), pack_hi16(pm[2], pm[3]),
+                                                    pack_hi16(pm[4], pm[5]), pack_hi16(pm[6], pm[7])});
+      pt[t][2] = __builtin_bit_cast(bf16x8, (u32x4){pack_hi16(pl[0], pl[1]), pack_hi16(pl[2], pl[3]),
+                                                    pack_hi16(pl[4], pl[5]), pack_hi16(pl[6], pl[7])});
+    }
+  };
+  for (int st = 0; st < stages; st += 2) {
+    stage(st, K0, KD ? K1 : K0, V0, V1);
+    if (st + 1 < stages) stage(st + 1, KD ? K1 : K0, K0, V1, V0);
+  }
+  split_barrier();  // the last values (no load may still be writing LDS when the workgroup ends)
+  if (live) pv((stages & 1) ? V0 : V1);
+
+  const float inv = 1.f / lanes4_sum(l_part);
+  if (!qvalid) return;
+  float* orow = p.out + ((int64_t)bh * p.T + qi) * HD + 4 * g;
+#pragma unroll
+  for (int db = 0; db < NDB; db++) *reinterpret_cast<f32x4*>(orow + 16 * db) = oacc[db] * inv;
+}
+
+struct SplitSizes {
+  int Hk, tiles;
+  int64_t blocks;  // images
+  size_t k_bytes, v_bytes;
+};
+SplitSizes split_sizes(const AttnGenericArgs& a) {
+  SplitSizes z;
+  z.Hk = a.k_sh == 0 && a.v_sh == 0 ? 1 : a.H;
+  const int sk = a.D == 64 ? 64 : 32;
+  z.tiles = (a.S + sk - 1) / sk * (sk / 32);
+  z.blocks = (int64_t)a.B * z.Hk * z.tiles;
+  z.k_bytes = (size_t)z.blocks * 2 * 32 * a.D * 2;
+  z.v_bytes = (size_t)z.blocks * 3 * 32 * a.D * 2;
+  return z;
+}
+
+template <int HD, int W>
+void launch_split(const SplitParams& p, int64_t grid, hipStream_t s) {
+  if (p.mask)
+    hipLaunchKernelGGL((attention_split_kernel<HD, W, true>), dim3((unsigned)grid), dim3(64 * W), 0, s, p);
+  else
+    hipLaunchKernelGGL((attention_split_kernel<HD, W, false>), dim3((unsigned)grid), dim3(64 * W), 0, s, p);
+}
+
+}  // namespace
+
+// With few keys or little work the image pass and the longer prologue cost
+// what the products save. Measured, us against attention_dense_kernel: 32 x 8
+// heads x 64 x 64 keys, head_dim 64: 14.5 and 7.9; 8 x 3 x 128 x 128, 256: 33 and
+// 22; 1 x 3 x 200 x 200, 256: 33 and 28; and 1 x 8 x 256 x 256, 64: 14 and 20; 2 x 4 x
+// 300 x 300, 128: 24 and 42; 1 x 3 x 512 x 512, 256: 58 and 65. (FA_ATTN_SPLIT=0
+// turns it off, for comparisons.)
+bool attention_split_ok(const AttnGenericArgs& a) {
+  static const bool off = [] {
+    const char* e = std::getenv("FA_ATTN_SPLIT");
+    return e && e[0] == '0';
+  }();
+  if (off || !attention_dense_ok(a) || (a.D != 64 && a.D != 128 && a.D != 256)) return false;
+  if (!(a.scale > 0.f) || a.S < 192 || 4.0 * a.B * a.H * (double)a.T * a.S * a.D < (a.D == 256 ? 5e8 : 1e8)) return false;
+  const SplitSizes z = split_sizes(a);
+  return z.blocks < INT32_MAX && (int64_t)a.B * a.H * ((a.T + 63) / 64) < INT32_MAX;
+}
+
+int launch_attention_split(fa_ctx* ctx, const AttnGenericArgs& a, hipStream_t s) {
+  if (!attention_split_ok(a)) return set_error(ctx, FA_ERR_UNSUPPORTED, "Attention: no split path for these operands");
+  const SplitSizes z = split_sizes(a);
+  DevBuf& buf = ctx->slot(slots::S_ATTN);
+  if (const int rc = buf.ensure(ctx, z.k_bytes + z.v_bytes + (size_t)z.blocks * 32 * 4)) return rc;
+  SplitKvParams kv;
+  kv.k = a.k; kv.v = a.v; kv.k_sb = a.k_sb; kv.k_sh = a.k_sh; kv.v_sb = a.v_sb; kv.v_sh = a.v_sh;
+  kv.Hk = z.Hk; kv.S = a.S; kv.tiles = z.tiles;
+  kv.kimg = buf.as<uint16_t>();
+  kv.vimg = reinterpret_cast<uint16_t*>(buf.as<char>() + z.k_bytes);
+  kv.kinv = reinterpret_cast<float*>(buf.as<char>() + z.k_bytes + z.v_bytes);
+  SplitParams p;
+  p.q = a.q; p.mask = a.mask; p.kimg = kv.kimg; p.vimg = kv.vimg; p.kinv = kv.kinv; p.out = a.out;
+  p.H = a.H; p.Hk = z.Hk; p.T = a.T; p.S = a.S; p.tiles = z.tiles;
+  p.q_sb = a.q_sb; p.q_sh = a.q_sh; p.m_sb = a.m_sb; p.m_sh = a.m_sh; p.m_sr = a.m_sr; p.m_sc = a.m_sc;
+  p.scale = a.scale;
+  // 128 queries per workgroup, or 64 where those leave CUs without one
+  const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  const int64_t bh = (int64_t)a.B * a.H;
+  const int W = bh * ((a.T + 127) / 128) >= cus / 2 && (a.T + 127) / 128 * 128 - a.T < 64 ? 8 : 4;
+  p.qblocks = (a.T + 16 * W - 1) / (16 * W);
+  const dim3 gk((unsigned)z.blocks), bk(256);
+  switch (a.D) {
+    case 64:
+      hipLaunchKernelGGL(split_kv_kernel<64>, gk, bk, 0, s, kv);
+      if (W == 8) launch_split<64, 8>(p, bh * p.qblocks, s);
+      else launch_split<64, 4>(p, bh * p.qblocks, s);
+      break;
+    case 128:
+      hipLaunchKernelGGL(split_kv_kernel<128>, gk, bk, 0, s, kv);
+      if (W == 8) launch_split<128, 8>(p, bh * p.qblocks, s);
+      else launch_split<128, 4>(p, bh * p.qblocks, s);
+      break;
+    default:
+      hipLaunchKernelGGL(split_kv_kernel<256>, gk, bk, 0, s, kv);
+      if (W == 8) launch_split<256, 8>(p, bh * p.qblocks, s);
+      else launch_split<256, 4>(p, bh * p.qblocks, s);
+      break;
+  }
+  FA_CHECK_LAUNCH(ctx);
+  return FA_OK;
+}
+
+}  // namespace fa

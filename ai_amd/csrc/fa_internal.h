@@ -57,6 +57,7 @@ enum : size_t {
   S_TOPK,                               // top-k candidates
   S_BPLANES,                            // B operand as bf16 [n x k] planes (matmul drop-in)
   S_APACK,                              // A operand packed to [nb][m][kp] (strided matmul)
+  S_ATTN,                               // key and value images (attention drop-in)
   S_COUNT
 };
 }  // namespace slots
@@ -236,6 +237,10 @@ int launch_attention_generic(fa_ctx* ctx, const AttnGenericArgs& a, hipStream_t 
 // turns it off, for comparisons), and its launch.
 bool attention_dense_ok(const AttnGenericArgs& a);
 int launch_attention_dense(fa_ctx* ctx, const AttnGenericArgs& a, hipStream_t s);
+// The same on the 16-bit MFMA (attention_split.hip): head_dim 64/128/256,
+// scale > 0, and enough work to pay for the key/value image pass.
+bool attention_split_ok(const AttnGenericArgs& a);
+int launch_attention_split(fa_ctx* ctx, const AttnGenericArgs& a, hipStream_t s);
 
 // Per-row top-k of scores [nq x nd] (1 <= topk <= 32, nq <= 65535) into
 // idx/val [nq x topk]; scratch holds topk_scratch_bytes(nq, nd, topk) bytes

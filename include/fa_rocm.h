@@ -36,6 +36,7 @@
  *   FA_GEMM_MFMA=f32            the model's and fa_matmul_fused's products on the fp32-MFMA
  *                               kernel (bf16 weights widened, float32 weights without the
  *                               three-plane rewrite)
+ *   FA_ATTN_SPLIT=0             fa_attention without the 16-bit MFMA kernel
  *   FA_ATTN_DENSE=0             fa_attention on the per-row kernel for every head dim
  *   FA_GEMM_H2=0                the encoder's products on the three-term bf16 kernels (also
  *                               implied by FA_GEMM_MFMA=f32 and FA_GEMM_XTILE)
@@ -208,7 +209,8 @@ int fa_rope(fa_ctx* ctx, const float* x, double base, const int32_t* positions, 
  * contiguous. Masked weights are exactly 0 (exp of inputs below -87 flushes
  * to 0, internal/kernel/generic.go:278-307). Head dims 64, 128, 256 and
  * 512 with 16-byte aligned rows (batch and head strides multiples of 4) run
- * on the fp32 MFMA; other shapes on a per-row kernel (D <= 512).
+ * on the fp32 MFMA, or (64, 128 and 256, from 192 keys and about 0.1 GFLOP)
+ * on the 16-bit MFMA with fp32 accuracy; other shapes on a per-row kernel (D <= 512).
  * Replaces tensor.AttentionScaled (tensor/attention.go:67-83,130-287). */
 int fa_attention(fa_ctx* ctx, const float* q, const float* k, const float* v, int32_t B, int32_t H, int32_t T,
                  int32_t S, int32_t D, int64_t q_sb, int64_t q_sh, int64_t k_sb, int64_t k_sh, int64_t v_sb,

@@ -396,3 +396,45 @@ def test_attention_mfma_dev_entry_point(ctx):
     for p in ptrs:
         L.fa_device_free(ctx.h, p)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("D,B,H,Hkv,Tq,Sk,kind", [
+    (64, 1, 8, 8, 129, 449, "none"), (64, 2, 8, 1, 128, 192, "pad"), (64, 3, 4, 4, 200, 257, "full"),
+    (128, 1, 7, 7, 33, 1023, "none"), (128, 4, 4, 1, 65, 225, "full"), (256, 2, 3, 1, 257, 479, "pad"),
+    (256, 4, 3, 3, 200, 256, "full"), (256, 1, 2, 2, 1000, 321, "none")])
+def test_attention_split_edges(ctx, D, B, H, Hkv, Tq, Sk, kind):
+    """The 16-bit MFMA attention (attention_split.hip) around its 64/128-query
+    items and 32/64-key stages against float64. Rows of q and k, and q and k
+    against each other, are of very different magnitudes (their products are
+    not); values behind the padding mask hold 1e30. A score of magnitude s carries a float32
+    rounding of s * 2^-23 or so into its weight, so with |s| below 8 and sums of
+    at most 1 023 weights the output is within 4e-6 of the largest value."""
+    r = np.random.default_rng(D + Tq)
+    q = r.standard_normal((B, H, Tq, D)) * 2.0 ** 20
+    k = r.standard_normal((B, Hkv, Sk, D)) * 2.0 ** -20
+    k *= 2.0 ** r.integers(-12, 1, (B, Hkv, Sk, 1))
+    q *= 2.0 ** r.integers(-12, 1, (B, H, Tq, 1))
+    v = r.standard_normal((B, Hkv, Sk, D))
+    mask = None
+    if kind == "pad":
+        mask = T.PaddingMask([Sk - 70 - 60 * b for b in range(B)], Sk)
+    elif kind == "full":  # a bias and a window, one row with a single key
+        i, j = np.arange(Tq)[:, None], np.arange(Sk)[None]
+        mask = np.where(np.abs(i * Sk // Tq - j) < 40, -0.01 * np.abs(i - j), -1e9).astype(np.float32)
+        mask[5] = -1e9
+        mask[5, 17] = 0
+    q, k, v = (a.astype(np.float32) for a in (q, k, v))
+    s = np.einsum("bhtd,bhsd->bhts", q.astype(np.float64), np.repeat(k, H // Hkv, 1).astype(np.float64)) / np.sqrt(D)
+    if mask is not None:
+        s = s + mask.astype(np.float64)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    want = np.einsum("bhts,bhsd->bhtd", p, np.repeat(v, H // Hkv, 1).astype(np.float64))
+    if kind == "pad":  # finite garbage behind the mask changes nothing
+        for b in range(B):
+            k[b, :, Sk - 70 - 60 * b:] = 3e-6
+            v[b, :, Sk - 70 - 60 * b:] = 1e30
+    kb, vb = (np.broadcast_to(a, (B, H, Sk, D)) if Hkv == 1 else a for a in (k, v))
+    got = T.AttentionScaled(q, kb, vb, mask, float(1 / np.sqrt(D)), ctx=ctx)
+    assert np.isfinite(got).all()
+    assert np.abs(got - want).max() <= 4e-6 * np.abs(want).max()
