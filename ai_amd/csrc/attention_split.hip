@@ -21,8 +21,9 @@
 // of two, in the order in which the attention's direct global->LDS loads and
 // operand reads take them: 16-byte chunk c of key k at c ^ (k mod 16) (head_dim
 // 64: c ^ (k / 2 mod 8)), slot 8g + 4h + r of a dim holding key 16h + 4g + r,
-// chunk g of dim d at g ^ (d / 4 mod 4); 16 lanes then read 16 different bank
-// groups. Heads that share one key/value head share its images.
+// chunk g of dim d at g ^ (d / 2 mod 4), both free of bank conflicts (d / 4 mod 4
+// had a third of the value reads in conflict). Heads that share one key/value
+// head share its images.
 //
 // attention_split_kernel: a workgroup of W waves takes 16 W queries of one
 // (batch, head), a wave 16 (v_mfma_f32_16x16x32): S^T = K . Q^T puts a query's
@@ -53,7 +54,7 @@ template <int HD>
 __device__ __forceinline__ int key_chunk(int key, int c) {
   return HD == 64 ? c ^ ((key >> 1) & 7) : c ^ (key & 15);
 }
-__device__ __forceinline__ int slot_chunk(int dim, int g) { return g ^ ((dim >> 2) & 3); }
+__device__ __forceinline__ int slot_chunk(int dim, int g) { return g ^ ((dim >> 1) & 3); }
 
 // The power of two that brings m (>= 0) to [2^14, 2^15), and its inverse; 1
 // for 0, infinities and NaN (whose terms are not finite either way).
