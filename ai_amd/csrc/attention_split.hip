@@ -57,7 +57,7 @@ __device__ __forceinline__ int key_chunk(int key, int c) {
 __device__ __forceinline__ int slot_chunk(int dim, int g) { return g ^ ((dim >> 1) & 3); }
 
 // The power of two that brings m (>= 0) to [2^14, 2^15), and its inverse; 1
-// for 0, infinities and NaN (whose terms are not finite either way).
+// for 0, infinities and NaN (whose scores come out as NaN: plain_query).
 __device__ __forceinline__ void row_pow2(float m, float& s, float& inv) {
   const int e = (int)((__float_as_uint(m) >> 23) & 0xFF) - 127;  // exponent; 128: not finite
   const int sh = m == 0.f || e == 128 ? 0 : 14 - max(e, -100);
@@ -160,14 +160,46 @@ __global__ __launch_bounds__(256) void split_kv_kernel(SplitKvParams p) {
 }
 
 struct SplitParams {
-  const float *q, *mask;
+  const float *q, *k, *v, *mask;
   const uint16_t *kimg, *vimg;
   const float* kinv;
   float* out;
   int H, Hk, T, S, tiles, qblocks;
-  int64_t q_sb, q_sh, m_sb, m_sh, m_sr, m_sc;
+  int64_t q_sb, q_sh, k_sb, k_sh, v_sb, v_sh, m_sb, m_sh, m_sr, m_sc;
   float scale;
 };
+
+// One query in plain fp32, by one wave, lane l holding dims l, l + 64, ...:
+// for queries whose split result is not finite. An infinity has no finite
+// second term, and factors of rows of extreme magnitude can overflow where
+// their product does not, so the split gives NaN where the operands
+// themselves give an infinity, or a weight of 0.
+template <int HD, bool MASK>
+__device__ void plain_query(const SplitParams& p, int b, int h, int qi, int lane) {
+  constexpr int N = HD / 64;
+  const float* qr = p.q + b * p.q_sb + h * p.q_sh + (int64_t)qi * HD + lane;
+  const float* kr = p.k + b * p.k_sb + h * p.k_sh + lane;
+  const float* vr = p.v + b * p.v_sb + h * p.v_sh + lane;
+  const float* mrow = MASK ? p.mask + b * p.m_sb + h * p.m_sh + (int64_t)qi * p.m_sr : nullptr;
+  auto score = [&](int j) {
+    float s = 0.f;
+    for (int i = 0; i < N; i++) s = fmaf(qr[64 * i], kr[(int64_t)j * HD + 64 * i], s);
+    s = wave_sum(s) * p.scale;
+    if constexpr (MASK) s += mrow[(int64_t)j * p.m_sc];
+    return s;
+  };
+  float m = -1e30f;
+  for (int j = 0; j < p.S; j++) m = fmaxf(m, score(j));
+  float l = 0.f, o[N];
+  for (int i = 0; i < N; i++) o[i] = 0.f;
+  for (int j = 0; j < p.S; j++) {
+    const float w = exp_flush(score(j) - m);
+    l += w;
+    for (int i = 0; i < N; i++) o[i] = fmaf(w, vr[(int64_t)j * HD + 64 * i], o[i]);
+  }
+  float* orow = p.out + (((int64_t)b * p.H + h) * p.T + qi) * HD + lane;
+  for (int i = 0; i < N; i++) orow[64 * i] = o[i] * (1.f / l);
+}
 
 // Workgroup barriers after the wave's vector loads and LDS accesses, and after
 // its LDS accesses alone.
@@ -426,10 +458,22 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
   if (live) pv((stages & 1) ? V0 : V1);
 
   const float inv = 1.f / lanes4_sum(l_part);
-  if (!qvalid) return;
+  float seen = 0.f;  // NaN if any output is not finite
   float* orow = p.out + ((int64_t)bh * p.T + qi) * HD + 4 * g;
 #pragma unroll
-  for (int db = 0; db < NDB; db++) *reinterpret_cast<f32x4*>(orow + 16 * db) = oacc[db] * inv;
+  for (int db = 0; db < NDB; db++) {
+    const f32x4 o = oacc[db] * inv;
+#pragma unroll
+    for (int r = 0; r < 4; r++) seen = fmaf(o[r], 0.f, seen);
+    if (qvalid) *reinterpret_cast<f32x4*>(orow + 16 * db) = o;
+  }
+  uint64_t redo = __ballot(qvalid && seen != seen);
+  redo = (redo | redo >> 16 | redo >> 32 | redo >> 48) & 0xFFFFu;  // queries of the wave
+  if (redo) {
+    __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0): the stores above, which other lanes write over
+    for (int i = 0; i < 16; i++)
+      if (redo >> i & 1) plain_query<HD, MASK>(p, b, h, (qblk * W + wave) * 16 + i, lane);
+  }
 }
 
 struct SplitSizes {
@@ -487,9 +531,10 @@ int launch_attention_split(fa_ctx* ctx, const AttnGenericArgs& a, hipStream_t s)
   kv.vimg = reinterpret_cast<uint16_t*>(buf.as<char>() + z.k_bytes);
   kv.kinv = reinterpret_cast<float*>(buf.as<char>() + z.k_bytes + z.v_bytes);
   SplitParams p;
-  p.q = a.q; p.mask = a.mask; p.kimg = kv.kimg; p.vimg = kv.vimg; p.kinv = kv.kinv; p.out = a.out;
+  p.q = a.q; p.k = a.k; p.v = a.v; p.mask = a.mask; p.kimg = kv.kimg; p.vimg = kv.vimg; p.kinv = kv.kinv; p.out = a.out;
   p.H = a.H; p.Hk = z.Hk; p.T = a.T; p.S = a.S; p.tiles = z.tiles;
-  p.q_sb = a.q_sb; p.q_sh = a.q_sh; p.m_sb = a.m_sb; p.m_sh = a.m_sh; p.m_sr = a.m_sr; p.m_sc = a.m_sc;
+  p.q_sb = a.q_sb; p.q_sh = a.q_sh; p.k_sb = a.k_sb; p.k_sh = a.k_sh; p.v_sb = a.v_sb; p.v_sh = a.v_sh;
+  p.m_sb = a.m_sb; p.m_sh = a.m_sh; p.m_sr = a.m_sr; p.m_sc = a.m_sc;
   p.scale = a.scale;
   // 128 queries per workgroup, or 64 where those leave CUs without one
   const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;

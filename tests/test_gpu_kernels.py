@@ -438,3 +438,42 @@ def test_attention_split_edges(ctx, D, B, H, Hkv, Tq, Sk, kind):
     got = T.AttentionScaled(q, kb, vb, mask, float(1 / np.sqrt(D)), ctx=ctx)
     assert np.isfinite(got).all()
     assert np.abs(got - want).max() <= 4e-6 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("D,B,H,Tq,Sk,masked", [(64, 1, 8, 129, 449, False), (128, 2, 4, 150, 225, True),
+                                               (256, 2, 3, 257, 479, True)])
+def test_attention_split_infinities(ctx, D, B, H, Tq, Sk, masked):
+    """Infinities in keys and values, and rows whose magnitudes only meet in a
+    finite product, give what the float32 products give (a score of -inf is a
+    weight of 0, an infinite value under a weight an infinite output), on the
+    size range of the 16-bit MFMA attention. Finite outputs hold
+    test_attention_split_edges' bound."""
+    r = np.random.default_rng(D)
+    q = np.abs(r.standard_normal((B, H, Tq, D))).astype(np.float32)
+    k = (0.1 * r.standard_normal((B, H, Sk, D))).astype(np.float32)
+    v = r.standard_normal((B, H, Sk, D)).astype(np.float32)
+    k[:, 2:, 7, 3] = -np.inf  # a score of -inf
+    v[:, 0, 40, 5] = np.inf
+    v[:, 0, Sk - 2, 9] = -np.inf
+    q[:, 1, 3] = 0  # a query and a key, disjoint, of 2^100 and 2^90
+    q[:, 1, 3, 0] = 2.0 ** 100
+    k[:, 1, :, 0] = 0
+    k[:, 1, 60] = 0
+    k[:, 1, 60, 1] = 2.0 ** 90
+    q[:, 1, :3, 1] = q[:, 1, 4:, 1] = 0
+    mask = T.PaddingMask([Sk - 50, Sk - 90], Sk) if masked else None
+    if masked:
+        v[:, 0, Sk - 2, 9] = 1
+    with np.errstate(invalid="ignore"):
+        s = (q.astype(np.float64) @ np.swapaxes(k, 2, 3).astype(np.float64)) / np.sqrt(D)
+        if masked:
+            s = s + mask.astype(np.float64)
+        p = np.exp(s - s.max(-1, keepdims=True))
+        p /= p.sum(-1, keepdims=True)
+        want = p @ v.astype(np.float64)
+    got = T.AttentionScaled(q, k, v, mask, float(1 / np.sqrt(D)), ctx=ctx)
+    fin = np.isfinite(want)
+    assert fin[:, 1:].any() and not fin[:, 0].all()
+    assert np.array_equal(np.isfinite(got), fin)
+    assert np.array_equal(got[~fin], want[~fin].astype(np.float32), equal_nan=True)
+    assert np.abs(got[fin] - want[fin]).max() <= 4e-6 * np.abs(want[fin]).max()
