@@ -41,6 +41,7 @@
 // exp(scale*row - scale*max) with the flush, P.V, times 1/sum.
 
 #include <cstdlib>
+#include <type_traits>
 
 #include "fa_internal.h"
 #include "device_math.h"
@@ -378,18 +379,221 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const float* __r
   }
 }
 
+// ---- short sequences -----------------------------------------------------------
+// Up to 64 tokens: q/k norm, RoPE, the q|k|v product's second K part and the
+// attention in one launch. Such a forward is a chain of dependent launches, of
+// which a near-empty one takes 2 to 4 us: the norm pass and the combine go, and
+// the keys of a sequence are normed once per (32 queries, head) instead of once.
+// MI355X, a layer of one 19-token sequence: 3.2 + 9.6 -> 10.2 us in the kernel
+// trace, the 24-layer forward with host ids 979 -> 916 us (the rule's figures: model.cpp). Latency bound:
+// by count the fp32 MFMAs are 2 of the 10.2 us, the rest is start-up, dependent
+// loads and reductions. (One row's norm at a time in place of three: 10.7.)
+//
+// One workgroup of 16 waves per item. The waves norm and rotate the
+// sequence's keys and the item's queries into LDS (a row per wave, up to three
+// rows' loads in flight), the values on their way to registers meanwhile: wave
+// w multiplies dims 16 w .. 16 w + 15 of them. Scores: wave (query block,
+// 16-key tile, half of the dims) on v_mfma_f32_16x16x4_f32, the halves added in
+// order. All keys are there at once, so the softmax needs no running maximum:
+// wave w takes queries 2 w and 2 w + 1, 32 lanes each.
+constexpr int kShortKeys = kAttnShortKeys, kShortWaves = 16;
+
+struct ShortParams {
+  const float *qkv, *qkv2;
+  float* out;
+  const int32_t *items, *ext;
+  int32_t H, Hkv, window, norm_v;
+  float scale, split, eps;
+  int64_t row0;
+  const float *gq, *gk, *cs, *sn;
+};
+
+// Over the 32 lanes of a half wave, in every lane.
+template <class F>
+__device__ __forceinline__ float half_wave_f(float x, F f) {
+  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  auto rot = [&](auto c) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(c)::value, 0xF, 0xF, false));
+  };
+  x = f(x, rot(std::integral_constant<int, 0x128>{}));
+  x = f(x, rot(std::integral_constant<int, 0x124>{}));
+  x = f(x, rot(std::integral_constant<int, 0x122>{}));
+  x = f(x, rot(std::integral_constant<int, 0x121>{}));
+  return x;
+}
+
+template <bool TWO>  // the product has a second K part
+__global__ __launch_bounds__(64 * kShortWaves) void attention_short_kernel(ShortParams p) {
+  constexpr int HD = 256, LD = HD + 4, LS = kShortKeys + 4, NT = kShortKeys / 16;
+  __shared__ __attribute__((aligned(16))) float Kt[kShortKeys * LD], Qt[QBLK * LD];
+  __shared__ __attribute__((aligned(16))) float Sx[2][QBLK * LS];  // scores by half of the dims; then [0]: weights
+  __shared__ float vinv[kShortKeys], linv[QBLK];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, lq = lane & 15;
+  const int item = blockIdx.x;
+  const int q0 = p.items[3 * item + 1], h = p.items[3 * item + 2];
+  const int hk = h / (p.H / p.Hkv);
+  const int4 e = reinterpret_cast<const int4*>(p.ext)[item];
+  const int L = min(e.y, kShortKeys), nq = min(QBLK, L - q0), nkt = (L + 15) / 16;
+  const int64_t start = e.x - p.row0;
+  const int W = (p.H + 2 * p.Hkv) * HD;
+  const float* base = p.qkv + start * W;
+  const float* base2 = TWO ? p.qkv2 + start * W : base;
+  const int qcol = h * HD, kcol = (p.H + hk) * HD, vcol = (p.H + p.Hkv + hk) * HD;
+
+  // rows 0 .. L - 1: keys, then the queries, then (norm_v) the values' norms
+  const int rows = L + nq + (p.norm_v ? L : 0);
+  struct Row {
+    f32x4 x, x2, c, s;
+  };
+  const float *cs = p.cs, *sn = p.sn;
+  const float eps = p.eps;
+  auto load = [=](int r) {
+    const bool isv = r >= L + nq, isq = r >= L && !isv;
+    const int t = isv ? r - L - nq : isq ? q0 + r - L : r;
+    const int64_t off = (int64_t)t * W + kcol + (isq ? qcol - kcol : 0) + (isv ? vcol - kcol : 0) + 4 * lane;
+    const int64_t at = (int64_t)t * (HD / 2) + 4 * (lane & 31);
+    Row y;
+    y.x = *reinterpret_cast<const f32x4*>(base + off);
+    if constexpr (TWO) y.x2 = *reinterpret_cast<const f32x4*>(base2 + off);
+    y.c = *reinterpret_cast<const f32x4*>(cs + at);
+    y.s = *reinterpret_cast<const f32x4*>(sn + at);
+    return y;
+  };
+  const f32x4 gk = *reinterpret_cast<const f32x4*>(p.gk + 4 * lane);
+  const f32x4 gq = *reinterpret_cast<const f32x4*>(p.gq + 4 * lane);
+  // values: dim 16 wave + lq of keys 16 t + 4 g + i (past the last: the last,
+  // whose weight there is 0)
+  float v[NT][4], v2[NT][4];
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+    if (t < nkt) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int64_t off = (int64_t)min(16 * t + 4 * g + i, L - 1) * W + vcol + 16 * wave + lq;
+        v[t][i] = base[off];
+        if constexpr (TWO) v2[t][i] = base2[off];
+      }
+    }
+  const float flip = lane < 32 ? -1.f : 1.f;  // y_i = x_i c - x_{i+h} s, y_{i+h} = x_{i+h} c + x_i s
+  auto finish = [=](const Row& y, int r, float inv) {
+    if (r >= L + nq) {
+      if (lane == 0) vinv[r - L - nq] = inv;
+      return;
+    }
+    f32x4 n, o;
+#pragma unroll
+    for (int i = 0; i < 4; i++) n[i] = y.x[i] * inv * (r < L ? gk[i] : gq[i]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = n[i] * y.c[i] + lane_xor32(n[i]) * (flip * y.s[i]);
+    *reinterpret_cast<f32x4*>((r < L ? Kt + r * LD : Qt + (r - L) * LD) + 4 * lane) = o;
+  };
+  auto square = [](Row& y) {
+    if constexpr (TWO) y.x = y.x + y.x2;
+    const f32x4 xs[1] = {y.x};
+    return sumsq<1>(xs);
+  };
+  for (int r0 = wave; r0 < rows; r0 += 3 * kShortWaves) {
+    const int r1 = min(r0 + kShortWaves, rows - 1), r2 = min(r0 + 2 * kShortWaves, rows - 1);
+    Row y0 = load(r0), y1 = load(r1), y2 = load(r2);  // (rows past the last repeat it)
+    // the three rows' double-precision square roots and quotients at once, in
+    // different lanes
+    const float s0 = square(y0), s1 = square(y1), s2 = square(y2);
+    const int inv = __float_as_int(rms_inv(lane == 0 ? s0 : lane == 1 ? s1 : s2, HD, eps));
+    finish(y0, r0, __int_as_float(__builtin_amdgcn_readlane(inv, 0)));
+    if (r0 + kShortWaves < rows) finish(y1, r1, __int_as_float(__builtin_amdgcn_readlane(inv, 1)));
+    if (r0 + 2 * kShortWaves < rows) finish(y2, r2, __int_as_float(__builtin_amdgcn_readlane(inv, 2)));
+  }
+  if constexpr (TWO) {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+      if (t < nkt) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[t][i] += v2[t][i];
+      }
+  }
+  __syncthreads();
+  const int nqb = (nq + 15) / 16;
+  {
+    const int qb = wave & 1, kt = (wave >> 1) & 3, dp = wave >> 3;
+    if (qb < nqb && kt < nkt) {
+      // rows past the last repeat it (their scores are not used)
+      const float* qr = Qt + min(16 * qb + lq, nq - 1) * LD + dp * (HD / 2) + 4 * g;
+      const float* kr = Kt + min(16 * kt + lq, L - 1) * LD + dp * (HD / 2) + 4 * g;
+      f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int s = 0; s < HD / 32; s++) {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(qr + 16 * s), b = *reinterpret_cast<const f32x4*>(kr + 16 * s);
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[s & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], acc[s & 1], 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++) Sx[dp][(16 * qb + 4 * g + r) * LS + 16 * kt + lq] = acc[0][r] + acc[1][r];
+    }
+  }
+  __syncthreads();
+  {
+    const int q = 2 * wave + (lane >> 5), j = lane & 31, qi = q0 + q;
+    float t[2], m = kNegBig;
+    bool ok[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int key = j + 32 * i;
+      ok[i] = q < nq && key < L && (p.window <= 0 || (qi - key < p.window && key - qi < p.window));
+      t[i] = ok[i] ? (Sx[0][q * LS + key] + Sx[1][q * LS + key]) * p.scale : 0.f;
+      if (ok[i]) m = fmaxf(m, t[i]);
+    }
+    m = half_wave_f(m, [](float a, float b) { return fmaxf(a, b); });
+    float l = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int key = j + 32 * i;
+      const float w = ok[i] ? exp_flush(t[i] - m) : 0.f;
+      l += w;
+      // (a query's scores are read and its weights written by its own half wave)
+      Sx[0][q * LS + key] = w != 0.f && p.norm_v ? w * vinv[key] : w;
+    }
+    l = half_wave_f(l, [](float a, float b) { return a + b; });
+    if (j == 0) linv[q] = 1.f / l;
+  }
+  __syncthreads();
+  const int OW = p.H * HD;
+  for (int qb = 0; qb < nqb; qb++) {
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+      if (t < nkt) {
+        const f32x4 w = *reinterpret_cast<const f32x4*>(&Sx[0][(16 * qb + lq) * LS + 16 * t + 4 * g]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], v[t][i], o, 0, 0, 0);
+      }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int q = 16 * qb + 4 * g + r;
+      const float val = o[r] * linv[q];
+      float* orow = p.out + (start + q0 + q) * OW + h * HD;
+      if (p.split != 0.f) store_split1(orow, 16 * wave + lq, val * p.split, q < nq);
+      else if (q < nq) orow[16 * wave + lq] = val;
+    }
+  }
+}
+
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f16x8 as_f16x8(u32x4 v) { return __builtin_bit_cast(f16x8, v); }
 
-// ---- split-bf16 model-path kernel over key/value tile images (head_dim 256) -----
+// ---- split-fp16 model-path kernel over key/value tile images (head_dim 256) -----
 // attention_tiles_kernel computes attention_varlen_kernel<256>'s result on
-// the bf16 MFMA (v_mfma_f32_16x16x32_bf16) with fp32 accuracy: every fp32
-// operand is the exact sum of three bf16 terms (split3) and a product a.b
-// the sum of the six term products ai.bj with i + j <= 2 (the three dropped
-// ones are below 2^-24 relative), accumulated in fp32.
+// the fp16 MFMA (v_mfma_f32_16x16x32_f16) with fp32 accuracy: every fp32
+// operand, times a power of two from a bound on all of them, is held as two
+// fp16 terms, and a product a.b is hi.hi + hi.lo + lo.hi (lo.lo is below 2^-24
+// relative), accumulated in fp32. Its error against float64 is below that of
+// three exact bf16 terms and six products (8 x 1 024..2 048 tokens, two layers:
+// 1.0e-6 -> 7.3e-7): half the MFMAs also means half the fp32 roundings.
 //
 // Rows. The query rows of kv head hk are the pairs (token t, query head
 // hk*G + g) of the G = H/Hkv heads that share it, numbered r = t*G + g. A
@@ -404,38 +608,37 @@ __device__ __forceinline__ f16x8 as_f16x8(u32x4 v) { return __builtin_bit_cast(f
 // kv_tiles_kernel: per (tile of 32 keys of one sequence, kv head) a key
 // image [term][key][256] whose 16-byte chunk c of key k sits at c ^ k, and
 // a value image [term][dim][32 slots] whose slot 8g + 4h + r holds key 16h +
-// 4g + r (chunk g of dim d at position g ^ ((d >> 1) & 3)); 48 KB each,
+// 4g + r (chunk g of dim d at position g ^ ((d >> 1) & 3)); 32 KB each,
 // copied to LDS unchanged by direct global->LDS loads (1 KB per wave
-// instruction). One key buffer and two value buffers: 144 KB (160 KB with
+// instruction). Two key buffers and two value buffers: 128 KB (144 KB with
 // the wave pairs' partial-score exchange), one workgroup per CU (two waves
 // per SIMD with eight waves, one with four).
 //
 // Formulation (lane l: lq = l % 16, g = l / 16). The q terms stay in
-// registers: lane l holds row lq's dims 32c + 8g .. +7 (c = 0..7), three
-// terms, 96 VGPRs.
+// registers: lane l holds row lq's dims 32c + 8g .. +7 (c = 0..7), two
+// terms, 64 VGPRs.
 //   S^T[key, row] = K . Q^T per block of 16 keys: A = a key term (lane l:
-//   key lq, dims 32c + 8g ..), B = a q term; 8 chunks x 6 term pairs per
+//   key lq, dims 32c + 8g ..), B = a q term; 8 chunks x 3 term pairs per
 //   block. Lane l ends with row lq's scores against keys 4g + r and 16 + 4g
 //   + r: the row's softmax is lane-local plus two exchanges (xor 16, 32).
-//   O^T[dim, row] += V^T . P^T, one 32-key step per block of 16 dims x 6
+//   O^T[dim, row] += V^T . P^T, one 32-key step per block of 16 dims x 3
 //   pairs: the lane's own eight probabilities are B (slot 8g + e: key 4g + e
 //   for e < 4, 16 + 4g + e - 4 after), A one 16-byte value-image read per
 //   term (dim 16db + lq, slots 8g ..). Row lq's O sits in the lanes with
 //   that lq (dims 16db + 4g + r), so the rescale and the final 1/sum are
 //   lane-local.
 // Lazy maximum: a row's exponent offset m moves only when a tile's maximum
-// exceeds it by more than 8 (O and the sum are then scaled by e^(m_old -
-// m_new)), so weights stay below e^8 and O is rarely touched outside the
+// exceeds it by more than 4 (O and the sum are then scaled by e^(m_old -
+// m_new)), so weights stay below e^4 and O is rarely touched outside the
 // MFMAs. A weight is 0 when its exponent t - m is below -87 (the reference
 // flushes against the row's final maximum; the two differ only in weights
 // below e^-87 of the row's largest).
 //
 // Per tile tt (software pipeline, detailed at the loop): barrier (keys of
 // tt and values of tt-1 landed; every wave done with iteration tt-1), load
-// the values of tt, scores of tt, barrier (every wave done reading the
-// keys), load the keys of tt+1 (past the last tile: the last again, so no
-// load is conditional), then P.V of tile tt-1 with tile tt's softmax spread
-// among its blocks.
+// the values of tt and the keys of tt+1 (past the last tile: the last again,
+// so no load is conditional), scores of tt, then P.V of tile tt-1 with tile
+// tt's softmax spread among its blocks.
 constexpr int TL_KEYS = 32;              // keys per tile
 constexpr int TL_IMG = 2 * 32 * 256;     // fp16 per key or value image
 constexpr float TL_TAU = 4.f;            // lazy-maximum slack
@@ -1276,6 +1479,23 @@ int launch_attention_varlen_items(fa_ctx* ctx, const AttnVarlenArgs& a, const in
       hipLaunchKernelGGL(attention_combine_kernel<512>, g2, b2, 0, s, a.part, a.kparts, a.rows, (int64_t)0, a.rows,
                          a.H, a.out, a.split != 0.f ? a.split : 1.f, a.split != 0.f ? 1 : 0);
   }
+  FA_CHECK_LAUNCH(ctx);
+  return FA_OK;
+}
+
+int launch_attention_short(fa_ctx* ctx, const AttnShortArgs& a, const int32_t* d_items, int32_t n_items,
+                           hipStream_t s) {
+  if (a.Hkv <= 0 || a.H % a.Hkv != 0)
+    return set_error(ctx, FA_ERR_ARG, "attention: %d query heads not a multiple of %d kv heads", a.H, a.Hkv);
+  if (!a.item_ext) return set_error(ctx, FA_ERR_ARG, "attention: no item extents");
+  if (n_items == 0) return FA_OK;
+  ShortParams p;
+  p.qkv = a.qkv; p.qkv2 = a.qkv2; p.out = a.out; p.items = d_items; p.ext = a.item_ext;
+  p.H = a.H; p.Hkv = a.Hkv; p.window = a.window; p.norm_v = a.norm_v ? 1 : 0;
+  p.scale = a.scale; p.split = a.split; p.eps = a.eps; p.row0 = a.row0;
+  p.gq = a.gq; p.gk = a.gk; p.cs = a.cos_t; p.sn = a.sin_t;
+  if (a.qkv2) hipLaunchKernelGGL(attention_short_kernel<true>, dim3((unsigned)n_items), dim3(64 * kShortWaves), 0, s, p);
+  else hipLaunchKernelGGL(attention_short_kernel<false>, dim3((unsigned)n_items), dim3(64 * kShortWaves), 0, s, p);
   FA_CHECK_LAUNCH(ctx);
   return FA_OK;
 }

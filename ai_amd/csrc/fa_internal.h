@@ -347,6 +347,23 @@ inline int64_t attention_part_floats(int kparts, int64_t rows, int H, int D) {
 // its n_items extents.
 int launch_attention_varlen_items(fa_ctx* ctx, const AttnVarlenArgs& a, const int32_t* d_items, int32_t n_items,
                                   hipStream_t s);
+// Attention of sequences of at most kAttnShortKeys tokens at head_dim 256
+// straight from the q|k|v product (qkv + qkv2, the latter null if the product
+// was not split): q/k norm (norm_v: the values' too) and RoPE included. The
+// same items as launch_attention_varlen_items.
+struct AttnShortArgs {
+  const float *qkv, *qkv2;
+  float* out;
+  int32_t H, Hkv, window;
+  float scale, split, eps;
+  int64_t row0;
+  const int32_t* item_ext;
+  const float *gq, *gk, *cos_t, *sin_t;
+  bool norm_v;
+};
+constexpr int kAttnShortKeys = 64;
+int launch_attention_short(fa_ctx* ctx, const AttnShortArgs& a, const int32_t* d_items, int32_t n_items,
+                           hipStream_t s);
 // Queries per workgroup of the varlen kernel (the item granularity).
 int attention_varlen_qblock();
 // head_dim 256, split-fp16 attention over key/value tile images: writes,

@@ -381,6 +381,16 @@ int attention_key_parts_forced() {
   return v;
 }
 
+// FA_ATTN_SHORT=0: the q/k norm pass and the fp32 attention for short
+// sequences too; also with forced key runs.
+bool attention_short_enabled() {
+  static const bool on = [] {
+    const char* e = std::getenv("FA_ATTN_SHORT");
+    return !(e && e[0] == '0');
+  }();
+  return on && attention_key_parts_forced() == 0;
+}
+
 // FA_ATTN_ROWS=64|128 forces the tile attention's rows per item (tuning);
 // 0 when unset.
 int attention_rows_forced() {
@@ -1208,6 +1218,17 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
       return rc;
     pr.done();
   }
+  // The fp32 path's layers of head_dim 256 take their q/k norm into the
+  // attention (FA_ATTN_SHORT=0 and forced key runs: the separate passes) where
+  // every sequence is short and the items are one round of workgroups. A few
+  // sequences above 32 tokens stay with the separate passes, whose key runs
+  // spread them over more CUs. Us per forward, separate and fused: 1 x 16 907
+  // and 844, 1 x 32 1 026 and 1 004, 1 x 48 1 014 and 1 057, 1 x 64 1 031 and
+  // 1 101, 4 x 64 (24 items) 1 346 and 1 362, 8 x 64 (48) 1 582 and 1 558, 16 x
+  // 64 1 827 and 1 758, 85 x 12 1 716 and 1 642, 80 x 32 (240) 2 533 and 2 526.
+  const int32_t longest = *std::max_element(lengths, lengths + B);
+  const bool short_seqs = fa::attention_short_enabled() && ap.n_items_v <= cus &&
+                          (longest <= 32 || (longest <= fa::kAttnShortKeys && ap.n_items_v >= 48));
   // one layer over rows [r0, r0 + rows) (the sequences of one group, whose
   // attention items are items_t[0, n_it_t) for a tile layer, items_v[0,
   // n_it_v) otherwise) on stream st
@@ -1218,6 +1239,7 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
     const int D = L.D, Hkv = L.Hkv;
     const bool sliding = L.sliding;
     const bool tiles = ap.layer_tiles(D);
+    const bool shrt = !tiles && D == 256 && short_seqs;
     // The N = hidden products (o, down, per-layer-input projection) split K
     // in two when their 128x128 tiles, counted over the concurrent groups,
     // give the CUs fewer than two each (C2: one stream 5 517 rows, or three
@@ -1277,7 +1299,7 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
                                     (int32_t)ntl, img, st, v2, L.s_k, L.s_att)))
         return rc;
       pr.done();
-    } else {
+    } else if (!shrt) {
       fa::Probe pr(m, FA_K_QKNORM_ROPE, 0, (double)rows * (H + (v2 ? 2 : 1) * Hkv) * D * 8.0);
       // a group of one sequence: row i is token i, no position table
       const int32_t* gpos = b1 - b0 == 1 ? nullptr : pos_d + r0;
@@ -1321,6 +1343,12 @@ int forward(fa_model* m, const int32_t* d_ids, const int32_t* lengths, int32_t B
           at.kparts = kparts_t; at.rows = M; at.nrows = rows; at.part = attn_part;
         }
         if ((rc = fa::launch_attention_tiles(ctx, at, items_t, (int32_t)n_it_t, st))) return rc;
+      } else if (shrt) {
+        fa::AttnShortArgs as;
+        as.qkv = qkvr; as.qkv2 = qkv2; as.out = attr; as.H = H; as.Hkv = Hkv; as.window = a.window; as.scale = a.scale;
+        as.split = a.split; as.eps = eps; as.row0 = r0; as.item_ext = a.item_ext;
+        as.gq = L.g_q; as.gk = L.g_k; as.cos_t = L.cos_t; as.sin_t = L.sin_t; as.norm_v = v2;
+        if ((rc = fa::launch_attention_short(ctx, as, items_v, (int32_t)n_it_v, st))) return rc;
       } else {
         if ((rc = fa::launch_attention_varlen_items(ctx, a, items_v, (int32_t)n_it_v, st))) return rc;
       }

@@ -46,6 +46,7 @@
  *   FA_MICROBATCH=0|<rows>      micro-batches off / from this many tokens (2048)
  *   FA_MICROBATCH_GROUPS=2..4   force the micro-batch count
  *   FA_ATTN_KEY_PARTS=1..8      force the key runs of the short-batch attention
+ *   FA_ATTN_SHORT=0             q/k norm and attention of short sequences (up to 64 tokens) in two passes
  *   FA_ATTN_ROWS=64|128         force the tile attention's rows per work item
  *   FA_ATTN_PAIRS=0             64-row tile items on four single waves instead of
  *                               eight waves in head-dimension pairs

@@ -525,6 +525,36 @@ def test_tile_attention_other_head_groupings(ctx, heads):
         om.close()
 
 
+@pytest.mark.parametrize("heads,window,lengths", [
+    ((3, 1), 512, [16]), ((3, 1), 512, [17]), ((3, 1), 512, [64]), ((3, 1), 16, [64, 63, 33, 1, 48] * 2), ((4, 2), 16, [32, 31, 2]),
+    ((3, 1), 512, [64] * 20), ((6, 1), 512, [49, 65]), ((3, 1), 512, [7] * 90)])
+def test_short_sequence_attention(ctx, heads, window, lengths):
+    """Sequences of up to 64 tokens take q/k norm, RoPE and attention in one
+    launch: around its 16-key tiles and 32-query items, with a window inside
+    the sequence (16: |i - j| < 9), other head groupings, on one stream with
+    q|k|v in two K parts and (1 280 tokens) over micro-batch streams; 65
+    tokens, 270 items and a lone 64-token sequence keep the separate passes. Every row and the states
+    against the oracle, with the bars of the encoder's other paths."""
+    H, Hkv = heads
+    shape = _shape_variant(num_attention_heads=H, num_key_value_heads=Hkv, num_hidden_layers=4,
+                           sliding_window_pattern=2, sliding_window=window)
+    lens = np.array(lengths, np.int32)
+    rng = np.random.default_rng(H * 100 + sum(lengths))
+    ids = rng.integers(3, shape.vocab_size, (len(lens), int(lens.max()))).astype(np.int32)
+    ids[:, 0] = 2
+    ids[np.arange(ids.shape[1])[None, :] >= lens[:, None]] = 0
+    gm = G.Model(shape, ctx)
+    gm.load_synthetic()
+    om = O.OracleModel(shape)
+    om.load_synthetic()
+    try:
+        compare(gm.embed_ids(ids, lens), oracle_embed(om, ids, lens), f"short {heads} {lengths[:5]}")
+        compare_states(gm, om, ids, lens, sorted({0, len(lens) - 1}), f"short {heads} states", layers=[1, 4, -1])
+    finally:
+        gm.close()
+        om.close()
+
+
 def _topk_checked(s64, gi, oi, bound, what):
     """Identity of top-k lists wherever the float64 scores s64's k+1 best are
     separated by more than 2*bound per row (bound: how far either side's
