@@ -20,9 +20,9 @@ Prints ONE JSON line (the driver's contract) with:
   roofline         the dominant kernel (the gate|up GEMM with the GeGLU
                    epilogue) timed with HIP events on the library's stream:
                    algorithmic flops (2*M*N*K) / mean launch duration vs the
-                   2.5 PFLOP/s dense bf16 MFMA peak, the unit the split-bf16
-                   GEMM runs on (three bf16 products per fp32 multiply-add,
-                   so its ceiling is a third of that peak)
+                   2.5 PFLOP/s dense 16-bit MFMA peak, the unit the split-fp16
+                   GEMM runs on (two fp16 products per fp32 multiply-add,
+                   so its ceiling is half of that peak)
   throughput_roofline
                    the timed throughput as a roofline fraction: the forward's
                    algorithmic flops (all GEMMs + attention) per timed step /
@@ -46,7 +46,7 @@ sys.path.insert(0, ROOT)
 
 FP32_MFMA_PEAK = 157.3e12  # MI355X dense fp32 matrix, FLOP/s
 BF16_MFMA_PEAK = 2.5e15    # MI355X dense bf16 matrix, FLOP/s
-SPLIT_TERMS = 3            # bf16 products per fp32 multiply-add in the split-bf16 GEMM
+SPLIT_TERMS = 2            # fp16 products per fp32 multiply-add in the split-fp16 GEMM
 HBM_PEAK = 8.0e12          # MI355X HBM3E, B/s
 
 METRIC = "sentences/sec @ batch32×seq256 on 1 MI355X; GEMM % of fp32 MFMA peak"
@@ -56,7 +56,7 @@ METRIC = "sentences/sec @ batch32×seq256 on 1 MI355X; GEMM % of fp32 MFMA peak"
 # 1 GiB copy kernel reads on the same counters (profiles/
 # gemm_gateup_c2_hbm_traffic.md). Re-measured whenever the kernel changes;
 # applies to the C2 workload only.
-GATEUP_TRAFFIC_C2 = {"bytes": (2 * 30326 + 29578) * 1024, "kernel_rev": "x3-128x256w8-chunkmajor-lds"}
+GATEUP_TRAFFIC_C2 = {"bytes": (2 * 23605 + 24826) * 1024, "kernel_rev": "h2-128x256"}
 
 
 def parse():
@@ -254,7 +254,7 @@ def main():
 
     gs, g_ms, g_flops, _ = kstat("gemm_gateup")
     achieved = g_flops / (g_ms * 1e-3) if g_ms > 0 else 0.0
-    roofline = {"kernel": "gemm_x3_kernel split-bf16, GeGLU epilogue (gate|up, M=%d N=%d K=%d)"
+    roofline = {"kernel": "gemm_h2_kernel split-fp16, GeGLU epilogue (gate|up, M=%d N=%d K=%d)"
                           % (batch.tokens, 2 * shape.intermediate_size, shape.hidden_size),
                 "bound": "mfma", "achieved": round(achieved / 1e12, 2), "peak": BF16_MFMA_PEAK / 1e12,
                 "unit": "TFLOP/s", "frac": round(achieved / BF16_MFMA_PEAK, 4),
