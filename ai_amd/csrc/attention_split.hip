@@ -2,8 +2,8 @@
 // MFMA with fp32 accuracy, for any operands: attention_dense_kernel
 // (attention.hip) runs the same products on the fp32 MFMA, a sixteenth of
 // that rate, and stays for small calls and head_dim 512. 8 x 8 heads x 512 x 512,
-// head_dim 64: 62 -> 40 us per call (8 of them the image pass); 32 x 3 x 256 x 256
-// on one kv head, head_dim 256, padded: 102 -> 65. What bounds it now: the
+// head_dim 64: 55 -> 35 us per call (8 of them the image pass); 32 x 3 x 256 x 256
+// on one kv head, head_dim 256, padded: 95 -> 62. What bounds it now: the
 // softmax's VALU work at head_dim 64, the operand reads from LDS (2.4 of 2.9 us
 // per 32 keys) and the prologue at 256.
 //
@@ -516,6 +516,9 @@ bool attention_split_ok(const AttnGenericArgs& a) {
   if (off || !attention_dense_ok(a) || (a.D != 64 && a.D != 128 && a.D != 256)) return false;
   if (!(a.scale > 0.f) || a.S < 192 || 4.0 * a.B * a.H * (double)a.T * a.S * a.D < (a.D == 256 ? 5e8 : 1e8)) return false;
   const SplitSizes z = split_sizes(a);
+  // images of at most 8 GiB: keys broadcast over a batch are written once per
+  // entry, and the context keeps the buffer
+  if (z.k_bytes + z.v_bytes > (8ULL << 30)) return false;
   return z.blocks < INT32_MAX && (int64_t)a.B * a.H * ((a.T + 63) / 64) < INT32_MAX;
 }
 

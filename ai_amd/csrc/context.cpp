@@ -475,7 +475,12 @@ int attention_check(fa_ctx* ctx, int32_t B, int32_t H, int32_t T, int32_t S, int
 
 int attention_launch(fa_ctx* ctx, const fa::AttnGenericArgs& a) {
   // the MFMA kernel for the head dims it covers, the per-row kernel otherwise
-  if (fa::attention_split_ok(a)) return fa::launch_attention_split(ctx, a, ctx->stream);
+  if (fa::attention_split_ok(a)) {
+    // (its images need memory that the others do without)
+    const int rc = fa::launch_attention_split(ctx, a, ctx->stream);
+    if (rc != FA_ERR_OOM) return rc;
+    (void)hipGetLastError();
+  }
   if (fa::attention_dense_ok(a)) return fa::launch_attention_dense(ctx, a, ctx->stream);
   return fa::launch_attention_generic(ctx, a, ctx->stream);
 }

@@ -440,6 +440,32 @@ def test_attention_split_edges(ctx, D, B, H, Hkv, Tq, Sk, kind):
     assert np.abs(got - want).max() <= 4e-6 * np.abs(want).max()
 
 
+def test_attention_broadcast_batch_beyond_the_images(ctx):
+    """Keys broadcast over a batch whose images would take 343 GB run on the
+    fp32 kernel as before: every entry equals the one-entry call (on the 16-bit
+    path, the same bound as test_attention_split_edges)."""
+    B, H, S, D = 512, 8, 131072, 64
+    r = rng(14)
+    q = np.tile(r.standard_normal((1, H, 1, D)).astype(np.float32), (B, 1, 1, 1))
+    k, v = (r.standard_normal((H, S, D)).astype(np.float32) for _ in range(2))
+    L = N.lib()
+    ptrs = []
+    for a in (q, k, v, np.empty_like(q)):
+        p = C.c_void_p()
+        N.check(ctx.h, L.fa_device_alloc(ctx.h, a.nbytes, C.byref(p)))
+        N.check(ctx.h, L.fa_memcpy_h2d(ctx.h, p, a.ctypes.data, a.nbytes))
+        ptrs.append(p)
+    got = {}
+    for n in (1, B):
+        N.check(ctx.h, L.fa_attention_dev(ctx.h, ptrs[0], ptrs[1], ptrs[2], n, H, 1, S, D, H * D, D, 0, S * D, 0, S * D,
+                                          None, 0, 0, 0, 0, 0.125, ptrs[3]))
+        got[n] = np.empty((n, H, 1, D), np.float32)
+        N.check(ctx.h, L.fa_memcpy_d2h(ctx.h, got[n].ctypes.data, ptrs[3], got[n].nbytes))
+    for p in ptrs:
+        L.fa_device_free(ctx.h, p)
+    assert np.abs(got[B] - got[1]).max() <= 4e-6 * np.abs(v).max()
+
+
 @pytest.mark.parametrize("D,B,H,Tq,Sk,masked", [(64, 1, 8, 129, 449, False), (128, 2, 4, 150, 225, True),
                                                (256, 2, 3, 257, 479, True)])
 def test_attention_split_infinities(ctx, D, B, H, Tq, Sk, masked):
