@@ -7,19 +7,17 @@
 // softmax's VALU work at head_dim 64, the operand reads from LDS (2.4 of 2.9 us
 // per 32 keys) and the prologue at 256.
 //
-// Scores: q and k as two fp16 terms each, hi = fp16(x s) and lo = fp16((x s -
-// hi) 2^11) with one power of two s per row (query or key) that brings the
-// row's largest value to [2^14, 2^15): 23 bits down to 2^-27 of the row's
-// largest value. Three MFMAs per pair, hi.hi, hi.lo and lo.hi (one factor of
-// each product with a lo carries 2^-11), and each score times its row's and
-// its key's power of two. Values and probabilities: three exact bf16 terms
-// each (split3), six MFMAs per pair. bf16 has float32's range, so a masked
-// key may hold any finite value without touching its neighbours.
+// Queries, keys, values and probabilities are three exact bf16 terms each
+// (split3), a product the six MFMAs whose terms' orders add up to at most two
+// (what is dropped, mid . lo and lo . lo, is below 2^-21 of the product of the two values). bf16 has
+// float32's range, so elements of one row may be of any magnitude beside each
+// other, and a masked key may hold any finite value without touching its
+// neighbours. (Two fp16 terms for the scores, scaled by a power of two per
+// row, took three MFMAs but lost the small elements of a row beside a large one.)
 //
 // split_kv_kernel writes, per (batch, kv head, tile of 32 keys), a key image
-// [term][key][HD], a value image [term][dim][32 slots] and the keys' powers
-// of two, in the order in which the attention's direct global->LDS loads and
-// operand reads take them: 16-byte chunk c of key k at c ^ (k mod 16) (head_dim
+// [term][key][HD] and a value image [term][dim][32 slots], in the order in
+// which the attention's direct global->LDS loads and operand reads take them: 16-byte chunk c of key k at c ^ (k mod 16) (head_dim
 // 64: c ^ (k / 2 mod 8)), slot 8g + 4h + r of a dim holding key 16h + 4g + r,
 // chunk g of dim d at g ^ (d / 2 mod 4), both free of bank conflicts (d / 4 mod 4
 // had a third of the value reads in conflict). Heads that share one key/value
@@ -30,8 +28,9 @@
 // scores in the four lanes that share l % 16, and its probabilities are then
 // the B operand of O^T += V^T . P^T as they are. Per stage of SK keys (64 at
 // head_dim 64): [barrier: this stage's keys and the previous stage's values
-// landed] load this stage's values and the next keys (head_dim 256 has room for
-// one key buffer: they load after a second barrier); scores; P.V of the previous
+// landed] load this stage's values and the next keys (with one key buffer they
+// load after a second barrier: head_dim 256 has room for no more, and four-wave
+// workgroups of the others fit a CU twice with one); scores; P.V of the previous
 // stage; softmax. P.V one stage behind leaves the values a whole stage to land
 // (2 048 queries and keys, 3 heads
 // of 256: 211 -> 192 us per call). The row maximum is lazy: the
@@ -44,7 +43,6 @@
 namespace fa {
 namespace {
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -56,21 +54,22 @@ __device__ __forceinline__ int key_chunk(int key, int c) {
 }
 __device__ __forceinline__ int slot_chunk(int dim, int g) { return g ^ ((dim >> 1) & 3); }
 
-// The power of two that brings m (>= 0) to [2^14, 2^15), and its inverse; 1
-// for 0, infinities and NaN (whose scores come out as NaN: plain_query).
-__device__ __forceinline__ void row_pow2(float m, float& s, float& inv) {
-  const int e = (int)((__float_as_uint(m) >> 23) & 0xFF) - 127;  // exponent; 128: not finite
-  const int sh = m == 0.f || e == 128 ? 0 : 14 - max(e, -100);
-  s = ldexpf(1.f, min(sh, 120));
-  inv = ldexpf(1.f, -min(sh, 120));
-}
-
-__device__ __forceinline__ void split_row8(const float (&x)[8], float s, f16x8& hi, f16x8& lo) {
+// Eight values as three bf16 terms, each packed as the 16 bytes it takes in an
+// image or an operand.
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&t)[3]) {
+  uint32_t h[8], m[8], l[8];
 #pragma unroll
   for (int e = 0; e < 8; e++) {
-    const uint32_t w = split2(x[e] * s);
-    hi[e] = __builtin_bit_cast(_Float16, (uint16_t)(w & 0xFFFFu));
-    lo[e] = __builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
+    const Split3 sp = split3(x[e]);
+    h[e] = sp.h;
+    m[e] = sp.m;
+    l[e] = sp.l;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    t[0][i] = pack_hi16(h[2 * i], h[2 * i + 1]);
+    t[1][i] = pack_hi16(m[2 * i], m[2 * i + 1]);
+    t[2][i] = pack_hi16(l[2 * i], l[2 * i + 1]);
   }
 }
 
@@ -79,7 +78,6 @@ struct SplitKvParams {
   int64_t k_sb, k_sh, v_sb, v_sh;
   int Hk, S, tiles;  // kv heads with images of their own; tiles per (batch, kv head)
   uint16_t *kimg, *vimg;
-  float* kinv;
 };
 
 template <int HD>
@@ -92,7 +90,7 @@ __global__ __launch_bounds__(256) void split_kv_kernel(SplitKvParams p) {
   const int b = (int)(bh / p.Hk), h = (int)(bh - (int64_t)b * p.Hk);
   const float* kb = p.k + b * p.k_sb + h * p.k_sh;
   const float* vb = p.v + b * p.v_sb + h * p.v_sh;
-  uint16_t* ko = p.kimg + at * (2 * 32 * HD);
+  uint16_t* ko = p.kimg + at * (3 * 32 * HD);
   uint16_t* vo = p.vimg + at * (3 * 32 * HD);
   constexpr int CH = HD / 8;          // chunks (threads) per key
   constexpr int KPP = 256 / CH;       // keys per pass
@@ -115,24 +113,11 @@ __global__ __launch_bounds__(256) void split_kv_kernel(SplitKvParams p) {
 #pragma unroll
   for (int i = 0; i < 32 / KPP; i++) {
     const int key = threadIdx.x / CH + i * KPP;
-    float m = 0.f;
-    bool fin = true;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      m = fmaxf(m, fabsf(x[i][e]));
-      fin = fin && x[i][e] == x[i][e];
-    }
-    if (!fin) m = INFINITY;
-#pragma unroll
-    for (int o = CH / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-    float s, inv;
-    row_pow2(m, s, inv);
-    f16x8 hi, lo;
-    split_row8(x[i], s, hi, lo);
+    u32x4 t[3];
+    split8(x[i], t);
     uint16_t* o16 = ko + key * HD + key_chunk<HD>(key, c) * 8;
-    *reinterpret_cast<f16x8*>(o16) = hi;
-    *reinterpret_cast<f16x8*>(o16 + 32 * HD) = lo;
-    if (c == 0) p.kinv[at * 32 + key] = inv;
+#pragma unroll
+    for (int j = 0; j < 3; j++) *reinterpret_cast<u32x4*>(o16 + j * 32 * HD) = t[j];
 #pragma unroll
     for (int e = 0; e < 8; e += 4)
       *reinterpret_cast<f32x4*>(&Vt[key * VST + 8 * c + e]) = f32x4{y[i][e], y[i][e + 1], y[i][e + 2], y[i][e + 3]};
@@ -141,28 +126,20 @@ __global__ __launch_bounds__(256) void split_kv_kernel(SplitKvParams p) {
 #pragma unroll
   for (int i = 0; i < HD * 4 / 256; i++) {
     const int u = threadIdx.x + 256 * i, d = u >> 2, g = u & 3;
-    uint32_t th[8], tm[8], tl[8];
+    float x8[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const Split3 sp = split3(Vt[((e >> 2) * 16 + 4 * g + (e & 3)) * VST + d]);
-      th[e] = sp.h;
-      tm[e] = sp.m;
-      tl[e] = sp.l;
-    }
+    for (int e = 0; e < 8; e++) x8[e] = Vt[((e >> 2) * 16 + 4 * g + (e & 3)) * VST + d];
+    u32x4 t[3];
+    split8(x8, t);
     uint16_t* o = vo + d * 32 + slot_chunk(d, g) * 8;
-    *reinterpret_cast<uint4*>(o) =
-        make_uint4(pack_hi16(th[0], th[1]), pack_hi16(th[2], th[3]), pack_hi16(th[4], th[5]), pack_hi16(th[6], th[7]));
-    *reinterpret_cast<uint4*>(o + 32 * HD) =
-        make_uint4(pack_hi16(tm[0], tm[1]), pack_hi16(tm[2], tm[3]), pack_hi16(tm[4], tm[5]), pack_hi16(tm[6], tm[7]));
-    *reinterpret_cast<uint4*>(o + 64 * HD) =
-        make_uint4(pack_hi16(tl[0], tl[1]), pack_hi16(tl[2], tl[3]), pack_hi16(tl[4], tl[5]), pack_hi16(tl[6], tl[7]));
+#pragma unroll
+    for (int j = 0; j < 3; j++) *reinterpret_cast<u32x4*>(o + j * 32 * HD) = t[j];
   }
 }
 
 struct SplitParams {
   const float *q, *k, *v, *mask;
   const uint16_t *kimg, *vimg;
-  const float* kinv;
   float* out;
   int H, Hk, T, S, tiles, qblocks;
   int64_t q_sb, q_sh, k_sb, k_sh, v_sb, v_sh, m_sb, m_sh, m_sr, m_sc;
@@ -170,10 +147,9 @@ struct SplitParams {
 };
 
 // One query in plain fp32, by one wave, lane l holding dims l, l + 64, ...:
-// for queries whose split result is not finite. An infinity has no finite
-// second term, and factors of rows of extreme magnitude can overflow where
-// their product does not, so the split gives NaN where the operands
-// themselves give an infinity, or a weight of 0.
+// for queries whose split result is not finite: an infinity has no finite
+// second term, so the split gives NaN where the operands themselves give an
+// infinity, or a weight of 0.
 template <int HD, bool MASK>
 __device__ void plain_query(const SplitParams& p, int b, int h, int qi, int lane) {
   constexpr int N = HD / 64;
@@ -233,71 +209,51 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
   constexpr int SK = HD == 64 ? 64 : 32;  // keys per stage
   constexpr int NT = SK / 32;             // tiles per stage
   constexpr int NC = HD / 32, NDB = HD / 16;
-  constexpr int KI = 2 * 32 * HD, VI = 3 * 32 * HD;  // 16-bit values of a tile's images
-  static_assert(NT * KI % (64 * W * 8) == 0 && NT * VI % (64 * W * 8) == 0, "whole loads");
-  constexpr bool KD = HD < 256;  // two key buffers
-  __shared__ __attribute__((aligned(16))) uint16_t K0[NT * KI], K1[KD ? NT * KI : 8], V0[NT * VI], V1[NT * VI];
+  constexpr int IMG = 3 * 32 * HD;        // 16-bit values of a tile's key or value image
+  static_assert(NT * IMG % (64 * W * 8) == 0, "whole loads");
+  constexpr bool KD = HD < 256 && W == 8;  // two key buffers (72 KB with one, 96 with two)
+  __shared__ __attribute__((aligned(16))) uint16_t K0[NT * IMG], K1[KD ? NT * IMG : 8], V0[NT * IMG], V1[NT * IMG];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lq = lane & 15, g = lane >> 4;
   const int bh = blockIdx.x / p.qblocks, qblk = blockIdx.x % p.qblocks;
   const int b = bh / p.H, h = bh % p.H;
   const int64_t img = ((int64_t)b * p.Hk + (p.Hk == 1 ? 0 : h)) * p.tiles;
-  const uint16_t* kimg = p.kimg + img * KI;
-  const uint16_t* vimg = p.vimg + img * VI;
-  const float* kinv = p.kinv + img * 32;
+  const uint16_t* kimg = p.kimg + img * IMG;
+  const uint16_t* vimg = p.vimg + img * IMG;
   const int stages = (p.S + SK - 1) / SK;
 
-  auto load_k = [&](uint16_t* dst, int st) {
+  auto load = [&](const uint16_t* src, uint16_t* dst, int st) {
 #pragma unroll
-    for (int i = 0; i < NT * KI / 8 / 64 / W; i++)
-      __builtin_amdgcn_global_load_lds(kimg + (int64_t)st * NT * KI + ((i * W + wave) * 64 + lane) * 8,
+    for (int i = 0; i < NT * IMG / 8 / 64 / W; i++)
+      __builtin_amdgcn_global_load_lds(src + (int64_t)st * NT * IMG + ((i * W + wave) * 64 + lane) * 8,
                                        (__attribute__((address_space(3))) void*)(dst + (i * W + wave) * 512), 16, 0, 0);
   };
-  auto load_v = [&](uint16_t* dst, int st) {
-#pragma unroll
-    for (int i = 0; i < NT * VI / 8 / 64 / W; i++)
-      __builtin_amdgcn_global_load_lds(vimg + (int64_t)st * NT * VI + ((i * W + wave) * 64 + lane) * 8,
-                                       (__attribute__((address_space(3))) void*)(dst + (i * W + wave) * 512), 16, 0, 0);
-  };
-  load_k(K0, 0);
+  load(kimg, K0, 0);
 
-  // the wave's queries: their terms in registers (qh2 = qh 2^-11, the factor
-  // of the keys' lo terms)
+  // the wave's queries: their terms in registers
   const int qi = (qblk * W + wave) * 16 + lq;
   const bool qvalid = qi < p.T;
   const int qc = min(qi, p.T - 1);
-  f16x8 qh[NC], qh2[NC], ql[NC];
-  float qinv;
+  bf16x8 qt[NC][3];
   {
     const float* qr = p.q + b * p.q_sb + h * p.q_sh + (int64_t)qc * HD + 8 * g;
-    float x[NC][8];
-    float m = 0.f;
-    bool fin = true;
 #pragma unroll
-    for (int c = 0; c < NC; c++)
+    for (int c = 0; c < NC; c++) {
+      float x[8];
 #pragma unroll
       for (int e = 0; e < 8; e += 4) {
         const f32x4 a = *reinterpret_cast<const f32x4*>(qr + 32 * c + e);
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-          x[c][e + u] = a[u];
-          m = fmaxf(m, fabsf(a[u]));
-          fin = fin && a[u] == a[u];
-        }
+        for (int u = 0; u < 4; u++) x[e + u] = a[u];
       }
-    if (!fin) m = INFINITY;
-    m = lanes4_max(m);
-    float s;
-    row_pow2(m, s, qinv);
+      u32x4 t[3];
+      split8(x, t);
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-      split_row8(x[c], s, qh[c], ql[c]);
-      qh2[c] = qh[c] * (_Float16)0x1p-11f;
+      for (int j = 0; j < 3; j++) qt[c][j] = __builtin_bit_cast(bf16x8, t[j]);
     }
   }
   const float* mrow = MASK ? p.mask + b * p.m_sb + h * p.m_sh + (int64_t)qc * p.m_sr : nullptr;
-  const float qf = qinv * p.scale;
 
   f32x4 oacc[NDB];  // O^T: dims 16 db + 4 g + r of query lq
 #pragma unroll
@@ -312,7 +268,7 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
 #pragma unroll
       for (int db = 0; db < NDB; db++) {
         const int dim = 16 * db + lq;
-        const uint16_t* vr = Vc + t * VI + dim * 32 + slot_chunk(dim, g) * 8;
+        const uint16_t* vr = Vc + t * IMG + dim * 32 + slot_chunk(dim, g) * 8;
         const bf16x8 v0 = *reinterpret_cast<const bf16x8*>(vr);
         const bf16x8 v1 = *reinterpret_cast<const bf16x8*>(vr + 32 * HD);
         const bf16x8 v2 = *reinterpret_cast<const bf16x8*>(vr + 64 * HD);
@@ -325,44 +281,38 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
         oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, pt[t][0], o, 0, 0, 0);
       }
   };
-  // a stage's key factors and mask values: keys 4g .. + 3 of the tiles' halves
-  float kn[NT][8], mn_[NT][8];
+  // a stage's mask values: keys 4g .. + 3 of the tiles' halves
+  float mn_[NT][8];
   auto fetch = [&](int st) {
+    if constexpr (MASK) {
 #pragma unroll
-    for (int t = 0; t < NT; t++)
+      for (int t = 0; t < NT; t++)
 #pragma unroll
-      for (int e = 0; e < 8; e += 4) {
-        const int j0 = st * SK + 32 * t + 4 * e + 4 * g;
-        const f32x4 a = *reinterpret_cast<const f32x4*>(kinv + j0);
-#pragma unroll
-        for (int u = 0; u < 4; u++) kn[t][e + u] = a[u];
-        if constexpr (MASK) {
-#pragma unroll
-          for (int u = 0; u < 4; u++) mn_[t][e + u] = mrow[(int64_t)min(j0 + u, p.S - 1) * p.m_sc];
+        for (int e = 0; e < 8; e++) {
+          const int j = st * SK + 32 * t + 16 * (e >> 2) + 4 * g + (e & 3);
+          mn_[t][e] = mrow[(int64_t)min(j, p.S - 1) * p.m_sc];
         }
-      }
+    }
   };
   fetch(0);
   auto stage = [&](int st, const uint16_t* Kc, uint16_t* Kn, uint16_t* Vn, const uint16_t* Vp) {
     split_barrier();  // this stage's keys, the last one's values landed; every wave is done with the last stage
-    // the key factors and mask values loaded during the last stage: taken here,
-    // where the barrier has waited for them. A use after the loads below would
-    // wait for those too (the compiler does not count direct loads in order).
-    float kf[NT][8], mv[NT][8];
+    // the mask values loaded during the last stage: taken here, where the
+    // barrier has waited for them. A use after the loads below would wait for
+    // those too (the compiler does not count direct loads in order).
+    float mv[NT][8];
+    if constexpr (MASK) {
 #pragma unroll
-    for (int t = 0; t < NT; t++)
+      for (int t = 0; t < NT; t++)
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        asm volatile("" : "+v"(kn[t][e]));
-        kf[t][e] = kn[t][e];
-        if constexpr (MASK) {
+        for (int e = 0; e < 8; e++) {
           asm volatile("" : "+v"(mn_[t][e]));
           mv[t][e] = mn_[t][e];
         }
-      }
+    }
     fetch(min(st + 1, stages - 1));
-    load_v(Vn, st);
-    if constexpr (KD) load_k(Kn, min(st + 1, stages - 1));
+    load(vimg, Vn, st);
+    if constexpr (KD) load(kimg, Kn, min(st + 1, stages - 1));
     f32x4 sacc[NT][2];
 #pragma unroll
     for (int t = 0; t < NT; t++)
@@ -370,21 +320,25 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
       for (int kb = 0; kb < 2; kb++) {
         f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
         const int key = 16 * kb + lq;
-        const uint16_t* kr = Kc + t * KI + key * HD;
+        const uint16_t* kr = Kc + t * IMG + key * HD;
 #pragma unroll
         for (int c = 0; c < NC; c++) {
           const int pos = key_chunk<HD>(key, 4 * c + g) * 8;
-          const f16x8 k0 = *reinterpret_cast<const f16x8*>(kr + pos);
-          const f16x8 k1 = *reinterpret_cast<const f16x8*>(kr + 32 * HD + pos);
-          s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, qh2[c], s, 0, 0, 0);
-          s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0 * (_Float16)0x1p-11f, ql[c], s, 0, 0, 0);
-          s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qh[c], s, 0, 0, 0);
+          const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(kr + pos);
+          const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(kr + 32 * HD + pos);
+          const bf16x8 k2 = *reinterpret_cast<const bf16x8*>(kr + 64 * HD + pos);
+          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, qt[c][0], s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qt[c][2], s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qt[c][1], s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qt[c][0], s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qt[c][1], s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qt[c][0], s, 0, 0, 0);
         }
         sacc[t][kb] = s;
       }
     if constexpr (!KD) {
       split_lds_barrier();  // every wave has read the keys
-      load_k(Kn, min(st + 1, stages - 1));
+      load(kimg, Kn, min(st + 1, stages - 1));
     }
     if (live) pv(Vp);
     float w[NT][8];
@@ -392,7 +346,7 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
     for (int t = 0; t < NT; t++)
 #pragma unroll
       for (int e = 0; e < 8; e++) {
-        w[t][e] = sacc[t][e >> 2][e & 3] * (kf[t][e] * qf);
+        w[t][e] = sacc[t][e >> 2][e & 3] * p.scale;
         if constexpr (MASK) w[t][e] += mv[t][e];
       }
     if (st * SK + SK > p.S) {  // the last stage: no keys past S
@@ -432,22 +386,16 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
 #pragma unroll
     for (int t = 0; t < NT; t++) {
       if (!live) break;
-      uint32_t ph[8], pm[8], pl[8];
+      float x[8];
 #pragma unroll
       for (int e = 0; e < 8; e++) {
-        const float x = exp_flush(w[t][e] - mn);
-        l_part += x;
-        const Split3 sp = split3(x);
-        ph[e] = sp.h;
-        pm[e] = sp.m;
-        pl[e] = sp.l;
+        x[e] = exp_flush(w[t][e] - mn);
+        l_part += x[e];
       }
-      pt[t][0] = __builtin_bit_cast(bf16x8, (u32x4){pack_hi16(ph[0], ph[1]), pack_hi16(ph[2], ph[3]),
-                                                    pack_hi16(ph[4], ph[5]), pack_hi16(ph[6], ph[7])});
-      pt[t][1] = __builtin_bit_cast(bf16x8, (u32x4){pack_hi16(pm[0], pm[1]), pack_hi16(pm[2], pm[3]),
-                                                    pack_hi16(pm[4], pm[5]), pack_hi16(pm[6], pm[7])});
-      pt[t][2] = __builtin_bit_cast(bf16x8, (u32x4){pack_hi16(pl[0], pl[1]), pack_hi16(pl[2], pl[3]),
-                                                    pack_hi16(pl[4], pl[5]), pack_hi16(pl[6], pl[7])});
+      u32x4 y[3];
+      split8(x, y);
+#pragma unroll
+      for (int j = 0; j < 3; j++) pt[t][j] = __builtin_bit_cast(bf16x8, y[j]);
     }
   };
   for (int st = 0; st < stages; st += 2) {
@@ -478,8 +426,8 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
 
 struct SplitSizes {
   int Hk, tiles;
-  int64_t blocks;  // images
-  size_t k_bytes, v_bytes;
+  int64_t blocks;  // key or value images
+  size_t bytes;    // of the key images, and of the value images
 };
 SplitSizes split_sizes(const AttnGenericArgs& a) {
   SplitSizes z;
@@ -487,8 +435,7 @@ SplitSizes split_sizes(const AttnGenericArgs& a) {
   const int sk = a.D == 64 ? 64 : 32;
   z.tiles = (a.S + sk - 1) / sk * (sk / 32);
   z.blocks = (int64_t)a.B * z.Hk * z.tiles;
-  z.k_bytes = (size_t)z.blocks * 2 * 32 * a.D * 2;
-  z.v_bytes = (size_t)z.blocks * 3 * 32 * a.D * 2;
+  z.bytes = (size_t)z.blocks * 3 * 32 * a.D * 2;
   return z;
 }
 
@@ -518,7 +465,7 @@ bool attention_split_ok(const AttnGenericArgs& a) {
   const SplitSizes z = split_sizes(a);
   // images of at most 8 GiB: keys broadcast over a batch are written once per
   // entry, and the context keeps the buffer
-  if (z.k_bytes + z.v_bytes > (8ULL << 30)) return false;
+  if (2 * z.bytes > (8ULL << 30)) return false;
   return z.blocks < INT32_MAX && (int64_t)a.B * a.H * ((a.T + 63) / 64) < INT32_MAX;
 }
 
@@ -526,15 +473,14 @@ int launch_attention_split(fa_ctx* ctx, const AttnGenericArgs& a, hipStream_t s)
   if (!attention_split_ok(a)) return set_error(ctx, FA_ERR_UNSUPPORTED, "Attention: no split path for these operands");
   const SplitSizes z = split_sizes(a);
   DevBuf& buf = ctx->slot(slots::S_ATTN);
-  if (const int rc = buf.ensure(ctx, z.k_bytes + z.v_bytes + (size_t)z.blocks * 32 * 4)) return rc;
+  if (const int rc = buf.ensure(ctx, 2 * z.bytes)) return rc;
   SplitKvParams kv;
   kv.k = a.k; kv.v = a.v; kv.k_sb = a.k_sb; kv.k_sh = a.k_sh; kv.v_sb = a.v_sb; kv.v_sh = a.v_sh;
   kv.Hk = z.Hk; kv.S = a.S; kv.tiles = z.tiles;
   kv.kimg = buf.as<uint16_t>();
-  kv.vimg = reinterpret_cast<uint16_t*>(buf.as<char>() + z.k_bytes);
-  kv.kinv = reinterpret_cast<float*>(buf.as<char>() + z.k_bytes + z.v_bytes);
+  kv.vimg = reinterpret_cast<uint16_t*>(buf.as<char>() + z.bytes);
   SplitParams p;
-  p.q = a.q; p.k = a.k; p.v = a.v; p.mask = a.mask; p.kimg = kv.kimg; p.vimg = kv.vimg; p.kinv = kv.kinv; p.out = a.out;
+  p.q = a.q; p.k = a.k; p.v = a.v; p.mask = a.mask; p.kimg = kv.kimg; p.vimg = kv.vimg; p.out = a.out;
   p.H = a.H; p.Hk = z.Hk; p.T = a.T; p.S = a.S; p.tiles = z.tiles;
   p.q_sb = a.q_sb; p.q_sh = a.q_sh; p.k_sb = a.k_sb; p.k_sh = a.k_sh; p.v_sb = a.v_sb; p.v_sh = a.v_sh;
   p.m_sb = a.m_sb; p.m_sh = a.m_sh; p.m_sr = a.m_sr; p.m_sc = a.m_sc;

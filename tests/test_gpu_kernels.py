@@ -503,3 +503,23 @@ def test_attention_split_infinities(ctx, D, B, H, Tq, Sk, masked):
     assert np.array_equal(np.isfinite(got), fin)
     assert np.array_equal(got[~fin], want[~fin].astype(np.float32), equal_nan=True)
     assert np.abs(got[fin] - want[fin]).max() <= 4e-6 * np.abs(want[fin]).max()
+
+
+@pytest.mark.parametrize("D,B,H,Tq,Sk", [(64, 1, 8, 129, 449), (64, 2, 8, 192, 256), (128, 1, 8, 150, 225),
+                                         (256, 2, 8, 150, 257)])
+@pytest.mark.parametrize("e", [20, 40, 60])
+def test_attention_rows_of_wide_range(ctx, D, B, H, Tq, Sk, e):
+    """Elements of very different magnitudes within one query or key: a query
+    element of 2^e where every key holds 0 (or 2^-e), a key element of 2^e where
+    every query does. The other elements make the score, as in float32, so
+    test_attention_split_edges' bound holds."""
+    r = np.random.default_rng(D + e)
+    q, k, v = (r.standard_normal((B, H, n, D)).astype(np.float32) for n in (Tq, Sk, Sk))
+    q[..., 3], k[..., 3] = 2.0 ** e, 0
+    k[..., 9], q[..., 9] = -(2.0 ** e), 0
+    q[..., 17], k[..., 17] = 2.0 ** e, 2.0 ** -e
+    s = q.astype(np.float64) @ np.swapaxes(k, 2, 3).astype(np.float64) / np.sqrt(D)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = (p / p.sum(-1, keepdims=True)) @ v.astype(np.float64)
+    got = T.AttentionScaled(q, k, v, None, float(1 / np.sqrt(D)), ctx=ctx)
+    assert np.abs(got - want).max() <= 4e-6 * np.abs(want).max()
