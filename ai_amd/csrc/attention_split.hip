@@ -146,37 +146,6 @@ struct SplitParams {
   float scale;
 };
 
-// One query in plain fp32, by one wave, lane l holding dims l, l + 64, ...:
-// for queries whose split result is not finite: an infinity has no finite
-// second term, so the split gives NaN where the operands themselves give an
-// infinity, or a weight of 0.
-template <int HD, bool MASK>
-__device__ void plain_query(const SplitParams& p, int b, int h, int qi, int lane) {
-  constexpr int N = HD / 64;
-  const float* qr = p.q + b * p.q_sb + h * p.q_sh + (int64_t)qi * HD + lane;
-  const float* kr = p.k + b * p.k_sb + h * p.k_sh + lane;
-  const float* vr = p.v + b * p.v_sb + h * p.v_sh + lane;
-  const float* mrow = MASK ? p.mask + b * p.m_sb + h * p.m_sh + (int64_t)qi * p.m_sr : nullptr;
-  auto score = [&](int j) {
-    float s = 0.f;
-    for (int i = 0; i < N; i++) s = fmaf(qr[64 * i], kr[(int64_t)j * HD + 64 * i], s);
-    s = wave_sum(s) * p.scale;
-    if constexpr (MASK) s += mrow[(int64_t)j * p.m_sc];
-    return s;
-  };
-  float m = -1e30f;
-  for (int j = 0; j < p.S; j++) m = fmaxf(m, score(j));
-  float l = 0.f, o[N];
-  for (int i = 0; i < N; i++) o[i] = 0.f;
-  for (int j = 0; j < p.S; j++) {
-    const float w = exp_flush(score(j) - m);
-    l += w;
-    for (int i = 0; i < N; i++) o[i] = fmaf(w, vr[(int64_t)j * HD + 64 * i], o[i]);
-  }
-  float* orow = p.out + (((int64_t)b * p.H + h) * p.T + qi) * HD + lane;
-  for (int i = 0; i < N; i++) orow[64 * i] = o[i] * (1.f / l);
-}
-
 // Workgroup barriers after the wave's vector loads and LDS accesses, and after
 // its LDS accesses alone.
 __device__ __forceinline__ void split_barrier() {
@@ -202,6 +171,75 @@ __device__ __forceinline__ float lanes4_sum(float x) {
   x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
   auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// The wave's 16 queries on the fp32 MFMA with operands straight from memory,
+// those in `redo` stored: for queries whose split result is not finite. An
+// infinity has no finite second term, so the split gives NaN where the
+// operands themselves give an infinity, or a weight of 0. The organisation is
+// attention_dense_kernel's without its staging: 16 keys a step, S^T = K . Q^T,
+// O^T += V^T . P^T. One query at a time in vector code took 42 ms where one key
+// of each head is infinite (32 x 8 heads x 512 x 1 024, head_dim 64) against
+// 0.86 here (0.25 with finite operands, 0.36 on attention_dense_kernel).
+template <int HD, bool MASK>
+__device__ __forceinline__ void plain_queries(const SplitParams& p, int b, int h, int q0, uint64_t redo, int lane) {
+  const int lq = lane & 15, g = lane >> 4;
+  const int qi = q0 + lq, qc = min(qi, p.T - 1);
+  const float* qr = p.q + b * p.q_sb + h * p.q_sh + (int64_t)qc * HD + 4 * g;
+  const float* kb = p.k + b * p.k_sb + h * p.k_sh + 4 * g;
+  const float* vb = p.v + b * p.v_sb + h * p.v_sh + lq;
+  const float* mrow = MASK ? p.mask + b * p.m_sb + h * p.m_sh + (int64_t)qc * p.m_sr : nullptr;
+  f32x4 q[HD / 16], o[HD / 16];  // dims 16 s + 4 g .. + 3 of query lq
+#pragma unroll
+  for (int s = 0; s < HD / 16; s++) {
+    q[s] = *reinterpret_cast<const f32x4*>(qr + 16 * s);
+    o[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  float m = -1e30f, l = 0.f;
+  for (int j0 = 0; j0 < p.S; j0 += 16) {
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};  // keys j0 + 4 g + r against query lq
+    const float* kr = kb + (int64_t)min(j0 + lq, p.S - 1) * HD;
+#pragma unroll
+    for (int c = 0; c < HD / 16; c++) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(kr + 16 * c);
+#pragma unroll
+      for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], q[c][e], s, 0, 0, 0);
+    }
+    float w[4], top = -1e30f;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int j = j0 + 4 * g + r;
+      w[r] = s[r] * p.scale;
+      if constexpr (MASK) w[r] += mrow[(int64_t)min(j, p.S - 1) * p.m_sc];
+      if (j < p.S) top = fmaxf(top, w[r]);
+    }
+    const float mn = fmaxf(m, lanes4_max(top));
+    const float alpha = exp_flush(m - mn);
+    m = mn;
+    l *= alpha;
+#pragma unroll
+    for (int c = 0; c < HD / 16; c++) o[c] *= alpha;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      w[r] = j0 + 4 * g + r < p.S ? exp_flush(w[r] - mn) : 0.f;
+      l += w[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int j = j0 + 4 * g + r;
+      const float* vr = vb + (int64_t)min(j, p.S - 1) * HD;
+#pragma unroll
+      for (int c = 0; c < HD / 16; c++) {
+        const float v = vr[16 * c];
+        o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(j < p.S ? v : 0.f, w[r], o[c], 0, 0, 0);
+      }
+    }
+  }
+  const float inv = 1.f / lanes4_sum(l);
+  if (!(redo >> lq & 1)) return;
+  float* orow = p.out + (((int64_t)b * p.H + h) * p.T + qi) * HD + 4 * g;
+#pragma unroll
+  for (int c = 0; c < HD / 16; c++) *reinterpret_cast<f32x4*>(orow + 16 * c) = o[c] * inv;
 }
 
 template <int HD, int W, bool MASK>
@@ -405,7 +443,8 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
   split_barrier();  // the last values (no load may still be writing LDS when the workgroup ends)
   if (live) pv((stages & 1) ? V0 : V1);
 
-  const float inv = 1.f / lanes4_sum(l_part);
+  const float l_tot = lanes4_sum(l_part);
+  const float inv = 1.f / l_tot;
   float seen = 0.f;  // NaN if any output is not finite
   float* orow = p.out + ((int64_t)bh * p.T + qi) * HD + 4 * g;
 #pragma unroll
@@ -415,12 +454,12 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
     for (int r = 0; r < 4; r++) seen = fmaf(o[r], 0.f, seen);
     if (qvalid) *reinterpret_cast<f32x4*>(orow + 16 * db) = o;
   }
-  uint64_t redo = __ballot(qvalid && seen != seen);
+  // (a query whose weights are all 0, masked entirely, is NaN either way)
+  uint64_t redo = __ballot(qvalid && seen != seen && l_tot != 0.f);
   redo = (redo | redo >> 16 | redo >> 32 | redo >> 48) & 0xFFFFu;  // queries of the wave
   if (redo) {
     __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0): the stores above, which other lanes write over
-    for (int i = 0; i < 16; i++)
-      if (redo >> i & 1) plain_query<HD, MASK>(p, b, h, (qblk * W + wave) * 16 + i, lane);
+    plain_queries<HD, MASK>(p, b, h, (qblk * W + wave) * 16, redo, lane);
   }
 }
 

@@ -7,6 +7,7 @@ are the reference's: |gpu - want| <= 1e-4 * (1 + |want|) for products
 (tensor/attention_test.go:64-91). Max |delta| is printed for each case.
 """
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -523,3 +524,52 @@ def test_attention_rows_of_wide_range(ctx, D, B, H, Tq, Sk, e):
     want = (p / p.sum(-1, keepdims=True)) @ v.astype(np.float64)
     got = T.AttentionScaled(q, k, v, None, float(1 / np.sqrt(D)), ctx=ctx)
     assert np.abs(got - want).max() <= 4e-6 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("D,B,H,Tq,Sk", [(64, 8, 8, 300, 500), (128, 4, 4, 300, 500), (256, 4, 4, 257, 479)])
+@pytest.mark.parametrize("what", ["value", "key", "masked"])
+def test_attention_split_non_finite_speed(ctx, D, B, H, Tq, Sk, what):
+    """A call whose every query meets an infinite value or key, or is masked
+    entirely, stays within eight times the finite call's time (the fp32 products
+    alone take two to three times as long; one query after the other took 50 and
+    more)."""
+    r = rng(D)
+    q, k, v = (r.standard_normal((B, H, n, D)).astype(np.float32) for n in (Tq, Sk, Sk))
+    mask = np.zeros((B, Sk), np.float32)
+    L = N.lib()
+    ptrs = []
+    for a in (q, k, v, mask, q):
+        p = C.c_void_p()
+        N.check(ctx.h, L.fa_device_alloc(ctx.h, a.nbytes, C.byref(p)))
+        N.check(ctx.h, L.fa_memcpy_h2d(ctx.h, p, a.ctypes.data, a.nbytes))
+        ptrs.append(p)
+
+    def best():
+        t = []
+        for _ in range(5):
+            ctx.sync()
+            t0 = time.perf_counter()
+            for _ in range(4):
+                N.check(ctx.h, L.fa_attention_dev(ctx.h, ptrs[0], ptrs[1], ptrs[2], B, H, Tq, Sk, D, H * Tq * D,
+                                                  Tq * D, H * Sk * D, Sk * D, H * Sk * D, Sk * D, ptrs[3], Sk, 0, 0, 1,
+                                                  0.1, ptrs[4]))
+            ctx.sync()
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    best()
+    finite = best()
+    k[:, :, 5, 3] = np.inf if what == "key" else k[:, :, 5, 3]
+    v[:, :, 5, 3] = np.inf if what == "value" else v[:, :, 5, 3]
+    mask[:] = -np.inf if what == "masked" else 0
+    for p, a in zip(ptrs[1:4], (k, v, mask)):
+        N.check(ctx.h, L.fa_memcpy_h2d(ctx.h, p, a.ctypes.data, a.nbytes))
+    assert best() <= 8 * finite
+    got = np.empty_like(q)
+    N.check(ctx.h, L.fa_memcpy_d2h(ctx.h, got.ctypes.data, ptrs[4], got.nbytes))
+    for p in ptrs:
+        L.fa_device_free(ctx.h, p)
+    if what == "value":  # an infinite output in that column, finite ones beside it
+        assert np.isposinf(got[..., 3]).all() and np.isfinite(np.delete(got, 3, -1)).all()
+    elif what == "masked":
+        assert np.isnan(got).all()
