@@ -35,6 +35,7 @@
 // (2 048 queries and keys, 3 heads
 // of 256: 211 -> 192 us per call). The row maximum is lazy: the
 // offset moves when a stage's maximum exceeds it by more than 8.
+#include <algorithm>
 #include <cstdlib>
 
 #include "fa_internal.h"
@@ -486,25 +487,51 @@ void launch_split(const SplitParams& p, int64_t grid, hipStream_t s) {
     hipLaunchKernelGGL((attention_split_kernel<HD, W, false>), dim3((unsigned)grid), dim3(64 * W), 0, s, p);
 }
 
+// The rule: the 16-bit path where the time it saves on the keys exceeds what
+// it adds, from both kernels' times at 156 shapes (1 to 1 024 queries, 32 to
+// 4 096 keys, 1 to 64 batches of 1 to 8 heads, with and without a shared
+// key/value head). It adds a launch, a longer prologue and the images, which
+// cost their 18 bytes per key element whatever the queries are (6 TB/s while
+// they stay in the last-level cache, 4 beyond). It saves microseconds per key
+// that grow with the 64-query blocks once those are more than one per CU (at
+// head_dim 256 the fp32 kernel slows down from half the CUs on). Below 192 keys
+// and 0.1 GFLOP (0.5 at 256) the fp32 kernel stays in any case. Us, fp32 and
+// 16-bit: 8 heads x 1 024 x 1 024, 64: 72 and 34; 51 x 8 x 1 x 1 024, 64: 103 and
+// 159; the same on one shared head: 102 and 63; 2 x 8 x 128 x 256, 256: 35 and 43;
+// 32 x 3 x 256 x 256, 256: 87 and 65; 4 x 3 x 1 024 x 1 024, 256: 194 and 118; 8 x 8 x
+// 32 x 256, 256: 34 and 45; 26 x 8 x 1 x 1 024, 128: 113 and 170.
+// (FA_ATTN_SPLIT=0 turns it off, for comparisons.)
+bool attention_split_pays(const AttnGenericArgs& a, const SplitSizes& z) {
+  if (a.S < 192 || 4.0 * a.B * a.H * (double)a.T * a.S * a.D < (a.D == 256 ? 5e8 : 1e8)) return false;
+  const double blocks = (double)a.B * a.H * ((a.T + 63) / 64);
+  const double image = 18.0 * a.D * a.B * z.Hk * (double)a.S;
+  double key, fixed;  // us saved per key, us added per call
+  if (a.D == 64) {
+    key = blocks <= 256 ? 0.04 : std::max(0.055, 9.5e-5 * blocks);
+    fixed = 7.5;
+  } else if (a.D == 128) {
+    key = blocks <= 256 ? 0.058 : std::max(0.095, 1.4e-4 * blocks);
+    fixed = 6.5;
+  } else {
+    key = blocks <= 128 ? 0.0236 : blocks <= 256 ? 0.085 : std::max(0.11, 4.2e-4 * blocks);
+    fixed = 12.;
+  }
+  return key * a.S >= fixed + image / (image < 2e8 ? 6e6 : 4e6);
+}
+
 }  // namespace
 
-// With few keys or little work the image pass and the longer prologue cost
-// what the products save. Measured, us against attention_dense_kernel: 32 x 8
-// heads x 64 x 64 keys, head_dim 64: 14.5 and 7.9; 8 x 3 x 128 x 128, 256: 33 and
-// 22; 1 x 3 x 200 x 200, 256: 33 and 28; and 1 x 8 x 256 x 256, 64: 14 and 20; 2 x 4 x
-// 300 x 300, 128: 24 and 42; 1 x 3 x 512 x 512, 256: 58 and 65. (FA_ATTN_SPLIT=0
-// turns it off, for comparisons.)
 bool attention_split_ok(const AttnGenericArgs& a) {
   static const bool off = [] {
     const char* e = std::getenv("FA_ATTN_SPLIT");
     return e && e[0] == '0';
   }();
   if (off || !attention_dense_ok(a) || (a.D != 64 && a.D != 128 && a.D != 256)) return false;
-  if (!(a.scale > 0.f) || a.S < 192 || 4.0 * a.B * a.H * (double)a.T * a.S * a.D < (a.D == 256 ? 5e8 : 1e8)) return false;
+  if (!(a.scale > 0.f) || a.S <= 0 || a.T <= 0) return false;
   const SplitSizes z = split_sizes(a);
   // images of at most 8 GiB: keys broadcast over a batch are written once per
   // entry, and the context keeps the buffer
-  if (2 * z.bytes > (8ULL << 30)) return false;
+  if (2 * z.bytes > (8ULL << 30) || !attention_split_pays(a, z)) return false;
   return z.blocks < INT32_MAX && (int64_t)a.B * a.H * ((a.T + 63) / 64) < INT32_MAX;
 }
 

@@ -402,7 +402,9 @@ def test_attention_mfma_dev_entry_point(ctx):
 @pytest.mark.parametrize("D,B,H,Hkv,Tq,Sk,kind", [
     (64, 1, 8, 8, 129, 449, "none"), (64, 2, 8, 1, 128, 192, "pad"), (64, 3, 4, 4, 200, 257, "full"),
     (128, 1, 7, 7, 33, 1023, "none"), (128, 4, 4, 1, 65, 225, "full"), (256, 2, 3, 1, 257, 479, "pad"),
-    (256, 4, 3, 3, 200, 256, "full"), (256, 1, 2, 2, 1000, 321, "none")])
+    (256, 4, 3, 3, 200, 256, "full"), (256, 1, 2, 2, 1000, 321, "none"),
+    # (head_dim 256 with more keys or blocks: the three above take the fp32 kernel)
+    (256, 16, 4, 1, 250, 321, "full"), (256, 1, 3, 3, 300, 1023, "none"), (256, 2, 6, 1, 300, 700, "pad")])
 def test_attention_split_edges(ctx, D, B, H, Hkv, Tq, Sk, kind):
     """The 16-bit MFMA attention (attention_split.hip) around its 64/128-query
     items and 32/64-key stages against float64. Rows of q and k, and q and k
@@ -468,7 +470,7 @@ def test_attention_broadcast_batch_beyond_the_images(ctx):
 
 
 @pytest.mark.parametrize("D,B,H,Tq,Sk,masked", [(64, 1, 8, 129, 449, False), (128, 2, 4, 150, 225, True),
-                                               (256, 2, 3, 257, 479, True)])
+                                               (256, 2, 3, 257, 479, True), (256, 2, 6, 300, 700, True)])
 def test_attention_split_infinities(ctx, D, B, H, Tq, Sk, masked):
     """Infinities in keys and values, and rows whose magnitudes only meet in a
     finite product, give what the float32 products give (a score of -inf is a
@@ -507,7 +509,7 @@ def test_attention_split_infinities(ctx, D, B, H, Tq, Sk, masked):
 
 
 @pytest.mark.parametrize("D,B,H,Tq,Sk", [(64, 1, 8, 129, 449), (64, 2, 8, 192, 256), (128, 1, 8, 150, 225),
-                                         (256, 2, 8, 150, 257)])
+                                         (256, 2, 8, 150, 257), (256, 1, 6, 300, 1000)])
 @pytest.mark.parametrize("e", [20, 40, 60])
 def test_attention_rows_of_wide_range(ctx, D, B, H, Tq, Sk, e):
     """Elements of very different magnitudes within one query or key: a query
@@ -526,7 +528,7 @@ def test_attention_rows_of_wide_range(ctx, D, B, H, Tq, Sk, e):
     assert np.abs(got - want).max() <= 4e-6 * np.abs(want).max()
 
 
-@pytest.mark.parametrize("D,B,H,Tq,Sk", [(64, 8, 8, 300, 500), (128, 4, 4, 300, 500), (256, 4, 4, 257, 479)])
+@pytest.mark.parametrize("D,B,H,Tq,Sk", [(64, 8, 8, 300, 500), (128, 4, 4, 300, 500), (256, 2, 6, 300, 700)])
 @pytest.mark.parametrize("what", ["value", "key", "masked"])
 def test_attention_split_non_finite_speed(ctx, D, B, H, Tq, Sk, what):
     """A call whose every query meets an infinite value or key, or is masked
@@ -573,3 +575,17 @@ def test_attention_split_non_finite_speed(ctx, D, B, H, Tq, Sk, what):
         assert np.isposinf(got[..., 3]).all() and np.isfinite(np.delete(got, 3, -1)).all()
     elif what == "masked":
         assert np.isnan(got).all()
+
+
+@pytest.mark.parametrize("D,B,H,Hkv,Tq,Sk", [(64, 51, 8, 8, 1, 1024), (64, 26, 8, 8, 8, 256), (128, 26, 8, 8, 1, 1024),
+                                             (256, 2, 8, 8, 128, 256), (256, 8, 8, 8, 32, 256),
+                                             (256, 20, 1, 1, 212, 212), (256, 42, 3, 3, 34, 971)])
+def test_attention_few_queries_stay_on_the_fp32_kernel(ctx, D, B, H, Hkv, Tq, Sk):
+    """Calls whose images would cost more than the 16-bit products save take the
+    fp32 kernel: every entry of the batch has the bits of its own call, whose
+    work is below the 16-bit path's least."""
+    r = rng(D + Tq)
+    q, k, v = (r.standard_normal((B, h, n, D)).astype(np.float32) for h, n in ((H, Tq), (Hkv, Sk), (Hkv, Sk)))
+    got = T.AttentionScaled(q, k, v, None, 0.1, ctx=ctx)
+    for b in (0, B - 1):
+        assert np.array_equal(got[b:b + 1], T.AttentionScaled(q[b:b + 1], k[b:b + 1], v[b:b + 1], None, 0.1, ctx=ctx))
