@@ -8,8 +8,8 @@
 // per 32 keys) and the prologue at 256.
 //
 // Queries, keys, values and probabilities are three exact bf16 terms each
-// (split3), a product the six MFMAs whose terms' orders add up to at most two
-// (what is dropped, mid . lo and lo . lo, is below 2^-21 of the product of the two values). bf16 has
+// (split8), a product the six MFMAs whose terms' orders add up to at most two
+// (what is dropped, mid . lo and lo . lo, is below 2^-25 of the product). bf16 has
 // float32's range, so elements of one row may be of any magnitude beside each
 // other, and a masked key may hold any finite value without touching its
 // neighbours. (Two fp16 terms for the scores, scaled by a power of two per
@@ -45,6 +45,8 @@ namespace fa {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr float kSplitTau = 8.f;
@@ -56,21 +58,21 @@ __device__ __forceinline__ int key_chunk(int key, int c) {
 __device__ __forceinline__ int slot_chunk(int dim, int g) { return g ^ ((dim >> 1) & 3); }
 
 // Eight values as three bf16 terms, each packed as the 16 bytes it takes in an
-// image or an operand.
+// image or an operand: hi the nearest bf16, mid that of the rest, lo the rest
+// of that, both rests exact in float32 and lo in bf16. Rounded terms leave
+// signed rests of half the size that cut ones (split3) leave: the dropped
+// products are a sixteenth of theirs and carry no bias.
 __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&t)[3]) {
-  uint32_t h[8], m[8], l[8];
-#pragma unroll
-  for (int e = 0; e < 8; e++) {
-    const Split3 sp = split3(x[e]);
-    h[e] = sp.h;
-    m[e] = sp.m;
-    l[e] = sp.l;
-  }
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    t[0][i] = pack_hi16(h[2 * i], h[2 * i + 1]);
-    t[1][i] = pack_hi16(m[2 * i], m[2 * i + 1]);
-    t[2][i] = pack_hi16(l[2 * i], l[2 * i + 1]);
+    f32x2 r = {x[2 * i], x[2 * i + 1]};
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+      t[j][i] = w;
+      r.x -= __uint_as_float(w << 16);
+      r.y -= __uint_as_float(w & 0xFFFF0000u);
+    }
   }
 }
 
@@ -357,7 +359,9 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
     for (int t = 0; t < NT; t++)
 #pragma unroll
       for (int kb = 0; kb < 2; kb++) {
-        f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+        // hi . hi and the smaller terms in sums of their own: a sum of all of them
+        // is rounded at full size six times per chunk
+        f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f}, y = s;
         const int key = 16 * kb + lq;
         const uint16_t* kr = Kc + t * IMG + key * HD;
 #pragma unroll
@@ -366,14 +370,14 @@ __global__ __launch_bounds__(64 * W, 2) void attention_split_kernel(SplitParams 
           const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(kr + pos);
           const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(kr + 32 * HD + pos);
           const bf16x8 k2 = *reinterpret_cast<const bf16x8*>(kr + 64 * HD + pos);
-          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, qt[c][0], s, 0, 0, 0);
-          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qt[c][2], s, 0, 0, 0);
-          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qt[c][1], s, 0, 0, 0);
-          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qt[c][0], s, 0, 0, 0);
-          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qt[c][1], s, 0, 0, 0);
+          y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, qt[c][0], y, 0, 0, 0);
+          y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qt[c][2], y, 0, 0, 0);
+          y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qt[c][1], y, 0, 0, 0);
+          y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qt[c][0], y, 0, 0, 0);
+          y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qt[c][1], y, 0, 0, 0);
           s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qt[c][0], s, 0, 0, 0);
         }
-        sacc[t][kb] = s;
+        sacc[t][kb] = s + y;
       }
     if constexpr (!KD) {
       split_lds_barrier();  // every wave has read the keys
