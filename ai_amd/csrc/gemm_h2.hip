@@ -277,11 +277,14 @@ __global__ __launch_bounds__(kSmallNW * 64) void gemm_h2_small_kernel(H2Params p
   const uint16_t* b0 = p.b + min(bn, N - 1) * p.ldb + k_off;
   const uint16_t* b1 = p.b + min(n0 + 32 + (lane & 31), N - 1) * p.ldb + k_off;
 
-  f32x16 acc[NB];
+  // hi . w and lo . w in sums of their own: one sum for both is rounded twice
+  // per step at full size (24 layers of 19 tokens: error against 64 bits 6.7e-7
+  // with one, 4.3e-7 with two, 6.6e-7 by the three-term bf16 products)
+  f32x16 acc[NB], low[NB];
 #pragma unroll
   for (int j = 0; j < NB; j++)
 #pragma unroll
-    for (int r = 0; r < 16; r++) acc[j][r] = 0.f;
+    for (int r = 0; r < 16; r++) acc[j][r] = low[j][r] = 0.f;
   struct Regs {
     u32x4 a[4];  // hi, lo of the slab's two k-steps
     u32x4 b[2 * NB];
@@ -302,8 +305,8 @@ __global__ __launch_bounds__(kSmallNW * 64) void gemm_h2_small_kernel(H2Params p
       const f16x8 hi = __builtin_bit_cast(f16x8, g.a[2 * st]), lo = __builtin_bit_cast(f16x8, g.a[2 * st + 1]);
 #pragma unroll
       for (int j = 0; j < NB; j++)
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-            lo, __builtin_bit_cast(f16x8, g.b[NB * st + j]) * (_Float16)0x1p-11f, acc[j], 0, 0, 0);
+        low[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+            lo, __builtin_bit_cast(f16x8, g.b[NB * st + j]) * (_Float16)0x1p-11f, low[j], 0, 0, 0);
 #pragma unroll
       for (int j = 0; j < NB; j++)
         acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, __builtin_bit_cast(f16x8, g.b[NB * st + j]), acc[j], 0, 0, 0);
@@ -330,7 +333,7 @@ __global__ __launch_bounds__(kSmallNW * 64) void gemm_h2_small_kernel(H2Params p
 #pragma unroll
   for (int j = 0; j < NB; j++)
 #pragma unroll
-    for (int r = 0; r < 16; r++) red[wave][j][r][lane] = acc[j][r];
+    for (int r = 0; r < 16; r++) red[wave][j][r][lane] = acc[j][r] + low[j][r];
   __syncthreads();
 
   // C element (j, r, l): row 8*(r/4) + 4*(l/32) + r%4, column 32*j + l%32.
