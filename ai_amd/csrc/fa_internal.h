@@ -201,11 +201,13 @@ int launch_gemm_h2(fa_ctx* ctx, const GemmH2Args& g, hipStream_t stream);
 bool gemm_h2_enabled();
 
 // Preparation of bf16 weights for launch_gemm_h2: *max_bits (zeroed by the
-// caller) becomes the largest |w| as bf16 bits; norms[r] the 2-norm of row r;
+// caller) becomes the largest |w| as bf16 bits; norms[r] the 2-norm of row r (its
+// columns weighted by t unless that is null);
 // dst = fp16(w * scale), *bad (zeroed by the caller) nonzero when one of them
 // is not exact.
 int launch_h2_absmax(fa_ctx* ctx, const uint16_t* w, int64_t n, uint32_t* max_bits, hipStream_t s);
-int launch_h2_row_norms(fa_ctx* ctx, const uint16_t* w, int64_t rows, int64_t cols, float* norms, hipStream_t s);
+int launch_h2_row_norms(fa_ctx* ctx, const uint16_t* w, int64_t rows, int64_t cols, const float* t, float* norms,
+                        hipStream_t s);
 int launch_h2_convert(fa_ctx* ctx, const uint16_t* w, int64_t n, float scale, uint16_t* dst, uint32_t* bad,
                       hipStream_t s);
 

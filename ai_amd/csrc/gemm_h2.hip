@@ -387,17 +387,18 @@ __global__ __launch_bounds__(256) void h2_absmax_kernel(const uint16_t* __restri
 }
 
 __global__ __launch_bounds__(256) void h2_row_norms_kernel(const uint16_t* __restrict__ w, int64_t rows, int64_t cols,
-                                                           float* __restrict__ norms) {
+                                                           const float* __restrict__ t, float* __restrict__ norms) {
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int lane = threadIdx.x & 63;
-  float s = 0.f;
+  double s = 0.;  // (squares of small weights leave float32's range)
   for (int64_t c = lane; c < cols; c += 64) {
-    const float x = __uint_as_float((uint32_t)w[row * cols + c] << 16);
-    s = fmaf(x, x, s);
+    const double x = (double)__uint_as_float((uint32_t)w[row * cols + c] << 16) * (t ? (double)t[c] : 1.);
+    s = fma(x, x, s);
   }
-  s = wave_sum(s);
-  if (lane == 0) norms[row] = sqrtf(s);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (lane == 0) norms[row] = (float)sqrt(s);
 }
 
 __global__ __launch_bounds__(256) void h2_convert_kernel(const uint16_t* __restrict__ w, int64_t n, float scale,
@@ -543,9 +544,11 @@ int launch_h2_absmax(fa_ctx* ctx, const uint16_t* w, int64_t n, uint32_t* max_bi
   return FA_OK;
 }
 
-int launch_h2_row_norms(fa_ctx* ctx, const uint16_t* w, int64_t rows, int64_t cols, float* norms, hipStream_t s) {
+int launch_h2_row_norms(fa_ctx* ctx, const uint16_t* w, int64_t rows, int64_t cols, const float* t, float* norms,
+                        hipStream_t s) {
   if (rows <= 0) return FA_OK;
-  hipLaunchKernelGGL(h2_row_norms_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, w, rows, cols, norms);
+  hipLaunchKernelGGL(h2_row_norms_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, w, rows, cols, t,
+                     norms);
   FA_CHECK_LAUNCH(ctx);
   return FA_OK;
 }

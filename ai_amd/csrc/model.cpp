@@ -183,23 +183,83 @@ void set_b(GemmArgs& g, const Mat& w, int64_t row0 = 0) {
   g.b_plane = w.plane();
 }
 
+// 2-norms of the rows of matrices (a three-plane one's hi plane, within 1 % of
+// the whole), each column weighted by t (all ones if empty).
+struct RowNorms {
+  struct Job {
+    const Mat* w;
+    std::vector<float> t;
+    std::vector<float> out;
+  };
+  std::vector<Job> jobs;
+  int add(const Mat& w, std::vector<float> t = {}) {
+    jobs.push_back({&w, std::move(t), {}});
+    return (int)jobs.size() - 1;
+  }
+  int run(fa_ctx* ctx, hipStream_t s) {
+    size_t nt = 0, rows = 0;
+    for (auto& j : jobs) {
+      nt += j.t.size();
+      rows += j.w->rows;
+    }
+    std::vector<float> t, host(rows);
+    for (auto& j : jobs) t.insert(t.end(), j.t.begin(), j.t.end());
+    DevBuf buf;
+    int rc = buf.ensure(ctx, (nt + rows) * 4);
+    auto work = [&]() -> int {
+      if (nt) FA_HIP_CHECK(ctx, hipMemcpyAsync(buf.ptr, t.data(), nt * 4, hipMemcpyHostToDevice, s));
+      size_t at = 0, out = nt;
+      for (auto& j : jobs) {
+        const float* jt = j.t.empty() ? nullptr : buf.as<float>() + at;
+        if (const int r = launch_h2_row_norms(ctx, j.w->p, j.w->rows, j.w->cols, jt, buf.as<float>() + out, s)) return r;
+        at += j.t.size();
+        out += j.w->rows;
+      }
+      FA_HIP_CHECK(ctx, hipMemcpyAsync(host.data(), buf.as<float>() + nt, rows * 4, hipMemcpyDeviceToHost, s));
+      FA_HIP_CHECK(ctx, hipStreamSynchronize(s));
+      return FA_OK;
+    };
+    if (!rc) rc = work();
+    buf.release();
+    if (rc) return rc;
+    size_t at = 0;
+    for (auto& j : jobs) {
+      j.out.assign(host.begin() + at, host.begin() + at + j.w->rows);
+      at += j.w->rows;
+    }
+    return FA_OK;
+  }
+};
+
 // Decides whether the layers' products can run on split activations
 // (gemm_h2.hip) and the head_dim-256 layers on the tile attention, and
-// prepares both: m->h2, m->tiles. They need
-//  - a bound for every split operand, from which its power of two is taken
-//    (the bound just below 2^15): a normed row has 2-norm at most sqrt(d)
-//    max|gain|, so |x_j| is at most that and |w . x| at most |w| times it;
-//    attention outputs are convex combinations of values; |gelu(g) u| <= |g|
-//    |u|; the residual stream is a sum of normed rows. The activations'
-//    split then keeps 23 bits down to 2^-29 of the bound (split2,
-//    device_math.h), the attention's, whose lo terms have no scale of their
-//    own, down to 2^-18. Gains whose largest value is far above their root
-//    mean square would put typical values too far below the bounds (64 times
-//    for the products and values, 1 024 for q and k): those models keep the
-//    three-term products and the fp32 attention, as do non-finite weights;
-//  - for the products, every layer matrix bf16-exact (terms == 1) and exact
-//    in fp16 after one power of two for the matrix (its largest value just
-//    below 2^15: values down to 2^-32 of that keep all their bits).
+// prepares both: m->h2, m->tiles.
+//
+// Each split operand needs a bound, from which its power of two is taken (the
+// bound just below 2^15). A normed row has 2-norm at most sqrt(d) before its
+// gains g, so a product with weights w of it is at most sqrt(d) |w o g|, the
+// gains taken into the row's norm (gains and weights may make up for each
+// other); attention outputs are convex combinations of values; |gelu(a) b| <=
+// |a| |b|; the residual stream is a sum of normed rows.
+//
+// A bound far above the values themselves costs them their low bits: an
+// element of the products' operands is off by 2^-36 of the scaled range where
+// that is more than 2^-23 of it, and one of the attention's, whose lo terms
+// have no scale of their own, by 2^-25. What that adds to an output is the
+// row's norm times it, to be held against the output itself, the row's norm
+// with each column weighted by its operand's typical size: the gain for a
+// normed row, the same with one in 32 for attention outputs (averaged over
+// keys), a quarter of the two factors' product for GeGLU. It has to stay below
+// 2^-28 (attention 2^-26) in every row: a sixteenth of a float32 rounding,
+// which leaves room for operands that far below their typical size (evenly
+// sized gains and weights come to 2^-40 to 2^-45, and 2^-34). The same for the
+// weights: w 2^-11, the factor of the lo terms, is rounded to 2^-24 of the
+// scaled range where w is below 2^-21 of its matrix's largest.
+//
+// Models that do not hold this keep the three-term products, or the fp32
+// attention, as do those with non-finite weights; the products also need
+// every layer matrix bf16-exact (terms == 1) and exact in fp16 after one power
+// of two for the matrix (its largest value just below 2^15).
 int prepare_h2(fa_model* m) {
   m->h2 = m->tiles = false;
   fa_ctx* ctx = m->ctx;
@@ -212,37 +272,27 @@ int prepare_h2(fa_model* m) {
     if (v2) mats.insert(mats.end(), {&L.wple_gate, &L.wple_proj});
   }
   if (v2) mats.push_back(&m->wple_model);
-  int64_t norm_rows = 0;
   bool ok = gemm_h2_enabled();
-  for (Mat* w : mats) {
-    ok = ok && w->terms == 1 && w->cols % 32 == 0;
-    norm_rows += w->rows;
-  }
-  // largest |w| of each matrix (and of the embedding table), row norms
+  for (Mat* w : mats) ok = ok && w->terms == 1 && w->cols % 32 == 0;
+  // largest |w| of each matrix (and of the embedding table)
   const size_t nm = mats.size();
   DevBuf tmp;
   const size_t head = (2 * (nm + 1) + 63) / 64 * 64;
-  int rc = tmp.ensure(ctx, (head + (size_t)norm_rows) * 4);
-  std::vector<uint32_t> host;
+  int rc = tmp.ensure(ctx, head * 4);
+  std::vector<uint32_t> host(head);
   hipStream_t s = ctx->stream;
   uint32_t* bits = tmp.as<uint32_t>();
-  float* norms = tmp.as<float>() + head;
-  auto run = [&]() -> int {
+  auto largest = [&]() -> int {
     int r;
     if ((r = launch_zero(ctx, bits, head * 4, s))) return r;
-    int64_t at = 0;
-    for (size_t i = 0; i < nm; i++) {
+    for (size_t i = 0; i < nm; i++)
       if ((r = launch_h2_absmax(ctx, mats[i]->p, mats[i]->plane(), bits + i, s))) return r;
-      if ((r = launch_h2_row_norms(ctx, mats[i]->p, mats[i]->rows, mats[i]->cols, norms + at, s))) return r;
-      at += mats[i]->rows;
-    }
     if ((r = launch_h2_absmax(ctx, m->embed.p, m->embed.plane(), bits + nm, s))) return r;
-    host.resize(head + norm_rows);
-    FA_HIP_CHECK(ctx, hipMemcpyAsync(host.data(), tmp.ptr, host.size() * 4, hipMemcpyDeviceToHost, s));
+    FA_HIP_CHECK(ctx, hipMemcpyAsync(host.data(), bits, head * 4, hipMemcpyDeviceToHost, s));
     FA_HIP_CHECK(ctx, hipStreamSynchronize(s));
     return FA_OK;
   };
-  if (!rc) rc = run();
+  if (!rc) rc = largest();
   auto value = [&](size_t i) {
     const uint32_t u = host[i] << 16;
     float f;
@@ -275,65 +325,166 @@ int prepare_h2(fa_model* m) {
       rc = set_error(ctx, FA_ERR_HIP, "gemma: reading the weights' range failed");
     for (uint32_t b : bad) ok = ok && b == 0;
   }
-  // operand bounds (three-plane matrices: of the hi plane, 1 % below theirs at most)
-  const double rd = std::sqrt((double)d);
-  auto gain = [&](const float* dev, int n, double most) -> double {  // max |gain|; infinite: unusable
-    std::vector<float> v(n);
-    if (hipMemcpy(v.data(), dev, (size_t)n * 4, hipMemcpyDeviceToHost) != hipSuccess) return INFINITY;
-    double mx = 0, ss = 0;
-    for (float x : v) {
-      if (!std::isfinite(x)) return INFINITY;
-      mx = std::max(mx, std::fabs((double)x));
-      ss += (double)x * x;
-    }
-    return mx > most * std::sqrt(ss / n) ? INFINITY : mx;
-  };
-  if (!rc) {
-    int64_t at = 0;
-    auto row_max = [&](int64_t r0, int64_t r1, int64_t group, int64_t which) {  // largest norm of the rows
-      double mx = 0;
-      for (int64_t r = r0; r < r1; r++)
-        if (group == 0 || (r / group) % 2 == which) {
-          float f;
-          std::memcpy(&f, &host[head + at + r], 4);
-          if (!std::isfinite(f)) return (double)INFINITY;
-          mx = std::max(mx, (double)f);
-        }
-      return 1.01 * mx;
-    };
-    double xb = value(nm) * 1.01 * rd;  // the residual stream's largest value (variant 2's products read it)
-    m->s_x0 = pow2_for(xb);
-    const double gple = v2 ? gain(m->g_ple_norm, P, 64) * std::sqrt((double)P) : 0;
-    bool tiles = true;
-    for (auto& L : m->layers) {
-      const double nin = rd * gain(L.g_in, d, 64), nffn = rd * gain(L.g_pre_ffn, d, 64);
-      L.s_in = pow2_for(nin);
-      L.s_att = pow2_for(v2 ? std::sqrt((double)L.D) : nin * row_max((int64_t)(H + L.Hkv) * L.D, L.width, 0, 0));
-      if (L.D == 256) {
-        L.s_q = pow2_for(16 * gain(L.g_q, 256, 1024));  // a rotated row keeps its norm
-        L.s_k = pow2_for(16 * gain(L.g_k, 256, 1024));
-        tiles = tiles && L.s_q != 0 && L.s_k != 0 && L.s_att != 0;
-      }
-      at += L.wqkv.rows + L.wo.rows;
-      L.s_ffn = pow2_for(nffn);
-      L.s_gu = pow2_for(nffn * row_max(0, 2LL * F, 32, 0) * nffn * row_max(0, 2LL * F, 32, 1));
-      at += L.wgu.rows + L.wdown.rows;
-      ok = ok && L.s_in != 0 && L.s_att != 0 && L.s_ffn != 0 && L.s_gu != 0;
-      if (v2) {
-        xb += rd * (gain(L.g_post_attn, d, 64) + gain(L.g_post_ffn, d, 64));
-        L.s_x = pow2_for(xb);
-        L.s_ple = pow2_for(row_max(0, P, 0, 0) * xb * rd * gple);
-        at += L.wple_gate.rows + L.wple_proj.rows;
-        xb = (xb + rd * gain(L.g_ple_post, d, 64)) * std::fabs((double)L.scalar);
-        ok = ok && L.s_x != 0 && L.s_ple != 0;
-      }
-    }
-    if (v2) ok = ok && m->s_x0 != 0;
-    m->h2 = ok;
-    m->tiles = tiles;
-  }
   tmp.release();
-  return rc;
+  if (rc) return rc;
+
+  // gains, as absolute values (a non-finite one: no bound, nothing is split)
+  typedef std::vector<float> Vec;
+  bool finite = true;
+  auto gains = [&](const float* dev, int n) {
+    Vec v(n);
+    finite = finite && hipMemcpy(v.data(), dev, (size_t)n * 4, hipMemcpyDeviceToHost) == hipSuccess;
+    for (float& x : v) {
+      finite = finite && std::isfinite(x);
+      x = std::fabs(x);
+    }
+    return v;
+  };
+  auto norm = [](const Vec& v) {
+    double t = 0;
+    for (float x : v) t += (double)x * x;
+    return std::sqrt(t);
+  };
+  auto top = [](const Vec& v) {  // +inf if one is not finite
+    double t = 0;
+    for (float x : v) t = std::isfinite(x) ? std::max(t, (double)x) : INFINITY;
+    return t;
+  };
+  const double rd = std::sqrt((double)d);
+  struct Range {  // a layer's operands: typical sizes, and jobs of the two passes below
+    Vec g_in, g_ffn, g_q, g_k, att, gu, x, xb, ple;
+    int qkv, qkv_g, o, o_t, gu_, gu_g, down, down_t, gate, gate_t, gate_b, proj, proj_t;
+  };
+  std::vector<Range> rs(m->layers.size());
+  RowNorms first, second;
+  const Vec g_ple = v2 ? gains(m->g_ple_norm, P) : Vec();
+  // variant 2's products also read the residual stream: per column, a bound
+  // and the typical square
+  Vec xb(v2 ? d : 0, (float)(value(nm) * 1.01 * rd)), x2(v2 ? d : 0);
+  const int emb = v2 ? first.add(m->embed) : 0, model_w = v2 ? first.add(m->wple_model) : 0;
+  for (size_t l = 0; l < rs.size(); l++) {
+    Layer& L = m->layers[l];
+    Range& r = rs[l];
+    r.g_in = gains(L.g_in, d);
+    r.g_ffn = gains(L.g_pre_ffn, d);
+    r.g_q = gains(L.g_q, L.D);
+    r.g_k = gains(L.g_k, L.D);
+    r.qkv = first.add(L.wqkv);
+    r.qkv_g = first.add(L.wqkv, r.g_in);
+    r.o = first.add(L.wo);
+    r.gu_ = first.add(L.wgu);
+    r.gu_g = first.add(L.wgu, r.g_ffn);
+    r.down = first.add(L.wdown);
+    if (!v2) continue;
+    const Vec ga = gains(L.g_post_attn, d), gf = gains(L.g_post_ffn, d), gp = gains(L.g_ple_post, d);
+    for (int j = 0; j < d; j++) {
+      xb[j] += (float)(rd * (ga[j] + gf[j]));
+      x2[j] += ga[j] * ga[j] + gf[j] * gf[j];
+    }
+    r.xb = xb;
+    for (int j = 0; j < d; j++) r.x.push_back(std::sqrt(x2[j]));
+    const float sc = std::fabs(L.scalar);
+    for (int j = 0; j < d; j++) {
+      xb[j] = (float)((xb[j] + rd * gp[j]) * sc);
+      x2[j] = (x2[j] + gp[j] * gp[j]) * sc * sc;
+    }
+    r.gate = first.add(L.wple_gate);
+    r.gate_t = first.add(L.wple_gate, r.x);
+    r.gate_b = first.add(L.wple_gate, r.xb);
+    r.proj = first.add(L.wple_proj);
+  }
+  if ((rc = first.run(ctx, s))) return rc;
+  if (!finite) return FA_OK;
+  auto out1 = [&](int j) -> const Vec& { return first.jobs[j].out; };
+  for (size_t l = 0; l < rs.size(); l++) {
+    Layer& L = m->layers[l];
+    Range& r = rs[l];
+    const Vec &nv = out1(r.qkv_g), &ng = out1(r.gu_g);
+    L.s_in = pow2_for(rd * top(r.g_in));
+    L.s_ffn = pow2_for(rd * top(r.g_ffn));
+    double att = v2 ? std::sqrt((double)L.D) : 0, gu = 0;
+    for (int h = 0; h < H; h++)
+      for (int i = 0; i < L.D; i++) {
+        const float n = v2 ? 1.f : nv[(size_t)(H + L.Hkv + h / (H / L.Hkv)) * L.D + i];
+        if (!v2) att = std::isfinite(n) ? std::max(att, 1.01 * rd * n) : INFINITY;
+        r.att.push_back(n / 32);
+      }
+    for (int f = 0; f < F; f++) {
+      const int64_t row = f / 32 * 64 + f % 32;  // gate rows first in each 64-row group, then up
+      const double p = (double)ng[row] * ng[row + 32];
+      gu = std::isfinite(p) ? std::max(gu, 1.02 * d * p) : INFINITY;
+      r.gu.push_back((float)(p / 4));
+    }
+    L.s_att = pow2_for(att);
+    L.s_gu = pow2_for(gu);
+    r.o_t = second.add(L.wo, r.att);
+    r.down_t = second.add(L.wdown, r.gu);
+    if (!v2) continue;
+    double ple = 0;
+    for (int p = 0; p < P; p++) {
+      const double b = rd * out1(r.gate_b)[p] * std::sqrt((double)P) * g_ple[p];  // sum |w x| <= sqrt(d) |w o xb|
+      ple = std::isfinite(b) ? std::max(ple, 1.01 * b) : INFINITY;
+      r.ple.push_back(out1(r.gate_t)[p] * g_ple[p] / 4);
+    }
+    L.s_x = pow2_for(top(r.xb));
+    L.s_ple = pow2_for(ple);
+    r.proj_t = second.add(L.wple_proj, r.ple);
+  }
+  if ((rc = second.run(ctx, s))) return rc;
+  auto out2 = [&](int j) -> const Vec& { return second.jobs[j].out; };
+
+  // whether a product whose operand carries scale a and has typical sizes t
+  // holds the limit in every row: plain and typical row norms n, nt
+  auto holds = [&](const Mat& w, const Vec& n, const Vec& nt, const Vec& t, float a) {
+    if (a == 0.f) return false;
+    const double act = 0x1p-36 / a, wt = 0x1p-25 / w.h_scale * norm(t);
+    for (size_t i = 0; i < n.size(); i++)
+      if (nt[i] != 0.f && !(act * n[i] + wt <= 0x1p-28 * nt[i])) return false;
+    return true;
+  };
+  bool tiles = true;
+  for (size_t l = 0; l < rs.size(); l++) {
+    Layer& L = m->layers[l];
+    const Range& r = rs[l];
+    ok = ok && holds(L.wqkv, out1(r.qkv), out1(r.qkv_g), r.g_in, L.s_in) &&
+         holds(L.wo, out1(r.o), out2(r.o_t), r.att, L.s_att) &&
+         holds(L.wgu, out1(r.gu_), out1(r.gu_g), r.g_ffn, L.s_ffn) &&
+         holds(L.wdown, out1(r.down), out2(r.down_t), r.gu, L.s_gu);
+    if (v2)
+      ok = ok && holds(L.wple_gate, out1(r.gate), out1(r.gate_t), r.x, L.s_x) &&
+           holds(L.wple_proj, out1(r.proj), out2(r.proj_t), r.ple, L.s_ple);
+    if (L.D != 256) continue;
+    // a rotated row keeps its norm; its dims j and j + 128 share their gains
+    L.s_q = pow2_for(16 * top(r.g_q));
+    L.s_k = pow2_for(16 * top(r.g_k));
+    if (L.s_q == 0 || L.s_k == 0 || L.s_att == 0) {
+      tiles = false;
+      continue;
+    }
+    double qq = 0, kk = 0, qk = 0;
+    for (int j = 0; j < 128; j++) {
+      const double q2 = (double)r.g_q[j] * r.g_q[j] + (double)r.g_q[j + 128] * r.g_q[j + 128];
+      const double k2 = (double)r.g_k[j] * r.g_k[j] + (double)r.g_k[j + 128] * r.g_k[j + 128];
+      qq += q2;
+      kk += k2;
+      qk += q2 * k2 / 2;
+    }
+    tiles = tiles && 0x1p-25 * (std::sqrt(kk) / L.s_q + std::sqrt(qq) / L.s_k) <= 0x1p-26 * std::sqrt(qk);
+    for (size_t i = 0; i < out1(r.o).size(); i++)  // (the values are not averaged yet: 32 r.att)
+      tiles = tiles && (out2(r.o_t)[i] == 0.f || 0x1p-25 / L.s_att * out1(r.o)[i] <= 0x1p-26 * 32 * out2(r.o_t)[i]);
+  }
+  if (v2) {
+    // the embeddings as an operand: a token's values have rms |its row|, and
+    // its result is normed, so the least row sets the limit
+    m->s_x0 = pow2_for(value(nm) * 1.01 * rd);
+    float least = INFINITY;
+    for (float n : out1(emb))
+      if (n != 0.f) least = std::min(least, n);
+    ok = ok && (least == INFINITY || holds(m->wple_model, out1(model_w), out1(model_w), Vec(d, 1.f), m->s_x0 * least));
+  }
+  m->h2 = ok;
+  m->tiles = tiles;
+  return FA_OK;
 }
 
 // Fills the operands of a product on split activations: A scaled by a_scale.

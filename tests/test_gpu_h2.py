@@ -2,7 +2,13 @@
 edges of their tiles, against the float64 restatement of the encoder: one row
 (the few-row kernel), row counts around 32, 64 and 128, a batch in
 micro-batches, widths that leave the column tiles partly empty; and models
-whose weights or gains keep them on the three-term products."""
+whose weights or gains are of very uneven ranges, on the split operands or,
+where those would lose bits, on the three-term products and the fp32
+attention."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -12,6 +18,8 @@ from ai_amd import synth as S
 from test_oracle import f64_encoder
 
 pytestmark = pytest.mark.gpu
+
+HERE = os.path.dirname(os.path.abspath(__file__))
 
 # float32 sums of at most 512 terms through two layers: every other layer
 # test of this suite holds hidden rows to 1e-5
@@ -34,7 +42,7 @@ def weights(sh, edit=None):
     return ws
 
 
-def check(sh, ws, lengths):
+def run(sh, ws, lengths):
     lengths = np.array(lengths, np.int32)
     r = np.random.default_rng(5)
     ids = np.zeros((len(lengths), int(lengths.max())), np.int32)
@@ -47,6 +55,11 @@ def check(sh, ws, lengths):
         m.finalize()
         got = m.encode_ids(ids, lengths)
         m.close()
+    return got, ids, lengths
+
+
+def check(sh, ws, lengths):
+    got, ids, lengths = run(sh, ws, lengths)
     states = []
     f64_encoder(sh, ws, ids, lengths, states=states)
     want = np.concatenate([s[-1] for s in states])
@@ -69,7 +82,95 @@ def outlier_gain(ws):  # one gain 1 000 times the others
     ws["layers.1.pre_feedforward_layernorm.weight"][7] = 1000.0
 
 
-@pytest.mark.parametrize("edit", [tiny_weight, outlier_gain])
-def test_models_outside_the_split_range(edit):
+def gain_for_weights(ws):  # a gain of 2^12 and columns that make up for it: the layer computes what it did
+    gain_and_columns(ws, 12)
+
+
+def gain_and_columns(ws, e):
+    g = "layers.0.pre_feedforward_layernorm.weight"
+    ws[g][7] = 2.0 ** e - 1  # the factor is 1 + w
+    for n in ("gate", "up"):
+        ws[f"layers.0.mlp.{n}_proj.weight"][:, 7] *= 2.0 ** -e
+
+
+def uneven_features(ws):  # and gate and up rows 64 times the others, their down columns a 64th
+    gain_and_columns(ws, 10)
+    for n, f in (("gate", 3), ("up", 5)):
+        ws[f"layers.0.mlp.{n}_proj.weight"][f] *= 64
+        ws["layers.0.mlp.down_proj.weight"][:, f] /= 64
+
+
+def very_uneven_features(ws):  # one feature 2^20 times the others
+    for n in ("gate", "up"):
+        ws[f"layers.0.mlp.{n}_proj.weight"][3] *= 2.0 ** 10
+    ws["layers.0.mlp.down_proj.weight"][:, 3] *= 2.0 ** -20
+
+
+@pytest.mark.parametrize("edit", [tiny_weight, outlier_gain, gain_for_weights, uneven_features, very_uneven_features])
+def test_models_of_uneven_ranges(edit):
+    """Weights and gains of very different sizes, also where they make up for
+    each other: on the split products or the three-term ones, as accurate."""
     sh = shape(256, 96)
     check(sh, weights(sh, edit), [40, 3])
+
+
+def uneven_gains(ws):  # spread over a factor of some hundreds (q and k: of the usual size in the mean)
+    r = np.random.default_rng(8)
+    for n, w in ws.items():
+        if w.ndim == 1:
+            g = np.exp(1.2 * r.standard_normal(w.shape))
+            w[:] = (g / np.sqrt((g * g).mean()) if "self_attn" in n else g) - 1
+
+
+def value_row(ws):  # a value dimension 2^20 times the others, its output columns make up for it
+    for l in (0, 1):
+        ws[f"layers.{l}.self_attn.v_proj.weight"][9] *= 2.0 ** 20
+        ws[f"layers.{l}.self_attn.o_proj.weight"][:, [9, 256 + 9]] *= 2.0 ** -20
+
+
+def query_gains(ws):  # a rotated pair of query gains 2^20 times the others, the key gains make up for it
+    for l in (0, 1):
+        for j in (7, 135):
+            ws[f"layers.{l}.self_attn.q_norm.weight"][j] = 2.0 ** 20 - 1
+            ws[f"layers.{l}.self_attn.k_norm.weight"][j] = 2.0 ** -20 - 1
+
+
+@pytest.mark.parametrize("edit", [None, uneven_gains, value_row, query_gains])
+def test_tile_attention_of_uneven_ranges(edit):
+    """More than 1 024 tokens: the tile attention, or the fp32 one where an
+    operand's range leaves its terms too few bits."""
+    sh = shape(256, 96)
+    check(sh, weights(sh, edit), [300, 300, 300, 290])
+
+
+ROUTE = """
+import sys
+sys.path[:0] = [{root!r}, {tests!r}]
+import numpy as np
+import test_gpu_h2 as t
+sh = t.shape(256, 96)
+out = [t.run(sh, t.weights(sh, getattr(t, e) if e else None), n)[0] for e in {edits!r} for n in ([40, 3], [300, 300, 300, 290])]
+np.savez({path!r}, *out)
+"""
+
+
+def test_routes(tmp_path):
+    """Which models run on the split operands: the bits are those of the
+    three-term products and the fp32 attention for models outside the range,
+    and others for ordinary and mildly uneven ones. (An environment variable
+    keeps a program on the three-term products, another on the fp32 attention.)"""
+    edits = ["", "uneven_gains", "gain_for_weights", "tiny_weight", "very_uneven_features", "value_row", "query_gains"]
+    got = []
+    for env in ({}, {"FA_GEMM_H2": "0"}, {"FA_TILE_MIN_ROWS": "1000000"}):
+        path = str(tmp_path / f"{len(got)}.npz")
+        code = ROUTE.format(root=os.path.dirname(HERE), tests=HERE, edits=edits, path=path)
+        subprocess.run([sys.executable, "-c", code], check=True, env={**os.environ, **env}, timeout=100)
+        f = np.load(path)
+        got.append([f[k] for k in f.files])
+    split, three, fp32 = got
+    for i, e in enumerate(edits):
+        on_split = not np.array_equal(split[2 * i], three[2 * i])
+        on_tiles = not np.array_equal(split[2 * i + 1], fp32[2 * i + 1])
+        print(e, on_split, on_tiles, flush=True)
+        assert on_split == (e not in ("tiny_weight", "very_uneven_features", "value_row")), e
+        assert on_tiles == (e not in ("value_row", "query_gains")), e
