@@ -26,6 +26,7 @@ BUILD = os.path.join(ROOT, "_build")
 INCLUDE = os.path.join(ROOT, "include")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+ROCM_LIB = os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "lib")
 ARCH = "gfx950"
 
 # Packed-FP32 instructions are disabled for device code (they are generated
@@ -89,6 +90,7 @@ CPP_CPU_TESTS = ["test_tokenizer", "test_config", "test_plan"]  # need no GPU
 CPP_PLAN_TEST = "test_plan"  # the encoder's host plan (csrc/plan.cpp) alone, no library
 CPP_DRIVERS = ["st_dump", "embed_dir"]  # programs the Python tests drive
 C_DRIVERS = ["exit_open"]  # C programs the Python tests drive
+C_SHIMS = ["fail_malloc"]  # libraries the Python tests load before libfa_rocm.so
 CPP_TEST_BIN = os.path.join(BUILD, "cpp_tests")
 
 
@@ -116,6 +118,10 @@ def build_host(verbose: bool = False) -> str:
     for t in C_DRIVERS:  # plain C callers of the C ABI
         jobs.append([cc, "-O2", "-std=c99", "-Wall", "-I", INCLUDE, os.path.join(tdir, t + ".c"),
                      "-o", os.path.join(CPP_TEST_BIN, t), "-L", LIB, "-lfa_rocm", "-lfa_synth", rpath])
+    for t in C_SHIMS:
+        jobs.append([cc, "-O2", "-std=c99", "-Wall", "-fPIC", "-shared", os.path.join(tdir, t + ".c"),
+                     "-o", os.path.join(CPP_TEST_BIN, f"lib{t}.so"), "-L", ROCM_LIB, "-Wl,--no-as-needed", "-lamdhip64",
+                     f"-Wl,-rpath,{ROCM_LIB}", "-ldl"])
     with cf.ThreadPoolExecutor(len(jobs)) as ex:
         for f in [ex.submit(_run, j, verbose) for j in jobs]:
             f.result()

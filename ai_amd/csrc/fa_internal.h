@@ -204,7 +204,7 @@ bool gemm_h2_enabled();
 // caller) becomes the largest |w| as bf16 bits; norms[r] the 2-norm of row r (its
 // columns weighted by t unless that is null);
 // dst = fp16(w * scale), *bad (zeroed by the caller) nonzero when one of them
-// is not exact.
+// is not exact (either may be null).
 int launch_h2_absmax(fa_ctx* ctx, const uint16_t* w, int64_t n, uint32_t* max_bits, hipStream_t s);
 int launch_h2_row_norms(fa_ctx* ctx, const uint16_t* w, int64_t rows, int64_t cols, const float* t, float* norms,
                         hipStream_t s);

@@ -408,9 +408,9 @@ __global__ __launch_bounds__(256) void h2_convert_kernel(const uint16_t* __restr
     const float x = __uint_as_float((uint32_t)w[i] << 16) * scale;
     const _Float16 h = (_Float16)x;
     off |= (float)h != x;
-    dst[i] = __builtin_bit_cast(uint16_t, h);
+    if (dst) dst[i] = __builtin_bit_cast(uint16_t, h);
   }
-  if (off) atomicOr(bad, 1u);
+  if (bad && off) atomicOr(bad, 1u);
 }
 
 // ---- launches -----------------------------------------------------------------

@@ -259,14 +259,13 @@ struct RowNorms {
 // Models that do not hold this keep the three-term products, or the fp32
 // attention, as do those with non-finite weights; the products also need
 // every layer matrix bf16-exact (terms == 1) and exact in fp16 after one power
-// of two for the matrix (its largest value just below 2^15).
-int prepare_h2(fa_model* m) {
-  m->h2 = m->tiles = false;
+// of two for the matrix (its largest value just below 2^15). Only then are the
+// fp16 copies made.
+int range_h2(fa_model* m, std::vector<Mat*>& mats) {
   fa_ctx* ctx = m->ctx;
   const fa_gemma_config& c = m->cfg;
   const bool v2 = m->variant == 2;
   const int d = c.hidden_size, H = c.num_attention_heads, F = c.intermediate_size, P = m->P;
-  std::vector<Mat*> mats;
   for (auto& L : m->layers) {
     mats.insert(mats.end(), {&L.wqkv, &L.wo, &L.wgu, &L.wdown});
     if (v2) mats.insert(mats.end(), {&L.wple_gate, &L.wple_proj});
@@ -310,12 +309,7 @@ int prepare_h2(fa_model* m) {
     const float mx = value(i);
     mats[i]->h_scale = mx == 0.f ? 1.f : pow2_for(mx);
     ok = mats[i]->h_scale != 0.f;
-    if (ok && !mats[i]->h) {
-      void* np = nullptr;
-      if ((rc = alloc_dev(m, (size_t)mats[i]->plane() * 2, &np))) break;
-      mats[i]->h = (uint16_t*)np;
-    }
-    if (ok) rc = launch_h2_convert(ctx, mats[i]->p, mats[i]->plane(), mats[i]->h_scale, mats[i]->h, bits + nm + 1 + i, s);
+    if (ok) rc = launch_h2_convert(ctx, mats[i]->p, mats[i]->plane(), mats[i]->h_scale, nullptr, bits + nm + 1 + i, s);
     if (rc) ok = false;
   }
   if (ok) {
@@ -482,9 +476,38 @@ int prepare_h2(fa_model* m) {
       if (n != 0.f) least = std::min(least, n);
     ok = ok && (least == INFINITY || holds(m->wple_model, out1(model_w), out1(model_w), Vec(d, 1.f), m->s_x0 * least));
   }
-  m->h2 = ok;
   m->tiles = tiles;
+  if (!ok) return FA_OK;
+  for (Mat* w : mats) {
+    if (!w->h) {
+      void* np = nullptr;
+      if ((rc = alloc_dev(m, (size_t)w->plane() * 2, &np))) return rc;
+      w->h = (uint16_t*)np;
+    }
+    if ((rc = launch_h2_convert(ctx, w->p, w->plane(), w->h_scale, w->h, nullptr, s))) return rc;
+  }
+  FA_HIP_CHECK(ctx, hipStreamSynchronize(s));
+  m->h2 = true;
   return FA_OK;
+}
+
+// The copies are for speed: where they, or the scratch of the checks, find no
+// memory, the model keeps the three-term products of the matrices it holds.
+int prepare_h2(fa_model* m) {
+  m->h2 = m->tiles = false;
+  std::vector<Mat*> mats;
+  int rc = range_h2(m, mats);
+  if (rc == FA_ERR_OOM) {
+    (void)hipGetLastError();
+    rc = FA_OK;
+  }
+  if (!m->h2)
+    for (Mat* w : mats)
+      if (w->h) {
+        free_dev(m, w->h);
+        w->h = nullptr;
+      }
+  return rc;
 }
 
 // Fills the operands of a product on split activations: A scaled by a_scale.

@@ -75,7 +75,7 @@ def test_split_products_at_tile_edges(hidden, ffn, lengths):
 
 
 def tiny_weight(ws):  # 2^-60 beside values near 0.1: no power of two makes both exact in fp16
-    ws["layers.0.self_attn.o_proj.weight"][3, 5] = 2.0 ** -60
+    ws["layers.1.mlp.down_proj.weight"][3, 5] = 2.0 ** -60
 
 
 def outlier_gain(ws):  # one gain 1 000 times the others
@@ -174,3 +174,59 @@ def test_routes(tmp_path):
         print(e, on_split, on_tiles, flush=True)
         assert on_split == (e not in ("tiny_weight", "very_uneven_features", "value_row")), e
         assert on_tiles == (e not in ("value_row", "query_gains")), e
+
+
+MEMORY = """
+import sys
+sys.path[:0] = [{root!r}, {tests!r}]
+import ctypes as C
+import numpy as np
+shim = C.CDLL({shim!r}, C.RTLD_GLOBAL)
+fail_from, failed = C.c_size_t.in_dll(shim, "fail_from"), C.c_int.in_dll(shim, "failed")
+import test_gpu_h2 as t
+from ai_amd import _native as N, gemma as G
+hip = C.CDLL("libamdhip64.so")
+free, total = C.c_size_t(), C.c_size_t()
+
+def used():
+    hip.hipMemGetInfo(C.byref(free), C.byref(total))
+    return total.value - free.value
+
+sh = t.shape(512, 6144)  # layer matrices of 43 MB in all
+ids, lengths = np.full((2, 40), 7, np.int32), np.array([40, 25], np.int32)
+out, grown, fails = [], [], []
+with N.Context(0) as ctx:
+    for edit, limit in ((None, 0), (None, 1), (None, 4 << 20), (t.tiny_weight, 0)):
+        m = G.Model(sh, ctx)
+        for name, w in t.weights(sh, edit).items():
+            m.set_weight(name, w)
+        before, failed.value, fail_from.value = used(), 0, limit
+        m.finalize()
+        fails.append(failed.value)
+        fail_from.value = 0
+        grown.append(used() - before)
+        out.append(m.encode_ids(ids, lengths))
+        m.close()
+np.savez({path!r}, grown, fails, *out)
+"""
+
+
+def test_memory_of_the_copies(tmp_path):
+    """finalize without memory for the fp16 copies, or for anything at all, keeps
+    the three-term products (their bits) and no memory; so does a model whose
+    last matrices are not exact in fp16."""
+    got = []
+    for env in ({}, {"FA_GEMM_H2": "0", "FA_TILE_MIN_ROWS": "1000000"}):
+        path = str(tmp_path / f"m{len(got)}.npz")
+        shim = os.path.join(os.path.dirname(HERE), "_build", "cpp_tests", "libfail_malloc.so")
+        code = MEMORY.format(root=os.path.dirname(HERE), tests=HERE, shim=shim, path=path)
+        subprocess.run([sys.executable, "-c", code], check=True, env={**os.environ, **env}, timeout=100)
+        f = np.load(path)
+        got.append([f[k] for k in f.files])
+    (grown, fails, *split), (_, _, *three) = got
+    print(grown, fails, flush=True)
+    assert fails[1] > 0 and fails[2] > 0 and fails[0] == fails[3] == 0
+    assert not np.array_equal(split[0], three[0]) and grown[0] > 35e6
+    for i in (1, 2, 3):
+        assert np.array_equal(split[i], three[i]), i
+        assert grown[i] < 4e6, grown
