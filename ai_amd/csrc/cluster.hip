@@ -697,14 +697,28 @@ int launch_sim(fa_ctx* ctx, const float* x, int64_t n, const float* c, int64_t k
   return launch_gemm(ctx, g, ctx->stream);
 }
 
-// assign, simil of every row: fused, or (more than 64 centres, other widths or
-// alignments) the product into sim [n x k] and the argmax of its rows.
-bool nearest_fused_ok(const float* x, const float* c, int64_t k, int d) {
-  return k <= kNearMax && d % 8 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(c)) & 15) == 0;
+// assign, simil of every row: fused, or the product into sim [n x k] and the
+// argmax of its rows, for more than 64 centres, other widths or alignments, and
+// where it is the faster one: up to a round of its 64-row tiles (the fused
+// kernel's 128-row workgroups leave half the CUs idle there), and with two
+// blocks of centres where those fill an odd number of rounds, so that the fused
+// kernel's last one is at most half full, until the bytes of the similarities
+// weigh more. Us at 768 columns, product and fused: 40 centres, 1 000 rows 21 and
+// 34, 16 000: 26 and 35, 28 000: 40 and 36, 42 000: 55 and 64, 50 000: 70 and 64,
+// 80 000: 90 and 94, 200 000: 404 and 227; 4 centres, 1 000: 21 and 23, 28 000: 40
+// and 24. At 256: 40 centres, 1 000: 11 and 15, 42 000: 29 and 26; 4 centres 11
+// and 10.
+bool nearest_fused_ok(fa_ctx* ctx, const float* x, int64_t n, const float* c, int64_t k, int d) {
+  if (k > kNearMax || d % 8 != 0 || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(c)) & 15) != 0)
+    return false;
+  const int64_t round = 64LL * (ctx->cu_count > 0 ? ctx->cu_count : 256);
+  if (k <= 32 && d <= 256) return true;
+  if (n <= round) return false;
+  return k <= 32 || d <= 256 || (n - 1) / round % 2 == 1 || n > 8 * round;
 }
 int launch_nearest(fa_ctx* ctx, const float* x, int64_t n, const float* c, int64_t k, int d, float* sim,
                    int32_t* assign, float* simil) {
-  if (nearest_fused_ok(x, c, k, d)) {
+  if (nearest_fused_ok(ctx, x, n, c, k, d)) {
     const dim3 grid((unsigned)((n + 127) / 128)), block(256);
     if (k <= 32) hipLaunchKernelGGL(nearest_kernel<1>, grid, block, 0, ctx->stream, x, n, d, c, (int)k, assign, simil);
     else hipLaunchKernelGGL(nearest_kernel<2>, grid, block, 0, ctx->stream, x, n, d, c, (int)k, assign, simil);
@@ -772,7 +786,7 @@ int fa_cluster_nearest_dev(fa_ctx* ctx, const float* x, int64_t n, const float* 
   }
   FA_HIP_CHECK(ctx, hipSetDevice(ctx->device));
   fa::DevBuf& ws = ctx->slot(S_CL_WORK);
-  if (!fa::nearest_fused_ok(x, centres, k, d) && (rc = ws.ensure(ctx, (size_t)n * k * 4))) return rc;
+  if (!fa::nearest_fused_ok(ctx, x, n, centres, k, d) && (rc = ws.ensure(ctx, (size_t)n * k * 4))) return rc;
   return fa::launch_nearest(ctx, x, n, centres, k, d, ws.as<float>(), index, similarity);
 }
 
@@ -833,7 +847,7 @@ int fa_cluster_kmeans_dev(fa_ctx* ctx, const float* x, int64_t n, int32_t d, int
     return o;
   };
   const size_t o_raw = take((size_t)k * d * 4), o_sums = take((size_t)k * d * 4), o_best = take((size_t)n * 4),
-               o_w = take((size_t)n * 8), o_part = take((size_t)nparts * 8), o_sim = take(fa::nearest_fused_ok(x, centres, k, d) ? 0 : (size_t)n * k * 4),
+               o_w = take((size_t)n * 8), o_part = take((size_t)nparts * 8), o_sim = take(fa::nearest_fused_ok(ctx, x, n, centres, k, d) ? 0 : (size_t)n * k * 4),
                o_cnt = take((size_t)nchunks * k * 4), o_chg = take((size_t)nchunks * 4), o_offs = take((size_t)k * 4),
                o_list = take((size_t)n * 4), o_prev = take((size_t)n * 4), o_summary = take(((size_t)k + 1) * 4),
                o_chosen = take((size_t)k * 4);

@@ -9,12 +9,14 @@ through products that differ by rounding); KMeans on rows with one nonzero
 dyadic coordinate (every step exact, empty-centre restarts included)
 bit-identical.
 """
+import ctypes as C
 import time
 
 import numpy as np
 import pytest
 
 import oracle_lib as O
+from ai_amd import _native as N
 from ai_amd import cluster as CL
 from ai_amd.tensor import TensorError
 
@@ -175,10 +177,11 @@ def test_nearest_and_kmeans_speed():
 
 
 @pytest.mark.parametrize("n,k,d", [(1, 1, 16), (31, 2, 8), (127, 16, 120), (129, 32, 128), (300, 33, 136), (513, 49, 264),
-                                   (1000, 64, 768)])
+                                   (1000, 64, 768), (16413, 33, 136), (17000, 49, 264), (16400, 64, 768)])
 def test_nearest_fused_edges(n, k, d):
     """The fused product and argmax at the edges of its 32-row and 32-centre
-    blocks and 128-column parts. Entries are small integers: every similarity
+    blocks and 128-column parts (more than 32 centres, or more than 256 columns:
+    from 16 385 rows; the product and the argmax of its rows below). Entries are small integers: every similarity
     is exact and ties are frequent (the first index wins); a NaN row takes
     centre 0, a NaN centre is never taken except as index 0 (the rule of
     Argmax, tensor/reduce.go:269-297)."""
@@ -205,3 +208,35 @@ def test_kmeans_group_edges(n, k):
     got, want = CL.KMeans(x, k, 10, 5), O.cluster_kmeans(x, k, 10, 5)
     assert np.array_equal(got.Assignment, want["assignment"]) and np.array_equal(got.Sizes, want["sizes"])
     np.testing.assert_allclose(got.Centres, want["centres"], rtol=0, atol=1e-5)
+
+
+@pytest.mark.parametrize("n,d", [(500, 768), (16000, 768), (2000, 128), (33000, 768), (200, 2048)])
+def test_nearest_no_slower_than_with_one_more_centre(n, d):
+    """64 centres, which the fused kernel could take, against 65, which it could
+    not: where it would be the slower one it is not used."""
+    rng = np.random.default_rng(n)
+    L = N.lib()
+    with N.Context(0) as ctx:
+        ptrs = []
+        for a in (rng.standard_normal((n, d)).astype(np.float32), rng.standard_normal((65, d)).astype(np.float32),
+                  np.empty(n, np.int32), np.empty(n, np.float32)):
+            p = C.c_void_p()
+            N.check(ctx.h, L.fa_device_alloc(ctx.h, a.nbytes, C.byref(p)))
+            N.check(ctx.h, L.fa_memcpy_h2d(ctx.h, p, a.ctypes.data, a.nbytes))
+            ptrs.append(p)
+
+        def best(k):
+            t = []
+            for _ in range(8):
+                ctx.sync()
+                t0 = time.perf_counter()
+                for _ in range(20):
+                    N.check(ctx.h, L.fa_cluster_nearest_dev(ctx.h, ptrs[0], n, ptrs[1], k, d, ptrs[2], ptrs[3]))
+                ctx.sync()
+                t.append(time.perf_counter() - t0)
+            return min(t)
+
+        best(65)
+        assert best(64) <= 1.15 * best(65)
+        for p in ptrs:
+            L.fa_device_free(ctx.h, p)
