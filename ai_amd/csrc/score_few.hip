@@ -332,9 +332,10 @@ __global__ __launch_bounds__(64 * kFewMergeWaves) void score_few_merge_kernel(co
   }
 }
 
-// Documents per workgroup: the fewest (16, 32, ... 512) that leave at most
-// about four workgroups per CU, so that a small corpus still spreads over
-// the CUs and a large one gives each wave whole blocks.
+// Documents per workgroup: the fewest of 16, 32, 64 and 128 that leave at most
+// about four workgroups per CU, so that a small corpus still spreads over the
+// CUs; from 65 537 documents on 128, a whole block for each wave, and the
+// workgroups (and the candidates of the merge) grow with the corpus.
 int few_docs(int64_t nd) {
   int per = 16;
   while (per < kFewMaxDocs && (nd + per - 1) / per > 1024) per *= 2;
@@ -345,11 +346,29 @@ size_t few_lds(int nq, int d, int k) { return (size_t)nq * (((size_t)d + 4 + kFe
 
 }  // namespace
 
+// Where the streaming pass is not the faster one, though it could run: its
+// merge reads the candidates, k of every 128 documents, with one workgroup per
+// query (0.5 to 1.5 us per thousand, more with more queries), which rows of at
+// least 256 columns hide behind their own bytes; and more than 16 queries
+// against a handful of documents pay for a second query block. Us, product and
+// streaming: 2 000 000 x 64, 32 queries, k = 32: 528 and 1 014; the same of one
+// query: 483 and 533, k = 1: 396 and 335; 500 000 x 64, 16 queries, k = 32: 205 and
+// 172, 32 queries: 211 and 235; 6 000 000 x 16, 16 queries, k = 10: 970 and 1 044;
+// 2 000 000 x 128, 32 queries, k = 10: 701 and 650, k = 32: 770 and 1 072; 500 000 x
+// 256, 32 queries, k = 32: 410 and 288; 50 x 128, 32 queries, k = 1: 15 and 19,
+// k = 10: 19 and 20, 300 documents, k = 10: 27 and 21.
+static bool score_few_pays(int64_t nq, int64_t nd, int d, int topk) {
+  if (nq >= 16 && topk < 4 && nd < 256 && d < 512) return false;
+  const int64_t cands = (nd + kFewMaxDocs - 1) / kFewMaxDocs * topk;
+  return d >= 256 || cands <= (d >= 128 ? 200000 : nq <= 16 ? 128000 : 40000);
+}
+
 bool score_few_ok(const float* q, int64_t nq, const float* docs, int64_t nd, int d, int topk) {
   return nq >= 1 && nq <= kScoreFewMax && topk >= 1 && topk <= 32 && d % 16 == 0 &&
          ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(docs)) & 15) == 0 &&
          few_lds((int)nq, d, topk) <= 150 * 1024 &&
-         (nd + kFewMaxDocs - 1) / kFewMaxDocs * topk < (1LL << 30) && nd <= INT32_MAX;
+         (nd + kFewMaxDocs - 1) / kFewMaxDocs * topk < (1LL << 30) && nd <= INT32_MAX &&
+         score_few_pays(nq, nd, d, topk);
 }
 
 size_t score_few_scratch(int64_t nq, int64_t nd, int topk) {

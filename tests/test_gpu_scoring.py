@@ -8,6 +8,9 @@ dot products rounded to float32: the expected lists are the float64 products
 rounded to float32, ordered by (value desc, index asc), with NaN scores below
 every number and index -1 past a row's non-NaN scores.
 """
+import ctypes as C
+import time
+
 import numpy as np
 import pytest
 
@@ -169,3 +172,36 @@ def test_few_queries_all_equal(nd):
     with N.Context(0) as ctx:
         N.check(ctx.h, N.lib().fa_similarities_topk(ctx.h, N.ptr(q), 3, N.ptr(docs), nd, 32, 10, N.ptr(idx), N.ptr(val)))
     assert np.array_equal(idx, np.tile(np.arange(10), (3, 1))) and (val == 32).all()
+
+
+@pytest.mark.parametrize("nd,d,k", [(2_000_000, 64, 32), (6_000_000, 16, 10), (2_000_000, 128, 32), (50, 128, 1),
+                                    (100, 64, 1), (20000, 768, 10)])
+def test_few_queries_no_slower_than_one_more(nd, d, k):
+    """32 queries, which the streaming pass could take, against 33, which it
+    could not: where it would be the slower one it is not used."""
+    L = N.lib()
+    r = np.random.default_rng(d)
+    with N.Context(0) as ctx:
+        ptrs = []
+        for a in (r.standard_normal((33, d)).astype(np.float32), r.standard_normal((nd, d), dtype=np.float32),
+                  np.empty((33, k), np.int32), np.empty((33, k), np.float32)):
+            p = C.c_void_p()
+            N.check(ctx.h, L.fa_device_alloc(ctx.h, a.nbytes, C.byref(p)))
+            N.check(ctx.h, L.fa_memcpy_h2d(ctx.h, p, a.ctypes.data, a.nbytes))
+            ptrs.append(p)
+
+        def best(nq):
+            t = []
+            for _ in range(8):
+                ctx.sync()
+                t0 = time.perf_counter()
+                for _ in range(5):
+                    N.check(ctx.h, L.fa_similarities_topk_dev(ctx.h, ptrs[0], nq, ptrs[1], nd, d, k, ptrs[2], ptrs[3]))
+                ctx.sync()
+                t.append(time.perf_counter() - t0)
+            return min(t)
+
+        best(33)
+        assert best(32) <= 1.15 * best(33)
+        for p in ptrs:
+            L.fa_device_free(ctx.h, p)
