@@ -264,7 +264,10 @@ template <Epi EPI, bool SPLIT, int NB>
 __global__ __launch_bounds__(kSmallNW * 64) void gemm_h2_small_kernel(H2Params p) {
   static_assert(NB == 2 || (NB == 1 && EPI == Epi::GeGLU), "narrow tiles: GeGLU only");
   constexpr int NW = kSmallNW;
-  __shared__ __attribute__((aligned(16))) float red[NW][NB][16][64];
+  // the waves' partial tiles: with two column blocks four rows of a lane beside
+  // each other (16-byte accesses), with one a row at a time
+  constexpr int RV = NB == 2 ? 4 : 1;
+  __shared__ __attribute__((aligned(16))) float red[NW][NB][16 / RV][64][RV];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t M = p.m, N = p.n;
   const int64_t m0 = (int64_t)(blockIdx.x / p.tiles_n) * 32;
@@ -333,7 +336,7 @@ __global__ __launch_bounds__(kSmallNW * 64) void gemm_h2_small_kernel(H2Params p
 #pragma unroll
   for (int j = 0; j < NB; j++)
 #pragma unroll
-    for (int r = 0; r < 16; r++) red[wave][j][r][lane] = acc[j][r] + low[j][r];
+    for (int r = 0; r < 16; r++) red[wave][j][r / RV][lane][r % RV] = acc[j][r] + low[j][r];
   __syncthreads();
 
   // C element (j, r, l): row 8*(r/4) + 4*(l/32) + r%4, column 32*j + l%32.
@@ -343,34 +346,42 @@ __global__ __launch_bounds__(kSmallNW * 64) void gemm_h2_small_kernel(H2Params p
   if constexpr (EPI == Epi::GeGLU) {
     const int64_t F = N / 2;
     constexpr int FW = NB == 1 ? 16 : 32;  // features of the tile
-    static_assert(16 * 2 * FW % 512 == 0 && NW * 64 == 512, "whole steps");
+    constexpr int V = NB;                  // rows per thread
+    static_assert(16 * 2 * FW == V * NW * 64, "one step");
+    const int r0 = tid / (2 * FW) * V, lq = tid % (2 * FW);
+    const int l = (lq % FW) + (lq / FW) * 32;  // gate lane; its up value: lane + 16 of block 0, or block 1
+    float g[V], u[V];
 #pragma unroll
-    for (int e = tid; e < 16 * 2 * FW; e += NW * 64) {
-      const int r = e / (2 * FW), lq = e % (2 * FW);
-      const int l = (lq % FW) + (lq / FW) * 32;  // gate lane; its up value: lane + 16 of block 0, or block 1
-      float g = 0.f, u = 0.f;
+    for (int i = 0; i < V; i++) g[i] = u[i] = 0.f;
 #pragma unroll
-      for (int w = 0; w < NW; w++) {
-        g += red[w][0][r][l];
-        u += NB == 1 ? red[w][0][r][(l + 16) & 63] : red[w][NB - 1][r][l];
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+      for (int i = 0; i < V; i++) {
+        g[i] += red[w][0][r0 / RV][l][(r0 + i) % RV];
+        u[i] += NB == 1 ? red[w][0][r0 / RV][(l + 16) & 63][0] : red[w][NB - 1][r0 / RV][l][(r0 + i) % RV];
       }
+#pragma unroll
+    for (int i = 0; i < V; i++) {
+      const int r = r0 + i;
       const int64_t row = m0 + (r >> 2) * 8 + (l >> 5) * 4 + (r & 3);
       const int64_t fcol = n0 / 2 + (lq % FW);
-      const float v = gelu_sigmoid(g * p.c_scale) * (u * p.c_scale);
+      const float v = gelu_sigmoid(g[i] * p.c_scale) * (u[i] * p.c_scale);
       put<SPLIT>(C + row * p.ldc, fcol, v, p.out_scale, row < M && fcol < F);
     }
   } else {
-    for (int e = tid; e < NB * 16 * 64; e += NW * 64) {
-      const int j = e >> 10, r = (e >> 6) & 15, l = e & 63;
-      float v = 0.f;
+    static_assert(NB * 16 * 64 == 4 * NW * 64, "four rows per thread");
+    const int j = tid >> 8, q = (tid >> 6) & 3, l = lane;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int w = 0; w < NW; w++) v += red[w][j][r][l];
-      const int64_t row = m0 + (r >> 2) * 8 + (l >> 5) * 4 + (r & 3);
-      const int64_t col = n0 + 32 * j + (l & 31);
+    for (int w = 0; w < NW; w++) v += *reinterpret_cast<const f32x4*>(red[w][j][q][l]);
+    const int64_t col = n0 + 32 * j + (l & 31);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const int64_t row = m0 + 8 * q + (l >> 5) * 4 + c;
       const bool ok = row < M && col < N;
-      v *= p.c_scale;
-      if constexpr (EPI == Epi::Generic) v = h2_generic(p, v, row, col, ok);
-      put<SPLIT>(C + row * p.ldc, col, v, p.out_scale, ok);
+      float x = v[c] * p.c_scale;
+      if constexpr (EPI == Epi::Generic) x = h2_generic(p, x, row, col, ok);
+      put<SPLIT>(C + row * p.ldc, col, x, p.out_scale, ok);
     }
   }
 }
