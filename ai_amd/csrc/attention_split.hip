@@ -555,10 +555,16 @@ int launch_attention_split(fa_ctx* ctx, const AttnGenericArgs& a, hipStream_t s)
   p.q_sb = a.q_sb; p.q_sh = a.q_sh; p.k_sb = a.k_sb; p.k_sh = a.k_sh; p.v_sb = a.v_sb; p.v_sh = a.v_sh;
   p.m_sb = a.m_sb; p.m_sh = a.m_sh; p.m_sr = a.m_sr; p.m_sc = a.m_sc;
   p.scale = a.scale;
-  // 128 queries per workgroup, or 64 where those leave CUs without one
+  // 64 queries per workgroup while those are at most one per CU, else 128 (at
+  // head_dim 64 and 128 only where they fill their last one to more than half:
+  // there two 64-query workgroups share a CU, at 256 a CU holds one of either).
+  // Us with 64 and 128 queries, 512 keys: 64 heads x 256, head_dim 64: 24 and 29,
+  // 256: 68 and 86; 64 x 512, 64: 32 and 31, 256: 124 and 91; 64 x 320, 64: 29 and
+  // 30, 256: 121 and 86; 64 x 700, 64: 44 and 51, 128: 75 and 85, 256: 179 and 161.
   const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
   const int64_t bh = (int64_t)a.B * a.H;
-  const int W = bh * ((a.T + 127) / 128) >= cus / 2 && (a.T + 127) / 128 * 128 - a.T < 64 ? 8 : 4;
+  const bool half = (a.T + 127) / 128 * 128 - a.T >= 64;
+  const int W = bh * ((a.T + 63) / 64) > cus && (a.D == 256 || !half) ? 8 : 4;
   p.qblocks = (a.T + 16 * W - 1) / (16 * W);
   const dim3 gk((unsigned)z.blocks), bk(256);
   switch (a.D) {
