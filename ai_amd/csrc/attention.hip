@@ -590,10 +590,16 @@ __device__ __forceinline__ f16x8 as_f16x8(u32x4 v) { return __builtin_bit_cast(f
 // attention_tiles_kernel computes attention_varlen_kernel<256>'s result on
 // the fp16 MFMA (v_mfma_f32_16x16x32_f16) with fp32 accuracy: every fp32
 // operand, times a power of two from a bound on all of them, is held as two
-// fp16 terms, and a product a.b is hi.hi + hi.lo + lo.hi (lo.lo is below 2^-24
-// relative), accumulated in fp32. Its error against float64 is below that of
-// three exact bf16 terms and six products (8 x 1 024..2 048 tokens, two layers:
-// 1.0e-6 -> 7.3e-7): half the MFMAs also means half the fp32 roundings.
+// fp16 terms (within 2^-23 of it), and a product a.b is hi.hi + hi.lo + lo.hi
+// (lo.lo, of either sign, is at most 2^-22 of it), accumulated in fp32. The
+// fp32 roundings of the sums weigh more, and half the MFMAs also means half of
+// them: the error against float64 is below that of three exact bf16 terms and
+// six products (8 x 1 024..2 048 tokens, two layers: 1.0e-6 -> 7.5e-7; EmbeddingGemma
+// 2's unscaled scores, 32 x 64..256: 2.4e-4 -> 2.0e-4). lo has no scale of its own:
+// layers whose gains or value rows are so uneven that this costs bits take the
+// fp32 kernel (prepare_h2, model.cpp). MFMA pipes busy 0.31 and 0.35 of the time
+// at 8 x 1 024..2 048 and 64 x 512 (rocprofv3, no bank conflicts), a wave waiting
+// 0.4 of its cycles: the barriers and the operand reads, one workgroup per CU.
 //
 // Rows. The query rows of kv head hk are the pairs (token t, query head
 // hk*G + g) of the G = H/Hkv heads that share it, numbered r = t*G + g. A
@@ -949,8 +955,8 @@ __global__ __launch_bounds__(64 * TL_W, TL_W == 8 ? 2 : 1) void attention_tiles_
     khi = min(L, tok + p.window);
   }
 
-  // The three term products of one 16-key block and one 32-dim chunk (lo . lo,
-  // below 2^-24 of the product, is dropped), smallest first, into s.
+  // The three term products of one 16-key block and one 32-dim chunk (lo . lo
+  // is dropped), smallest first, into s.
   auto qk_chunk = [&](f32x4& s, const f16x8& k0, const f16x8& k1, int c) {
     s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, qt[0][c], s, 0, 0, 0);
     s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qt[1][c], s, 0, 0, 0);

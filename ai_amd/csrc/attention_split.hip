@@ -1,11 +1,14 @@
 // The tensor.AttentionScaled drop-in at head_dim 64, 128 and 256 on the 16-bit
 // MFMA with fp32 accuracy, for any operands: attention_dense_kernel
 // (attention.hip) runs the same products on the fp32 MFMA, a sixteenth of
-// that rate, and stays for small calls and head_dim 512. 8 x 8 heads x 512 x 512,
-// head_dim 64: 55 -> 35 us per call (8 of them the image pass); 32 x 3 x 256 x 256
-// on one kv head, head_dim 256, padded: 95 -> 62. What bounds it now: the
-// softmax's VALU work at head_dim 64, the operand reads from LDS (2.4 of 2.9 us
-// per 32 keys) and the prologue at 256.
+// that rate, and stays for small calls, few queries and head_dim 512
+// (attention_split_pays). 8 x 8 heads x 512 x 512, head_dim 64: 55 -> 36 us per call
+// (10 of them the image pass); 32 x 3 x 256 x 256 on one kv head, head_dim 256, padded:
+// 95 -> 65. What bounds it now: at head_dim 64 the MFMAs (busy 0.45 of the time)
+// and the softmax between them; at 256 one workgroup per CU, two waves per SIMD
+// that wait half their cycles at the two barriers of a stage (MFMAs busy 0.25).
+// The error against float64 is below the fp32 kernel's (5.0e-7 -> 3.7e-7 and 3.6e-7
+// -> 2.5e-7), whose sums take more roundings.
 //
 // Queries, keys, values and probabilities are three exact bf16 terms each
 // (split8), a product the six MFMAs whose terms' orders add up to at most two
@@ -17,8 +20,8 @@
 //
 // split_kv_kernel writes, per (batch, kv head, tile of 32 keys), a key image
 // [term][key][HD] and a value image [term][dim][32 slots], in the order in
-// which the attention's direct global->LDS loads and operand reads take them: 16-byte chunk c of key k at c ^ (k mod 16) (head_dim
-// 64: c ^ (k / 2 mod 8)), slot 8g + 4h + r of a dim holding key 16h + 4g + r,
+// which the attention's direct global->LDS loads and operand reads take them:
+// 16-byte chunk c of key k at c ^ (k mod 16) (head_dim 64: c ^ (k / 2 mod 8)), slot 8g + 4h + r of a dim holding key 16h + 4g + r,
 // chunk g of dim d at g ^ (d / 2 mod 4), both free of bank conflicts (d / 4 mod 4
 // had a third of the value reads in conflict). Heads that share one key/value
 // head share its images.
@@ -32,9 +35,8 @@
 // load after a second barrier: head_dim 256 has room for no more, and four-wave
 // workgroups of the others fit a CU twice with one); scores; P.V of the previous
 // stage; softmax. P.V one stage behind leaves the values a whole stage to land
-// (2 048 queries and keys, 3 heads
-// of 256: 211 -> 192 us per call). The row maximum is lazy: the
-// offset moves when a stage's maximum exceeds it by more than 8.
+// (2 048 queries and keys, 3 heads of 256: 211 -> 192 us per call). The row maximum
+// is lazy: the offset moves when a stage's maximum exceeds it by more than 8.
 #include <algorithm>
 #include <cstdlib>
 

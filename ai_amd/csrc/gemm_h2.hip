@@ -4,18 +4,27 @@
 //
 // A value a, scaled by a power of two that keeps its product's whole operand
 // inside fp16's range, is stored by the kernel that produces it as
-// hi = fp16(a) and lo = fp16((a - hi) * 2^11): 22 to 24 significant bits
-// (a - hi is exact; one bit in four values rounds in the last place), the
-// same 4 bytes as the float. lo carries its own 2^11 so that it stays a
-// normal fp16 number down to 2^-25 of the largest value. A weight w times
-// its matrix's power of two is exact in fp16 (checked when the model is
-// finalized; otherwise the model keeps the three-term bf16 products of
-// gemm.hip). Two v_mfma_f32_32x32x16_f16 per operand pair, hi . w and
-// lo . (w * 2^-11), accumulate in fp32; the epilogue takes the powers of two
-// back out. Against the exact three-term bf16 split this is two thirds of
-// the MFMA work, no split in the product (each value is split once, where it
-// is made, instead of once per column tile), and fewer fp32 roundings per
-// sum: the error against float64 is smaller (tests/test_gpu_h2.py).
+// hi = fp16(a) and lo = fp16((a - hi) * 2^11): within 2^-23 of a (a - hi is
+// exact; lo rounds one value in four), the same 4 bytes as the float. lo
+// carries its own 2^11 so that it stays a normal fp16 number down to 2^-25 of
+// the largest value. A weight w times its matrix's power of two is exact in
+// fp16 (checked when the model is finalized; otherwise the model keeps the
+// three-term bf16 products of gemm.hip); w * 2^-11, the lo terms' factor, is
+// rounded where w is below 2^-21 of its matrix's largest, and prepare_h2
+// (model.cpp) holds what that and the operands' range add below a sixteenth of a
+// float32 rounding in every row. Two v_mfma_f32_32x32x16_f16 per operand pair,
+// hi . w and lo . (w * 2^-11), accumulate in fp32; the epilogue takes the
+// powers of two back out. Against the exact three-term bf16 split this is two
+// thirds of the MFMA work, no split in the product (each value is split once,
+// where it is made, instead of once per column tile), and fewer fp32 roundings
+// per sum, which is what the error against float64 comes from: two layers of
+// 30 x 60..150 tokens 7.9e-7 by three terms and 6.8e-7, of 19 tokens 4.3e-7 and
+// 3.8e-7, the 24-layer forward of 19 tokens 6.6e-7 and 4.1e-7.
+//
+// What bounds the large tiles: their MFMA pipes are busy 0.45 to 0.56 of the time
+// (rocprofv3; LDS without a bank conflict), a wave waits a third of its cycles
+// at the slab barriers, and the clock falls under the load: 32 768 x 2 304 x 768
+// takes 453 thousand cycles in 252 to 275 us, 1.7 of 2.4 GHz, 0.92 PF/s executed.
 //
 // Layout of a split operand: row-major like the float matrix it replaces,
 // with each 8 values as 16 bytes of hi then 16 bytes of lo.
@@ -444,6 +453,20 @@ int forced_htile() {
   return v;
 }
 
+// Tile by the workgroups each would launch. Us per launch, K = 768 (o: K parts
+// included), small, 64x128, 128x128 and 128x256:
+//  - small while its 32 x 64 tiles have a CU each (40 rows of q|k|v 8.0, 9.4,
+//    10.6; of gate|up 9.1, 12.9, 14.7; 200 rows 10.9, 12.8, 15.2 and 11.4, 13.4,
+//    15.7; 256 rows of gate|up 14.4, 13.2, 15.8: level);
+//  - GeGLU on 128x256 from four per CU (32 768 rows -, 301, 258, 251; 24 576: 223,
+//    193, 195; 16 384: 143, 127, 139: the line lies low), or where they fill one
+//    and a quarter to two rounds that 128x128 does not fit into (5 504: 55, 53, 51;
+//    6 912: 63, 57, 55);
+//  - 64x128 where 128x128 leaves most CUs with one or less (512 rows of q|k|v 13.0
+//    and 14.9; 1 280: 13.8 and 15.4; 1 792: 16.3 and 15.9) or would begin a third
+//    round of two per CU (o at 5 504: 24.9 and 26.1);
+//  - launches beside other groups' (shared): 128x128 unless it fills less than
+//    half the CUs; the other streams fill what it leaves.
 HTileId pick_htile(int64_t m, int64_t n, int ksplit, Epi epi, int cus, bool shared) {
   if (((m + 31) / 32) * ((n + 63) / 64) * ksplit <= cus) return HTileId::small;
   const int64_t t128 = ((m + 127) / 128) * ((n + 127) / 128) * ksplit;

@@ -210,8 +210,10 @@ int fa_rope(fa_ctx* ctx, const float* x, double base, const int32_t* positions, 
  * contiguous. Masked weights are exactly 0 (exp of inputs below -87 flushes
  * to 0, internal/kernel/generic.go:278-307). Head dims 64, 128, 256 and
  * 512 with 16-byte aligned rows (batch and head strides multiples of 4) run
- * on the fp32 MFMA, or (64, 128 and 256, from 192 keys and about 0.1 GFLOP)
- * on the 16-bit MFMA with fp32 accuracy; other shapes on a per-row kernel (D <= 512).
+ * on the fp32 MFMA, or (64, 128 and 256, with enough keys and queries for it to be
+ * the faster one) on the 16-bit MFMA from exact 16-bit terms of the operands, with
+ * the fp32 path's range and no more than its error; other shapes on a per-row
+ * kernel (D <= 512).
  * Replaces tensor.AttentionScaled (tensor/attention.go:67-83,130-287). */
 int fa_attention(fa_ctx* ctx, const float* q, const float* k, const float* v, int32_t B, int32_t H, int32_t T,
                  int32_t S, int32_t D, int64_t q_sb, int64_t q_sh, int64_t k_sb, int64_t k_sh, int64_t v_sb,
@@ -237,7 +239,8 @@ int fa_attention_dev(fa_ctx* ctx, const float* q, const float* k, const float* v
  * formed (blocks of 256 queries); otherwise the scores are fp32-MFMA sums
  * (within a few units of the last place of the exact score), up to 32
  * queries with d % 16 == 0 and 16-byte aligned rows in one pass over the docs
- * that selects as it goes, else by a product and a two-pass top-k. A query's scores, and its order among
+ * that selects as it goes (where that is the faster way), else by a product and a
+ * two-pass top-k. A query's scores, and its order among
  * candidates whose scores agree to that precision, can therefore differ
  * between a call with fewer than 128 queries (or topk > 16) and one with
  * more; fa_similarities_topk_dev_noalloc takes the exact path for any nq. */
