@@ -469,11 +469,14 @@ int range_h2(fa_model* m, std::vector<Mat*>& mats) {
   }
   if (v2) {
     // the embeddings as an operand: a token's values have rms |its row|, and
-    // its result is normed, so the least row sets the limit
+    // its result is normed, so the least row sets the limit, down to where the
+    // norm's eps outweighs the result (|w| |row| / sqrt(d) < sqrt(eps))
     m->s_x0 = pow2_for(value(nm) * 1.01 * rd);
     float least = INFINITY;
+    const double w_top = top(out1(model_w));
+    const float from = w_top > 0 ? (float)(rd * std::sqrt((double)c.rms_norm_eps) / w_top) : 0.f;
     for (float n : out1(emb))
-      if (n != 0.f) least = std::min(least, n);
+      if (n != 0.f) least = std::min(least, std::max(n, from));
     ok = ok && (least == INFINITY || holds(m->wple_model, out1(model_w), out1(model_w), Vec(d, 1.f), m->s_x0 * least));
   }
   m->tiles = tiles;

@@ -108,6 +108,40 @@ def test_gpu_matches_oracle(eg2, B, T, lo):
     assert np.allclose(np.linalg.norm(got, axis=1), 1, atol=1e-5)
 
 
+def ple_gain(ws):  # a per-layer-input gain of 2^24, the projections' columns make up for it
+    ws["ple.per_layer_projection_norm.weight"][3] = 2.0 ** 24
+    for n, w in ws.items():
+        if n.endswith("ple_block.per_layer_projection.weight"):
+            w[:, 3] = np.sign(w[:, 3]) * 2.0 ** -29
+
+
+def small_rows(ws):  # embedding rows 2^-9 and 2^-40 times the others
+    ws["embed_tokens.weight"][5::7] *= 2.0 ** -9
+    ws["embed_tokens.weight"][6::7] *= 2.0 ** -40
+
+
+@pytest.mark.parametrize("edit", [ple_gain, small_rows])
+def test_gpu_uneven_ranges_match_oracle(ctx, edit):
+    """Operands of very different sizes in the per-layer-input block: on the
+    split products or the three-term ones, at the bars of every other model."""
+    shape = eg2_shape()
+    ws = weights(shape, 32)
+    edit(ws)
+    om = O.OracleModel2(shape)
+    for k, v in ws.items():
+        om.set(k, v)
+    om.finalize()
+    gm = gpu_model(shape, ws, ctx)
+    ids, lengths = batch(77, 4, 120, 20, shape.vocab_size)
+    got, want = gm.embed_ids(ids, lengths), om.embed(ids, lengths)
+    gm.close()
+    om.close()
+    d = np.abs(got - want).max()
+    print(f"EG2 {edit.__name__}: cosine {cos_rows(got, want).min():.9f}, max|d| {d:.3g}", flush=True)
+    assert cos_rows(got, want).min() >= 0.9999999
+    assert d <= 5e-5
+
+
 @pytest.mark.parametrize("B,T", [(3, 400), (2, 512)])
 def test_gpu_few_sequences_tile_items(eg2, B, T):
     """A few long sequences on one stream: 3 x 400 tokens (more than 1 024)
